@@ -180,7 +180,7 @@ int need_fft(cup2d_ctx* c) {
 // and boundary-band blocks afterwards.
 int pressure_single(cup2d_ctx* c, int fused) {
   RC(need_fft(c));
-  if (fused && c->flux_deferred && c->cfg.poisson != CUP2D_POISSON_COSINE) {
+  if (fused && c->flux_deferred) {
     RC(join_obstacles(c));
     RC(enqueue_rhs_obstacles(c, 1));
     // after an early row pass the fade factor is already reduced (the patch
@@ -511,6 +511,9 @@ int cup2d_create(const cup2d_cfg* cfg, cup2d_ctx** out) {
   g.nu = cfg->nu; g.CFL = cfg->CFL; g.lambda = cfg->lambda;
   g.fadeLenX = cfg->fadeLen * cfg->extent;  // Simulation.cpp:97-98
   g.fadeLenY = cfg->fadeLen * cfg->extent;
+  constexpr double eps = 2.220446049250313e-16;  // std::numeric_limits<double>::epsilon()
+  g.invFadeX = 1 / dmax(g.fadeLenX, eps);
+  g.invFadeY = 1 / dmax(g.fadeLenY, eps);
   g.implicit_penal = cfg->implicit_penal;
   g.nshapes = 0;
   g.nfish = 0;

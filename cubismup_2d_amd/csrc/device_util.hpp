@@ -69,12 +69,10 @@ __host__ __device__ inline bool band_block(const Grid& g, int bx, int by) {
 
 // cub2rhs fadeArg (PoissonSolver.cpp:88-93) at cell centre (px, py).
 __host__ __device__ inline double fade_arg(const Grid& g, double px, double py) {
-  constexpr double eps = 2.220446049250313e-16;  // std::numeric_limits<double>::epsilon()
-  const double invFadeX = 1 / dmax(g.fadeLenX, eps), invFadeY = 1 / dmax(g.fadeLenY, eps);
-  const double yt = invFadeY * dmax(0.0, g.fadeLenY - g.extent1 + py);
-  const double yb = invFadeY * dmax(0.0, g.fadeLenY - py);
-  const double xt = invFadeX * dmax(0.0, g.fadeLenX - g.extent0 + px);
-  const double xb = invFadeX * dmax(0.0, g.fadeLenX - px);
+  const double yt = g.invFadeY * dmax(0.0, g.fadeLenY - g.extent1 + py);
+  const double yb = g.invFadeY * dmax(0.0, g.fadeLenY - py);
+  const double xt = g.invFadeX * dmax(0.0, g.fadeLenX - g.extent0 + px);
+  const double xb = g.invFadeX * dmax(0.0, g.fadeLenX - px);
   return dmin(dmax(dmax(dmax(yt, yb), xt), xb), 1.0);
 }
 

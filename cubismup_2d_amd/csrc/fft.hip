@@ -14,19 +14,23 @@
 //      zero-pruned: only the NY data rows are read and written.
 //   3. rows inverse: unpack two half-spectrum rows, inverse complex FFT, real
 //      part -> row y, imaginary part -> row y+1.
-// Cosine solver (FFTW_dirichlet, FFTW_dirichlet.h:23-148): a DCT-II of an
-// N-point sequence x is, up to the phase exp(i pi k / 2N), the FFT of its
-// 2N-point mirror image (x, reversed x), and a DCT-III of real coefficients
-// multiplied by a symbol s(k) is the first N points of the inverse FFT of
-// s(k) times that spectrum when s is extended evenly, s(2N-k) = s(k).  So the
-// 2D cosine solve is the free-space pipeline with the mirrored grid in place
-// of the zero padding (the row pass reads x reversed past NX, the column pass
-// reads the spectrum rows reversed past NY) and the DCT-domain symbol.
+// Cosine solver (FFTW_dirichlet, FFTW_dirichlet.h:23-148): the same three
+// passes at the grid's own lengths.  With v[n] = x[2n], v[N-1-n] = x[2n+1]
+// (Makhoul, IEEE Trans. ASSP 28, 1980) and V its N-point FFT, the DCT-II is
+// C[k] = Re(w_k V[k]), C[N-k] = -Im(w_k V[k]) with w_k = exp(-i pi k / 2N);
+// the DCT-III is the same steps backwards.  The row pass stores a row's real
+// coefficients k and N-k as one complex column (conj(w_k V[k])), so the
+// spectrum has NX/2 complex columns as in the periodic case, and the column
+// pass transforms two real columns at once.  (Transforming the 2NX x 2NY
+// mirror image instead took twice the spectrum and four times the column
+// work: column pass at 2048 x 1024 36.2 us, solve at 1024 x 512 47 us.)
 // The FFT core is a radix-16 Stockham autosort (radix 2/4/8 for the last
 // pass), 16 complex values per thread in registers, LDS padded by one slot
 // every 16 entries so stride-16 stores are bank-conflict free.  Twiddles come
 // from per-length tables exp(-2 pi i k/L) built in long double on the host.
 #include <cmath>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "device_util.hpp"
@@ -46,7 +50,7 @@ struct FFTPlan {
   int NYs = 0;            // rows stored in the spectrum
   int ncg = 0;            // column groups
   int fs = 0;             // free-space
-  int cs = 0;             // cosine (Neumann) solver on the mirrored 2NX x 2NY grid
+  int cs = 0;             // cosine (Neumann) solver
   double2* spec = nullptr;
   double2* tw_r = nullptr;
   double2* tw_c = nullptr;
@@ -56,6 +60,12 @@ struct FFTPlan {
   void* tw_c32 = nullptr;
   double* ghat = nullptr;   // free-space: [ncg][Lc/2+1][G]
   double* ghatN = nullptr;  // free-space Nyquist column [Lc/2+1]
+  // cosine: exp(-i pi k / 2NX), k <= NX/2, and the same for NY; rounded to
+  // float for the FP32 solve
+  double2* dct_r = nullptr;
+  double2* dct_c = nullptr;
+  void* dct_r32 = nullptr;
+  void* dct_c32 = nullptr;
   double* cosX = nullptr;   // cosine: (float) cos(2 pi i / NX), i < NX
   double* cosY = nullptr;   // cosine: (float) cos(2 pi j / NY), j < NY
 };
@@ -357,7 +367,7 @@ __device__ __forceinline__ void fft_regs(V* x, V* lds, int base, int stride, int
 template <int L, int E>
 constexpr int lds_len() { return L + L / E; }
 template <int L, int E>
-constexpr int rows_np() { return (L / E) >= 256 ? 1 : 256 / (L / E); }
+constexpr int rows_np() { return (L / E) >= 64 ? 1 : 64 / (L / E); }
 
 // ---------------------------------------------------------- rows forward
 // in: nrows rows of ncols valid reals (row pitch in_pitch), zero beyond;
@@ -378,7 +388,8 @@ constexpr int rows_np() { return (L / E) >= 256 ? 1 : 256 / (L / E); }
 // neighbours; v of rows y0-1 .. y0+2 stays in registers.
 //
 // store_all (SRC_FADE, SRC_DIV): every cell's final RHS is written to the
-// RHS plane, not only the faded band cells (the FP64 refinement reads it).
+// RHS plane, not only the faded band cells (the FP64 refinement reads it; a
+// step with the cosine solver leaves the whole RHS there).
 //
 // SRC_DIV with obmap == nullptr is the early pass: every block's RHS is the
 // divergence (obstacle blocks included), run before the obstacle lists
@@ -392,6 +403,17 @@ constexpr int rows_np() { return (L / E) >= 256 ? 1 : 256 / (L / E); }
 // costing about a whole pass: the early launch exits at once and SRC_PATCH
 // does the whole pass.
 enum { SRC_PLAIN = 0, SRC_FADE = 1, SRC_DIV = 2, SRC_PATCH = 3 };
+
+// What a row or column of the transform length holds: the sequence itself
+// (periodic; zero padding past the data), or with KIND_COS the DCT's
+// reordering, element m being grid cell row_cell<KIND, L>(m).  The row passes
+// read and write the grid in its own order and reorder in LDS.
+enum { KIND_SEQ = 0, KIND_COS = 1 };
+template <int KIND, int L>
+__device__ __forceinline__ int row_cell(int m) {
+  if constexpr (KIND == KIND_COS) return m < L / 2 ? 2 * m : 2 * (L - 1 - m) + 1;
+  return m;
+}
 struct RowSource {
   Grid g;
   int npart;            // fade-sum workgroups (0: no fade)
@@ -400,7 +422,7 @@ struct RowSource {
   const void* u;        // SRC_DIV: advDiff output (S)
   const void* v;
   const unsigned char* obmap;
-  int mirror;           // cosine: columns past ncols read the row reversed
+  const void* dct;      // KIND_COS: w_k = exp(-i pi k / 2L), k <= L/2 (cplx<S>)
   int store_all;
   const double* fadepart;  // SRC_PATCH redo: the fade sums' partials (npart x 3)
 };
@@ -409,11 +431,14 @@ struct RowSource {
 // of row y0 + i row y0+1) and its split into the two rows' half spectra,
 // stored (or with patch added) at spec[cg][y0, y0+1][G].  Every thread of the
 // workgroup takes part (the barriers); invalid pairs store nothing.
-template <int L, int E, typename S>
+// KIND_COS: column k holds the rows' DCT coefficients k and L-k, column 0
+// those of 0 and L/2.
+template <int L, int E, int KIND, typename S>
 __device__ __forceinline__ void rows_fwd_transform_store(cplx<S>* x, cplx<S>* lds, int base, int t,
                                                          const cplx<S>* w, bool valid,
                                                          cplx<S>* __restrict__ spec,
-                                                         int spec_rows, int y0, bool patch) {
+                                                         int spec_rows, int y0, bool patch,
+                                                         const cplx<S>* __restrict__ dct) {
   using V = cplx<S>;
   constexpr int NT = L / E;
   fft_regs<L, E, true>(x, lds, base, 1, t, w);
@@ -430,7 +455,11 @@ __device__ __forceinline__ void rows_fwd_transform_store(cplx<S>* x, cplx<S>* ld
     const V Z = x[q];
     V A, B;
     if (k == 0) {
-      const V ZN = x[E / 2];  // element L/2
+      V ZN = x[E / 2];  // element L/2
+      if constexpr (KIND == KIND_COS) {  // C[L/2] = cos(pi/4) V[L/2]
+        constexpr S h = (S)0.70710678118654752440;
+        ZN = mk<V>(h * ZN.x, h * ZN.y);
+      }
       A = mk<V>(Z.x, ZN.x);
       B = mk<V>(Z.y, ZN.y);
     } else {
@@ -439,6 +468,13 @@ __device__ __forceinline__ void rows_fwd_transform_store(cplx<S>* x, cplx<S>* ld
       const V d = mk<V>(Z.x - Zm.x, Z.y + Zm.y);   // Z - conj(Zm)
       A = mk<V>(half * sm.x, half * sm.y);
       B = mk<V>(half * d.y, -half * d.x);
+      if constexpr (KIND == KIND_COS) {
+        const V wk = dct[k];
+        A = cmul(A, wk);
+        B = cmul(B, wk);
+        A.y = -A.y;
+        B.y = -B.y;
+      }
     }
     const int cg = k / G, c = k % G;
     V* o = spec + ((size_t)cg * spec_rows + y0) * G + c;
@@ -455,7 +491,7 @@ __device__ __forceinline__ void rows_fwd_transform_store(cplx<S>* x, cplx<S>* ld
 
 // One group of NP row pairs (group wg: pairs wg*NP .. wg*NP + NP-1) of
 // k_rows_fwd; tw is the length-L twiddle table.
-template <int L, int NP, int E, int SRC, typename S>
+template <int L, int NP, int E, int SRC, int KIND, typename S>
 __device__ __forceinline__ void rows_fwd_group(int wg, const S* in, int in_pitch, int ncols,
                                                int nrows, cplx<S>* __restrict__ spec,
                                                int spec_rows, const cplx<S>* __restrict__ tw,
@@ -509,6 +545,15 @@ __device__ __forceinline__ void rows_fwd_group(int wg, const S* in, int in_pitch
     // has all of them in flight (storing u into LDS inside this loop would
     // wait for each group in turn)
     S u0[E], u1[E], vm[E], v0[E], v1[E], vp[E];
+    unsigned obm = 0;  // bit q: the cell's block is an obstacle block (a pair lies in one block row)
+    if (fd.obmap) {
+      const unsigned char* om = fd.obmap + (yc / BS) * g.bpdx;
+#pragma unroll
+      for (int q = 0; q < E; ++q) {
+        const int i = t + q * NT;
+        if (i < NX) obm |= om[i / BS] != 0 ? 1u << q : 0u;
+      }
+    }
 #pragma unroll
     for (int q = 0; q < E; ++q) {
       const int i = t + q * NT;
@@ -548,20 +593,28 @@ __device__ __forceinline__ void rows_fwd_group(int wg, const S* in, int in_pitch
         const S vn1 = flux_fixed<S>(vp[q], yp, NY, fcorr);
         r0 = facDiv * ((ue0 - uw0) + (vc1 - vs0));
         r1 = facDiv * ((ue1 - uw1) + (vn1 - vc0));
-        const int bx = i / BS;
-        if (patch) {  // a pair lies in one block row
-          if (fd.obmap[(y0 / BS) * g.bpdx + bx]) {
-            r0 = rhsp[(size_t)y0 * NX + i] - r0;
-            r1 = rhsp[(size_t)(y0 + 1) * NX + i] - r1;
-          } else {
-            r0 = r1 = 0;
-          }
-        } else if (fd.obmap) {
-          if (fd.obmap[(y0 / BS) * g.bpdx + bx]) r0 = rhsp[(size_t)y0 * NX + i];
-          if (fd.obmap[((y0 + 1) / BS) * g.bpdx + bx]) r1 = rhsp[(size_t)(y0 + 1) * NX + i];
-        }
       }
       x[q] = mk<V>(r0, r1);
+    }
+    // the obstacle blocks' final RHS (patch: less the divergence, and zero
+    // elsewhere); all its loads are issued before the first use
+    if (obm != 0 && valid) {
+      S o0[E], o1[E];
+#pragma unroll
+      for (int q = 0; q < E; ++q)
+        if (obm >> q & 1) {
+          o0[q] = rhsp[(size_t)y0 * NX + t + q * NT];
+          o1[q] = rhsp[(size_t)(y0 + 1) * NX + t + q * NT];
+        }
+#pragma unroll
+      for (int q = 0; q < E; ++q)
+        if (obm >> q & 1)
+          x[q] = patch ? mk<V>(o0[q] - x[q].x, o1[q] - x[q].y) : mk<V>(o0[q], o1[q]);
+    }
+    if (patch) {
+#pragma unroll
+      for (int q = 0; q < E; ++q)
+        if (!(obm >> q & 1)) x[q] = mk<V>(0, 0);
     }
     __syncthreads();  // ud is reused below
   } else {
@@ -569,8 +622,7 @@ __device__ __forceinline__ void rows_fwd_group(int wg, const S* in, int in_pitch
     const S* r1 = r0 + in_pitch;
 #pragma unroll
     for (int q = 0; q < E; ++q) {
-      int i = t + q * NT;
-      if (fd.mirror && i >= ncols) i = 2 * ncols - 1 - i;
+      const int i = t + q * NT;
       S a = 0, b = 0;
       if (valid && i < ncols) { a = r0[i]; b = r1[i]; }
       x[q] = mk<V>(a, b);
@@ -586,10 +638,8 @@ __device__ __forceinline__ void rows_fwd_group(int wg, const S* in, int in_pitch
       if (valid) {
 #pragma unroll
         for (int q = 0; q < E; ++q) {
-          const int iq = t + q * NT;
-          const int i = fd.mirror && iq >= ncols ? 2 * ncols - 1 - iq : iq;
+          const int i = t + q * NT;
           if (i >= ncols) continue;
-          const bool own = i == iq;  // the mirrored copy is written back once
           const int bx = i / BS;
           const bool col = band_col(g, bx);
           if (!(row0 || row1 || col)) continue;
@@ -597,12 +647,12 @@ __device__ __forceinline__ void rows_fwd_group(int wg, const S* in, int in_pitch
           if (row0 || col) {
             const double py = cell_pos(by0, y0 % BS, g.hb, g.h);
             x[q].x = (S)fade_cell((double)x[q].x, fade_arg(g, px, py), corr);
-            if (own && !fd.store_all) rhsp[(size_t)y0 * in_pitch + i] = x[q].x;
+            if (!fd.store_all) rhsp[(size_t)y0 * in_pitch + i] = x[q].x;
           }
           if (row1 || col) {
             const double py = cell_pos(by1, (y0 + 1) % BS, g.hb, g.h);
             x[q].y = (S)fade_cell((double)x[q].y, fade_arg(g, px, py), corr);
-            if (own && !fd.store_all) rhsp[(size_t)(y0 + 1) * in_pitch + i] = x[q].y;
+            if (!fd.store_all) rhsp[(size_t)(y0 + 1) * in_pitch + i] = x[q].y;
           }
         }
       }
@@ -618,15 +668,27 @@ __device__ __forceinline__ void rows_fwd_group(int wg, const S* in, int in_pitch
       }
     }
   }
+  if constexpr (KIND == KIND_COS) {  // the DCT's order (row_cell), through LDS
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+      const int i = t + q * NT;
+      lds[base + padE<E>(i & 1 ? L - 1 - i / 2 : i / 2)] = x[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < E; ++q) x[q] = lds[base + padE<E>(t + q * NT)];
+    __syncthreads();
+  }
   // the thread's twiddle bases, loaded only now: held through the loads of
   // the source rows they would push the kernel past its register budget
   asm volatile("" ::: "memory");
   V w[TwCount<L, E, E>::n];
   tw_load<L, E, E>(tw, t, w);
-  rows_fwd_transform_store<L, E, S>(x, lds, base, t, w, valid, spec, spec_rows, y0, patch);
+  rows_fwd_transform_store<L, E, KIND, S>(x, lds, base, t, w, valid, spec, spec_rows, y0, patch,
+                                          static_cast<const V*>(fd.dct));
 }
 
-template <int L, int NP, int E, int SRC, typename S>
+template <int L, int NP, int E, int SRC, typename S, int KIND = KIND_SEQ>
 __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_fwd(
     const S* in, int in_pitch, int ncols, int nrows, cplx<S>* __restrict__ spec,
     int spec_rows, const cplx<S>* __restrict__ tw, RowSource fd) {
@@ -644,7 +706,7 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_fwd(
   if constexpr (SRC == SRC_PATCH) xcd_order = fd.st->rows_redo != 0 || fd.st->rows_early_on == 0;
   int wg = blockIdx.x;
   if (xcd_order && gridDim.x % 8 == 0) wg = (wg % 8) * (gridDim.x / 8) + wg / 8;
-  rows_fwd_group<L, NP, E, SRC, S>(wg, in, in_pitch, ncols, nrows, spec, spec_rows, tw, fd, lds);
+  rows_fwd_group<L, NP, E, SRC, KIND, S>(wg, in, in_pitch, ncols, nrows, spec, spec_rows, tw, fd, lds);
 }
 
 // ---------------------------------------------------------- rows inverse
@@ -658,14 +720,14 @@ enum { OUT_SET = 0, OUT_ADD = 1, OUT_RES = 2, OUT_RES_FWD = 3 };
 // rounded to float as OUT_RES stores them, are transformed forward in FP32
 // at once into spec32 (k_rows_fwd<SRC_PLAIN, float>'s arithmetic and
 // layout) instead of being stored: the FP32 solve of the residual starts at
-// the column pass.  Rows without a mirror only (L == ncols).
+// the column pass.  Periodic grid only.
 // OUT_ADD also subtracts *mean (the solution's mean before the update, which
 // the spectral operator cannot see: the solve's convention is a zero mean).
 // OUT_RES also writes the workgroup's statistics of r and b to
 // respart[5 wg .. 5 wg + 4]: cell count, sum r, sum (r - mean_wg r)^2, sum b,
 // sum (b - mean_wg b)^2 (the residual norm of the sweep without the mean,
 // which the operator does not see; k_res_reduce merges them).
-template <int L, int NP, int E, typename S, int OUT>
+template <int L, int NP, int E, typename S, int OUT, int KIND = KIND_SEQ>
 __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const cplx<S>* __restrict__ spec,
                                                          int spec_rows, void* __restrict__ outv,
                                                          const float* __restrict__ bres,
@@ -674,7 +736,8 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
                                                          const double* __restrict__ mean,
                                                          double* __restrict__ respart,
                                                          float2* __restrict__ spec32,
-                                                         const float2* __restrict__ tw32) {
+                                                         const float2* __restrict__ tw32,
+                                                         const cplx<S>* __restrict__ dct) {
   using V = cplx<S>;
   constexpr int NT = L / E, PADL = lds_len<L, E>();
   constexpr bool RES = OUT == OUT_RES || OUT == OUT_RES_FWD;
@@ -705,11 +768,22 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
 #pragma unroll
   for (int q = 0; q < E / 2; ++q) {
     const int k = t + q * NT;
-    const V A = As[q], B = Bs[q];
+    V A = As[q], B = Bs[q];
     if (k == 0) {
       x[0] = mk<V>(A.x, B.x);
       x[E / 2] = mk<V>(A.y, B.y);
+      if constexpr (KIND == KIND_COS) {  // V[L/2] = sqrt(2) F[L/2]
+        constexpr S r2 = (S)1.41421356237309504880;
+        x[E / 2] = mk<V>(r2 * A.y, r2 * B.y);
+      }
     } else {
+      if constexpr (KIND == KIND_COS) {  // V[k] = conj(w_k (F[k] + i F[L-k]))
+        const V wk = dct[k];
+        A = cmul(A, wk);
+        B = cmul(B, wk);
+        A.y = -A.y;
+        B.y = -B.y;
+      }
       x[q] = mk<V>(A.x - B.y, A.y + B.x);
       lds[base + padE<E>(L - k)] = mk<V>(A.x + B.y, -A.y + B.x);
     }
@@ -722,6 +796,15 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
   }
   __syncthreads();
   fft_regs<L, E, false>(x, lds, base, 1, t, w);
+  if constexpr (KIND == KIND_COS) {  // back to the grid's order, through LDS
+#pragma unroll
+    for (int q = 0; q < E; ++q)
+      lds[base + padE<E>(row_cell<KIND, L>(t + q * NT))] = x[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < E; ++q) x[q] = lds[base + padE<E>(t + q * NT)];
+    if constexpr (RES) __syncthreads();  // the reductions reuse the LDS
+  }
   if constexpr (RES) {
     constexpr int NTB = NP * L / E;
     // r is held for the second moments; b is read again there (the same
@@ -790,8 +873,9 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
       asm volatile("" ::: "memory");  // the float bases are loaded only now
       float2 wf[TwCount<L, E, E>::n];
       tw_load<L, E, E>(tw32, t, wf);
-      rows_fwd_transform_store<L, E, float>(xf, ldsf, base, t, wf, valid, spec32, spec_rows, y0,
-                                            false);
+      static_assert(KIND == KIND_SEQ, "the fused pass is the periodic grid's");
+      rows_fwd_transform_store<L, E, KIND_SEQ, float>(xf, ldsf, base, t, wf, valid, spec32,
+                                                      spec_rows, y0, false, nullptr);
     }
   } else {
     if (!valid) return;
@@ -846,8 +930,8 @@ __global__ __launch_bounds__(256) void k_res_reduce(const double* __restrict__ r
 
 // --------------------------------------------------------------- columns
 // MODE 0: periodic solve, 1: free-space solve (zero-pruned), 2: forward only,
-// 3: cosine solve, 4: periodic apply, 5: cosine apply.  The apply modes
-// multiply by the inverse of the solve symbol (zero at the DC mode, which
+// 4: periodic apply (k_cols); 3: cosine solve, 5: cosine apply (k_cols_cos).
+// The apply modes multiply by the inverse of the solve symbol (zero at the DC mode, which
 // the solve discards): the FP64 spectral operator whose residual the
 // refinement sweeps correct.
 struct ColParams {
@@ -860,16 +944,25 @@ struct ColParams {
   int GH;
   const double* cosX;    // MODE 3, 5
   const double* cosY;
+  const void* dct;       // MODE 3, 5: w_k = exp(-i pi k / 2NY), k <= NY/2 (the spectrum's type)
   double* dc_out;        // MODE 4, 5: receives the input's mean (its DC coefficient * norm)
 };
+
+// 1 / d for a normal d > 0: the hardware's estimate and two Newton steps
+// (within an ulp), half the instructions of the IEEE division, of which a
+// column pass takes one or two per element.
+__device__ __forceinline__ double reciprocal(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma_s(r, fma_s(-d, r, 1.0), r);
+  return fma_s(r, fma_s(-d, r, 1.0), r);
+}
 
 __device__ __forceinline__ double periodic_factor(int kx, int ky, const ColParams& P) {
   // FFTW_periodic.h:82-91: kinv*norm_factor, DC set to zero
   const int kyy = ky <= P.NY / 2 ? ky : P.NY - ky;
-  if (kx == 0 && kyy == 0) return 0.0;
   const double rkx = kx * P.waveFactX, rky = kyy * P.waveFactY;
-  const double kinv = -1 / (rkx * rkx + rky * rky);
-  return kinv * P.norm;
+  const double s = -P.norm * reciprocal(rkx * rkx + rky * rky);
+  return kx == 0 && kyy == 0 ? 0.0 : s;
 }
 // the operator whose pseudo-inverse periodic_factor applies: -k^2 norm
 __device__ __forceinline__ double periodic_apply(int kx, int ky, const ColParams& P) {
@@ -883,20 +976,17 @@ __device__ __forceinline__ double periodic_apply(int kx, int ky, const ColParams
 // (NX, NY).  Line 51 declares the blend weight as `static constexpr tol =
 // 0.1;`, which has no type; it is taken as the double 0.1 the initializer
 // states.  COScoef are floats (FFTW_dirichlet.h:26-27,65-68).
-__device__ __forceinline__ double cosine_denom(int i, int j, const ColParams& P) {
+// cosine_part(i, waveFact, COScoef[i]) is one direction's share of the
+// denominator.
+__device__ __forceinline__ double cosine_part(int i, double waveFact, double coef) {
   const double tol = 0.1;
-  const double rkx = (i + 0.5) * P.waveFactX, rky = (j + 0.5) * P.waveFactY;
-  const double denomFD = 1 - P.cosX[i] / 2 - P.cosY[j] / 2;
-  const double denomSP = rkx * rkx + rky * rky;
-  return (1 - tol) * denomFD + tol * denomSP;
+  const double rk = (i + 0.5) * waveFact;
+  return (1 - tol) * (0.5 - coef / 2) + tol * (rk * rk);
 }
-__device__ __forceinline__ double cosine_factor(int i, int j, const ColParams& P) {
-  if (i == 0 && j == 0) return 0.0;  // in_out[0] = 0
-  return -P.norm / cosine_denom(i, j, P);
-}
-__device__ __forceinline__ double cosine_apply(int i, int j, const ColParams& P) {
-  if (i == 0 && j == 0) return 0.0;
-  return -P.norm * cosine_denom(i, j, P);
+template <int MODE>
+__device__ __forceinline__ double cosine_symbol(double partX, double partY, const ColParams& P) {
+  const double den = partX + partY;
+  return MODE == 3 ? -P.norm * reciprocal(den) : -P.norm * den;
 }
 
 template <int LC, int MODE>
@@ -905,11 +995,6 @@ __device__ __forceinline__ double col_symbol(int kx, int cg, int c, int ky, cons
     return periodic_factor(kx, ky, P);
   } else if constexpr (MODE == 4) {
     return periodic_apply(kx, ky, P);
-  } else if constexpr (MODE == 3 || MODE == 5) {
-    // symbol extended evenly about NX and NY; zero at the mirror Nyquist
-    if (kx >= P.NX || ky == P.NY) return 0.0;
-    const int kyy = ky < P.NY ? ky : LC - ky;
-    return MODE == 3 ? cosine_factor(kx, kyy, P) : cosine_apply(kx, kyy, P);
   } else {
     const int kyy = ky <= P.GH ? ky : LC - ky;
     return P.ghat[((size_t)cg * (P.GH + 1) + kyy) * G + c];
@@ -942,7 +1027,7 @@ __global__ __launch_bounds__(CW * LC / E, min_waves<E>()) void k_cols(cplx<S>* _
                                                       const cplx<S>* __restrict__ tw) {
   using V = cplx<S>;
   constexpr int NT = LC / E;
-  constexpr bool MIRROR = MODE == 3 || MODE == 5;
+  static_assert(MODE != 3 && MODE != 5, "k_cols_cos");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   V* lds = reinterpret_cast<V*>(smem_raw);
   const int cl = threadIdx.x % CW, t = threadIdx.x / CW;
@@ -956,9 +1041,7 @@ __global__ __launch_bounds__(CW * LC / E, min_waves<E>()) void k_cols(cplx<S>* _
 #pragma unroll
   for (int q = 0; q < E; ++q) {
     const int i = t + q * NT;
-    if constexpr (MIRROR)  // mirrored grid: rows past NY are rows NY-1, NY-2, ...
-      x[q] = col[(size_t)(i < P.rows ? i : 2 * P.rows - 1 - i) * G + c];
-    else if constexpr (MODE == 1)  // zero padding: rows <= LC/2 (checked at launch)
+    if constexpr (MODE == 1)  // zero padding: rows <= LC/2 (checked at launch)
       x[q] = q < E / 2 && i < P.rows ? col[(size_t)i * G + c] : mk<V>(0, 0);
     else
       x[q] = col[(size_t)i * G + c];
@@ -977,9 +1060,9 @@ __global__ __launch_bounds__(CW * LC / E, min_waves<E>()) void k_cols(cplx<S>* _
 #pragma unroll
       for (int q = 0; q < E; ++q) lds[padE<E>(t + q * NT) * CW + cl] = x[q];
       // apply modes: the DC coefficient (real part of the packed DC column
-      // at ky = 0) is the input's sum, times 4 on the mirrored grid; the
-      // operator discards it, the refinement removes it from the solution
-      if constexpr (MODE == 4 || MODE == 5)
+      // at ky = 0) is the input's sum; the operator discards it, the
+      // refinement removes it from the solution
+      if constexpr (MODE == 4)
         if (t == 0 && cl == 0 && P.dc_out) *P.dc_out = (double)x[0].x * P.norm;
       __syncthreads();
 #pragma unroll
@@ -990,7 +1073,6 @@ __global__ __launch_bounds__(CW * LC / E, min_waves<E>()) void k_cols(cplx<S>* _
           double sN;
           if constexpr (MODE == 0) sN = periodic_factor(P.NX / 2, i, P);
           else if constexpr (MODE == 4) sN = periodic_apply(P.NX / 2, i, P);
-          else if constexpr (MIRROR) sN = 0.0;  // mirror Nyquist kx = NX
           else sN = P.ghatN[i <= P.GH ? i : LC - i];
           const V m = lds[padE<E>((LC - i) % LC) * CW + cl];
           const S a = (S)(0.5 * (s0 + sN)), b = (S)(0.5 * (s0 - sN));
@@ -1018,9 +1100,87 @@ __global__ __launch_bounds__(CW * LC / E, min_waves<E>()) void k_cols(cplx<S>* _
     for (int q = 0; q < E; ++q) {
       const int i = t + q * NT;
       if (MODE == 1 && q >= E / 2) continue;
-      if ((MODE != 1 && !MIRROR) || i < P.rows) col[(size_t)i * G + c] = x[q];
+      if (MODE != 1 || i < P.rows) col[(size_t)i * G + c] = x[q];
     }
   }
+}
+
+// The cosine solver's column pass (MODE 3) and its apply (MODE 5).  A complex
+// column is two real columns of x coefficients, kx = k (real part) and NX - k
+// (imaginary part; column 0: 0 and NX/2).  The DCT is linear, so the complex
+// sequence takes it as a whole: with V the N-point FFT of the reordered
+// column, C[j] = (w_j V[j] + conj(w_j) V[N-j]) / 2 and
+// C[N-j] = i (w_j V[j] - conj(w_j) V[N-j]) / 2; the symbol multiplies the two
+// parts separately, and the inverse's input is V[j] = conj(w_j) (F[j] - i
+// F[N-j]), V[N-j] = i w_j (F[N-j] - i F[j]).  A thread holds j = t + q NT
+// of the lower half and takes N-j from LDS, so each pair's symbols and
+// products are formed once.
+template <int N, int E, int MODE, typename S>
+__global__ __launch_bounds__(CW * N / E, min_waves<E>()) void k_cols_cos(
+    cplx<S>* __restrict__ spec, ColParams P, const cplx<S>* __restrict__ tw) {
+  using V = cplx<S>;
+  constexpr int NT = N / E;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  V* lds = reinterpret_cast<V*>(smem_raw);
+  const int cl = threadIdx.x % CW, t = threadIdx.x / CW;
+  int cg, half;
+  col_group_of_block(blockIdx.x, gridDim.x, &cg, &half);
+  const int c = half * CW + cl, kx = cg * G + c;
+  const V* dct = static_cast<const V*>(P.dct);
+  V* col = spec + (size_t)cg * P.stride * G + c;
+  V x[E];
+#pragma unroll
+  for (int q = 0; q < E; ++q) x[q] = col[(size_t)row_cell<KIND_COS, N>(t + q * NT) * G];
+  V w[TwCount<N, E, E>::n];
+  tw_load<N, E, E>(tw, t, w);
+  fft_regs<N, E, true>(x, lds, cl, CW, t, w);
+#pragma unroll
+  for (int q = E / 2; q < E; ++q) lds[padE<E>(t + q * NT) * CW + cl] = x[q];
+  __syncthreads();
+  const int kx2 = kx == 0 ? P.NX / 2 : P.NX - kx;
+  const double px1 = cosine_part(kx, P.waveFactX, P.cosX[kx]);
+  const double px2 = cosine_part(kx2, P.waveFactX, P.cosX[kx2]);
+  const S hf = (S)0.5;
+#pragma unroll
+  for (int q = 0; q < E / 2; ++q) {
+    const int j = t + q * NT;
+    const double py1 = cosine_part(j, P.waveFactY, P.cosY[j]);
+    const S s11 = kx == 0 && j == 0 ? (S)0 : (S)cosine_symbol<MODE>(px1, py1, P);
+    const S s21 = (S)cosine_symbol<MODE>(px2, py1, P);
+    if (j == 0) {
+      // the input's mean: its DC coefficient (the operator discards it, the
+      // refinement removes it from the solution)
+      if (MODE == 5 && kx == 0 && P.dc_out) *P.dc_out = (double)x[0].x * P.norm;
+      x[0] = mk<V>(s11 * x[0].x, s21 * x[0].y);
+      // j = N/2, its own partner: C = cos(pi/4) V, the inverse's input sqrt(2) F
+      const double pyh = cosine_part(N / 2, P.waveFactY, P.cosY[N / 2]);
+      const V z = x[E / 2];
+      x[E / 2] = mk<V>((S)cosine_symbol<MODE>(px1, pyh, P) * z.x,
+                       (S)cosine_symbol<MODE>(px2, pyh, P) * z.y);
+      lds[padE<E>(N / 2) * CW + cl] = x[E / 2];
+    } else {
+      V* m = lds + padE<E>(N - j) * CW + cl;
+      const double py2 = cosine_part(N - j, P.waveFactY, P.cosY[N - j]);
+      const S s12 = (S)cosine_symbol<MODE>(px1, py2, P), s22 = (S)cosine_symbol<MODE>(px2, py2, P);
+      const V wj = dct[j];
+      const V A = cmul(x[q], wj), B = cmulc(*m, wj);
+      // F[j] = s o (A + B)/2, F[N-j] = s o i (A - B)/2
+      const V F1 = mk<V>(hf * s11 * (A.x + B.x), hf * s21 * (A.y + B.y));
+      const V F2 = mk<V>(hf * s12 * (B.y - A.y), hf * s22 * (A.x - B.x));
+      x[q] = cmulc(mk<V>(F1.x + F2.y, F1.y - F2.x), wj);  // conj(w) (F1 - i F2)
+      const V z = cmul(mk<V>(F2.x + F1.y, F2.y - F1.x), wj);  // w (F2 - i F1)
+      *m = mk<V>(-z.y, z.x);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = E / 2; q < E; ++q) x[q] = lds[padE<E>(t + q * NT) * CW + cl];
+  __syncthreads();
+  asm volatile("" ::: "memory");  // the bases again, as in k_cols
+  tw_load<N, E, E>(tw, t, w);
+  fft_regs<N, E, false>(x, lds, cl, CW, t, w);
+#pragma unroll
+  for (int q = 0; q < E; ++q) col[(size_t)row_cell<KIND_COS, N>(t + q * NT) * G] = x[q];
 }
 
 // Green's function spectrum: Re(FFT G) * norm, even-folded to ky <= GH =
@@ -1044,7 +1204,10 @@ __global__ void k_ghat_extract(const double2* __restrict__ spec, int Lc, int ncg
 }
 
 // ----------------------------------------------------------- dispatch
-template <int L, typename S>
+// largest row and column transform lengths
+constexpr int MAX_LR = 8192, MAX_LC = 4096;
+
+template <int L, int KIND, typename S>
 static void launch_rows_fwd(cup2d_ctx* c, const S* in, int pitch, int ncols, int nrows,
                             cplx<S>* spec, int spec_rows, const cplx<S>* tw, int src,
                             const RowSource& fd, hipStream_t st) {
@@ -1053,31 +1216,31 @@ static void launch_rows_fwd(cup2d_ctx* c, const S* in, int pitch, int ncols, int
   const size_t shm = (size_t)NP * lds_len<L, RE>() * sizeof(cplx<S>);
   const dim3 grid((nrows / 2 + NP - 1) / NP), block(NP * L / RE);
   if (src == SRC_DIV)
-    CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_DIV, S>), grid, block, shm, st, in,
-                       pitch, ncols, nrows, spec, spec_rows, tw, fd);
-  else if (src == SRC_PATCH)
-    CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_PATCH, S>), grid, block, shm, st, in,
+    CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_DIV, S, KIND>), grid, block, shm, st, in,
                        pitch, ncols, nrows, spec, spec_rows, tw, fd);
   else if (src == SRC_FADE)
-    CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_FADE, S>), grid, block, shm, st, in,
+    CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_FADE, S, KIND>), grid, block, shm, st, in,
                        pitch, ncols, nrows, spec, spec_rows, tw, fd);
-  else
-    CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_PLAIN, S>), grid, block, shm, st,
+  else if (src == SRC_PLAIN)
+    CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_PLAIN, S, KIND>), grid, block, shm, st,
                        in, pitch, ncols, nrows, spec, spec_rows, tw, fd);
+  else if constexpr (KIND != KIND_COS)  // the cosine solver has no early row pass to patch
+    CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_PATCH, S, KIND>), grid, block, shm, st, in,
+                       pitch, ncols, nrows, spec, spec_rows, tw, fd);
 }
-template <int L, typename S, int OUT>
+template <int L, int KIND, typename S, int OUT>
 static void launch_rows_inv(cup2d_ctx* c, const cplx<S>* spec, int spec_rows, void* out,
                             const float* bres, int pitch, int ncols, int nrows,
                             const cplx<S>* tw, const double* mean, float2* spec32,
-                            const float2* tw32) {
+                            const float2* tw32, const cplx<S>* dct) {
   constexpr int RE = row_e<L>();
   c->rows_inv_wgs = (nrows / 2 + rows_np<L, RE>() - 1) / rows_np<L, RE>();
   constexpr int NP = rows_np<L, RE>();
   const size_t shm = (size_t)NP * lds_len<L, RE>() * sizeof(cplx<S>);
   const int pairs = nrows / 2;
-  CUP2D_TIMED_LAUNCH(c, (k_rows_inv<L, NP, RE, S, OUT>), dim3((pairs + NP - 1) / NP),
+  CUP2D_TIMED_LAUNCH(c, (k_rows_inv<L, NP, RE, S, OUT, KIND>), dim3((pairs + NP - 1) / NP),
                      dim3(NP * L / RE), shm, c->stream, spec, spec_rows, out, bres, pitch,
-                     ncols, nrows, tw, mean, c->respart, spec32, tw32);
+                     ncols, nrows, tw, mean, c->respart, spec32, tw32, dct);
 }
 template <int LC, int MODE, typename S>
 static int launch_cols(cup2d_ctx* c, cplx<S>* spec, int ncg, const ColParams& P,
@@ -1085,130 +1248,128 @@ static int launch_cols(cup2d_ctx* c, cplx<S>* spec, int ncg, const ColParams& P,
   constexpr int CE = col_e<LC>();
   if (MODE == 1 && 2 * P.rows > LC) return CUP2D_ERR_ARG;  // k_cols reads rows < LC/2 only
   const size_t shm = (size_t)lds_len<LC, CE>() * CW * sizeof(cplx<S>);
-  CUP2D_TIMED_LAUNCH(c, (k_cols<LC, MODE, CE, S>), dim3(ncg * (G / CW)), dim3(CW * LC / CE), shm,
-                     c->stream, spec, P, tw);
+  const dim3 grid(ncg * (G / CW)), block(CW * LC / CE);
+  if constexpr (MODE == 3 || MODE == 5)
+    CUP2D_TIMED_LAUNCH(c, (k_cols_cos<LC, CE, MODE, S>), grid, block, shm, c->stream, spec, P, tw);
+  else
+    CUP2D_TIMED_LAUNCH(c, (k_cols<LC, MODE, CE, S>), grid, block, shm, c->stream, spec, P, tw);
   return CUP2D_OK;
 }
 
-template <typename S>
+// fn(std::integral_constant<int, L>) for the row (column) length L, with the
+// cosine solver's lengths capped at half the largest (its limits are those
+// of the 2N-point mirror image)
+template <int MAXL, int L = 32, typename F>
+static int with_length(int len, F&& fn) {
+  if constexpr (L > MAXL) {
+    return CUP2D_ERR_ARG;
+  } else {
+    if (len == L) return fn(std::integral_constant<int, L>{});
+    return with_length<MAXL, 2 * L>(len, std::forward<F>(fn));
+  }
+}
+
+template <typename S, int KIND = KIND_SEQ>
 static int rows_fwd(cup2d_ctx* c, int L, const S* in, int pitch, int ncols, int nrows,
                     cplx<S>* spec, int spec_rows, const cplx<S>* tw, int src,
                     const RowSource& fd, hipStream_t st = nullptr) {
   if (!st) st = c->stream;
-  switch (L) {
-    case 32: launch_rows_fwd<32, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    case 64: launch_rows_fwd<64, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    case 128: launch_rows_fwd<128, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    case 256: launch_rows_fwd<256, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    case 512: launch_rows_fwd<512, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    case 1024: launch_rows_fwd<1024, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    case 2048: launch_rows_fwd<2048, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    case 4096: launch_rows_fwd<4096, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    case 8192: launch_rows_fwd<8192, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st); break;
-    default: return CUP2D_ERR_ARG;
-  }
-  return CUP2D_OK;
+  return with_length<KIND == KIND_COS ? MAX_LR / 2 : MAX_LR>(L, [&](auto len) {
+    launch_rows_fwd<len(), KIND, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st);
+    return CUP2D_OK;
+  });
 }
-template <typename S, int OUT>
+template <typename S, int OUT, int KIND = KIND_SEQ>
 static int rows_inv(cup2d_ctx* c, int L, const cplx<S>* spec, int spec_rows, void* out,
                     const float* bres, int pitch, int ncols, int nrows, const cplx<S>* tw,
                     const double* mean = nullptr, float2* spec32 = nullptr,
-                    const float2* tw32 = nullptr) {
-  switch (L) {
-    case 32: launch_rows_inv<32, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    case 64: launch_rows_inv<64, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    case 128: launch_rows_inv<128, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    case 256: launch_rows_inv<256, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    case 512: launch_rows_inv<512, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    case 1024: launch_rows_inv<1024, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    case 2048: launch_rows_inv<2048, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    case 4096: launch_rows_inv<4096, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    case 8192: launch_rows_inv<8192, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw, mean, spec32, tw32); break;
-    default: return CUP2D_ERR_ARG;
-  }
-  return CUP2D_OK;
+                    const float2* tw32 = nullptr, const cplx<S>* dct = nullptr) {
+  return with_length<KIND == KIND_COS ? MAX_LR / 2 : MAX_LR>(L, [&](auto len) {
+    launch_rows_inv<len(), KIND, S, OUT>(c, spec, spec_rows, out, bres, pitch, ncols, nrows, tw,
+                                         mean, spec32, tw32, dct);
+    return CUP2D_OK;
+  });
 }
 template <int MODE, typename S>
 static int cols(cup2d_ctx* c, int LC, cplx<S>* spec, int ncg, const ColParams& P,
                 const cplx<S>* tw) {
-  switch (LC) {
-    case 32: return launch_cols<32, MODE, S>(c, spec, ncg, P, tw);
-    case 64: return launch_cols<64, MODE, S>(c, spec, ncg, P, tw);
-    case 128: return launch_cols<128, MODE, S>(c, spec, ncg, P, tw);
-    case 256: return launch_cols<256, MODE, S>(c, spec, ncg, P, tw);
-    case 512: return launch_cols<512, MODE, S>(c, spec, ncg, P, tw);
-    case 1024: return launch_cols<1024, MODE, S>(c, spec, ncg, P, tw);
-    case 2048: return launch_cols<2048, MODE, S>(c, spec, ncg, P, tw);
-    case 4096: return launch_cols<4096, MODE, S>(c, spec, ncg, P, tw);
-    default: return CUP2D_ERR_ARG;
-  }
-  return CUP2D_OK;
+  return with_length<MODE == 3 || MODE == 5 ? MAX_LC / 2 : MAX_LC>(
+      LC, [&](auto len) { return launch_cols<len(), MODE, S>(c, spec, ncg, P, tw); });
 }
 
-template <int L, typename S>
-static void set_rows_attr_LS() {
+static void set_shm(const void* k, int shm) {
+  (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+}
+template <int L, int KIND, typename S>
+static void set_rows_attr_S() {
   constexpr int RE = row_e<L>();
   constexpr int NP = rows_np<L, RE>();
   const int shm = NP * lds_len<L, RE>() * (int)sizeof(cplx<S>);
-  (void)hipFuncSetAttribute((const void*)k_rows_fwd<L, NP, RE, SRC_PLAIN, S>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-  (void)hipFuncSetAttribute((const void*)k_rows_fwd<L, NP, RE, SRC_FADE, S>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-  (void)hipFuncSetAttribute((const void*)k_rows_fwd<L, NP, RE, SRC_DIV, S>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-  (void)hipFuncSetAttribute((const void*)k_rows_fwd<L, NP, RE, SRC_PATCH, S>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-  (void)hipFuncSetAttribute((const void*)k_rows_inv<L, NP, RE, S, OUT_SET>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-  if constexpr (sizeof(S) == 4)
-    (void)hipFuncSetAttribute((const void*)k_rows_inv<L, NP, RE, S, OUT_ADD>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-  else {
-    (void)hipFuncSetAttribute((const void*)k_rows_inv<L, NP, RE, S, OUT_RES>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-    (void)hipFuncSetAttribute((const void*)k_rows_inv<L, NP, RE, S, OUT_RES_FWD>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+  set_shm((const void*)k_rows_fwd<L, NP, RE, SRC_PLAIN, S, KIND>, shm);
+  set_shm((const void*)k_rows_fwd<L, NP, RE, SRC_FADE, S, KIND>, shm);
+  set_shm((const void*)k_rows_fwd<L, NP, RE, SRC_DIV, S, KIND>, shm);
+  if constexpr (KIND != KIND_COS)
+    set_shm((const void*)k_rows_fwd<L, NP, RE, SRC_PATCH, S, KIND>, shm);
+  set_shm((const void*)k_rows_inv<L, NP, RE, S, OUT_SET, KIND>, shm);
+  if constexpr (sizeof(S) == 4) {
+    set_shm((const void*)k_rows_inv<L, NP, RE, S, OUT_ADD, KIND>, shm);
+  } else {
+    set_shm((const void*)k_rows_inv<L, NP, RE, S, OUT_RES, KIND>, shm);
+    if constexpr (KIND == KIND_SEQ)
+      set_shm((const void*)k_rows_inv<L, NP, RE, S, OUT_RES_FWD, KIND>, shm);
   }
 }
-template <int L>
-static void set_rows_attr_L() {
-  set_rows_attr_LS<L, double>();
-  set_rows_attr_LS<L, float>();
+template <int L, int KIND>
+static void set_rows_attr() {
+  set_rows_attr_S<L, KIND, double>();
+  set_rows_attr_S<L, KIND, float>();
 }
 template <int LC>
 static void set_cols_attr() {
   constexpr int CE = col_e<LC>();
   const int shm = lds_len<LC, CE>() * CW * (int)sizeof(double2);
   const int shm32 = lds_len<LC, CE>() * CW * (int)sizeof(float2);
-  const hipFuncAttribute A = hipFuncAttributeMaxDynamicSharedMemorySize;
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 0, CE, double>, A, shm);
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 1, CE, double>, A, shm);
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 2, CE, double>, A, shm);
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 3, CE, double>, A, shm);
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 4, CE, double>, A, shm);
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 5, CE, double>, A, shm);
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 0, CE, float>, A, shm32);
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 1, CE, float>, A, shm32);
-  (void)hipFuncSetAttribute((const void*)k_cols<LC, 3, CE, float>, A, shm32);
+  set_shm((const void*)k_cols<LC, 0, CE, double>, shm);
+  set_shm((const void*)k_cols<LC, 1, CE, double>, shm);
+  set_shm((const void*)k_cols<LC, 2, CE, double>, shm);
+  set_shm((const void*)k_cols<LC, 4, CE, double>, shm);
+  set_shm((const void*)k_cols<LC, 0, CE, float>, shm32);
+  set_shm((const void*)k_cols<LC, 1, CE, float>, shm32);
+  if constexpr (2 * LC <= MAX_LC) {
+    set_shm((const void*)k_cols_cos<LC, CE, 3, double>, shm);
+    set_shm((const void*)k_cols_cos<LC, CE, 5, double>, shm);
+    set_shm((const void*)k_cols_cos<LC, CE, 3, float>, shm32);
+  }
+}
+// the kernels of one plan's lengths and kind
+static void set_fft_attrs(const FFTPlan* P) {
+  if (P->cs)
+    with_length<MAX_LR / 2>(P->Lr, [](auto len) { set_rows_attr<len(), KIND_COS>(); return 0; });
+  else
+    with_length<MAX_LR>(P->Lr, [](auto len) { set_rows_attr<len(), KIND_SEQ>(); return 0; });
+  with_length<MAX_LC>(P->Lc, [](auto len) { set_cols_attr<len()>(); return 0; });
 }
 
-static std::vector<double2> twiddles(int L) {
-  std::vector<double2> w(L);
+// exp(-2 pi i k / L), k < n, rounded to V's type
+template <typename V>
+static std::vector<V> roots(int n, long long L) {
+  using S = typename ScalarOf<V>::type;
+  std::vector<V> w(n);
   const long double pi = 3.141592653589793238462643383279502884L;
-  for (int k = 0; k < L; ++k) {
+  for (int k = 0; k < n; ++k) {
     const long double a = -2.0L * pi * (long double)k / (long double)L;
-    w[k] = make_double2((double)cosl(a), (double)sinl(a));
+    w[k].x = (S)cosl(a);
+    w[k].y = (S)sinl(a);
   }
   return w;
 }
-static std::vector<float2> twiddles32(int L) {
-  std::vector<float2> w(L);
-  const long double pi = 3.141592653589793238462643383279502884L;
-  for (int k = 0; k < L; ++k) {
-    const long double a = -2.0L * pi * (long double)k / (long double)L;
-    w[k] = make_float2((float)cosl(a), (float)sinl(a));
-  }
-  return w;
+// the same as a new device table
+template <typename V, typename T>
+static int root_table(cup2d_ctx* c, T** out, int n, long long L) {
+  const std::vector<V> w = roots<V>(n, L);
+  CUP2D_HIP_CHECK(c, hipMalloc((void**)out, sizeof(V) * n));
+  CUP2D_HIP_CHECK(c, hipMemcpy(*out, w.data(), sizeof(V) * n, hipMemcpyHostToDevice));
+  return CUP2D_OK;
 }
 
 static bool pow2(int n) { return n >= 32 && (n & (n - 1)) == 0; }
@@ -1229,43 +1390,38 @@ int fft_create(cup2d_ctx* c) {
   // Free-space: any cyclic length >= 2N - 1 gives the linear convolution on
   // the N data points (FFTW_freespace.h:25-27 uses 2N - 1), so the rows and
   // columns take the next power of two >= 2N and any grid of 32-cell blocks
-  // is solved.  Periodic (N) and cosine (mirrored 2N) lengths must be powers
-  // of two themselves.
-  P->Lr = fs ? next_pow2(2 * NX) : cs ? 2 * NX : NX;
-  P->Lc = fs ? next_pow2(2 * NY) : cs ? 2 * NY : NY;
+  // is solved.  Periodic and cosine lengths (N) must be powers of two
+  // themselves.
+  P->Lr = fs ? next_pow2(2 * NX) : NX;
+  P->Lc = fs ? next_pow2(2 * NY) : NY;
   P->NYs = NY + SPEC_PAD;
   P->ncg = (P->Lr / 2) / G;
-  if ((!fs && (!pow2(NX) || !pow2(NY))) || P->Lr > 8192 || P->Lc > 4096) {
+  const int most = cs ? 2 : 1;  // the cosine solver's limits are half the periodic ones
+  if ((!fs && (!pow2(NX) || !pow2(NY))) || most * P->Lr > MAX_LR || most * P->Lc > MAX_LC) {
     c->err = "FFT Poisson: periodic and cosine NX and NY must be powers of two; row length "
              "<= 8192 and column length <= 4096 (periodic NX <= 8192, NY <= 4096; cosine "
              "NX <= 4096, NY <= 2048; free-space next_pow2(2 NX) <= 8192, next_pow2(2 NY) "
              "<= 4096)";
     return CUP2D_ERR_ARG;
   }
-  set_rows_attr_L<32>(); set_rows_attr_L<64>(); set_rows_attr_L<128>(); set_rows_attr_L<256>();
-  set_rows_attr_L<512>(); set_rows_attr_L<1024>(); set_rows_attr_L<2048>();
-  set_rows_attr_L<4096>(); set_rows_attr_L<8192>();
-  set_cols_attr<32>(); set_cols_attr<64>(); set_cols_attr<128>(); set_cols_attr<256>();
-  set_cols_attr<512>(); set_cols_attr<1024>(); set_cols_attr<2048>(); set_cols_attr<4096>();
+  set_fft_attrs(P);
 
   const size_t nspec = (size_t)P->ncg * G * P->NYs;
   CUP2D_HIP_CHECK(c, hipMalloc(&P->spec, sizeof(double2) * nspec));
-  const std::vector<double2> twr = twiddles(P->Lr), twc = twiddles(P->Lc);
-  CUP2D_HIP_CHECK(c, hipMalloc(&P->tw_r, sizeof(double2) * twr.size()));
-  CUP2D_HIP_CHECK(c, hipMalloc(&P->tw_c, sizeof(double2) * twc.size()));
-  CUP2D_HIP_CHECK(c, hipMemcpy(P->tw_r, twr.data(), sizeof(double2) * twr.size(), hipMemcpyHostToDevice));
-  CUP2D_HIP_CHECK(c, hipMemcpy(P->tw_c, twc.data(), sizeof(double2) * twc.size(), hipMemcpyHostToDevice));
+  int rc = root_table<double2>(c, &P->tw_r, P->Lr, P->Lr);
+  if (!rc) rc = root_table<double2>(c, &P->tw_c, P->Lc, P->Lc);
+  if (!rc && cs) rc = root_table<double2>(c, &P->dct_r, NX / 2 + 1, 4LL * NX);
+  if (!rc && cs) rc = root_table<double2>(c, &P->dct_c, NY / 2 + 1, 4LL * NY);
+  if (rc) return rc;
   if (c->f32) {
     // the FP32 solve's spectrum, tables rounded to float; P->spec (FP64)
     // serves the refinement's operator apply
     CUP2D_HIP_CHECK(c, hipMalloc(&P->spec32, sizeof(float2) * nspec));
-    const std::vector<float2> twr32 = twiddles32(P->Lr), twc32 = twiddles32(P->Lc);
-    CUP2D_HIP_CHECK(c, hipMalloc(&P->tw_r32, sizeof(float2) * twr32.size()));
-    CUP2D_HIP_CHECK(c, hipMalloc(&P->tw_c32, sizeof(float2) * twc32.size()));
-    CUP2D_HIP_CHECK(c, hipMemcpy(P->tw_r32, twr32.data(), sizeof(float2) * twr32.size(),
-                                 hipMemcpyHostToDevice));
-    CUP2D_HIP_CHECK(c, hipMemcpy(P->tw_c32, twc32.data(), sizeof(float2) * twc32.size(),
-                                 hipMemcpyHostToDevice));
+    rc = root_table<float2>(c, &P->tw_r32, P->Lr, P->Lr);
+    if (!rc) rc = root_table<float2>(c, &P->tw_c32, P->Lc, P->Lc);
+    if (!rc && cs) rc = root_table<float2>(c, &P->dct_r32, NX / 2 + 1, 4LL * NX);
+    if (!rc && cs) rc = root_table<float2>(c, &P->dct_c32, NY / 2 + 1, 4LL * NY);
+    if (rc) return rc;
   }
   if (cs) {  // FFTW_dirichlet.h:65-68: COScoef[i] = (float) cos(pi/M * 2 i)
     std::vector<double> cx(NX), cy(NY);
@@ -1300,7 +1456,7 @@ int fft_create(cup2d_ctx* c) {
   CUP2D_HIP_CHECK(c, hipMemcpy(dG, Gk.data(), sizeof(double) * Gk.size(), hipMemcpyHostToDevice));
   CUP2D_HIP_CHECK(c, hipMalloc(&P->ghat, sizeof(double) * (size_t)P->ncg * G * (GH + 1)));
   CUP2D_HIP_CHECK(c, hipMalloc(&P->ghatN, sizeof(double) * (size_t)(GH + 1)));
-  int rc = rows_fwd<double>(c, P->Lr, dG, MX, MX, MY, tspec, MY, P->tw_r, SRC_PLAIN,
+  rc = rows_fwd<double>(c, P->Lr, dG, MX, MX, MY, tspec, MY, P->tw_r, SRC_PLAIN,
                             RowSource{});
   if (rc) return rc;
   ColParams cp{};
@@ -1327,6 +1483,10 @@ void fft_destroy(cup2d_ctx* c) {
   if (P->spec32) (void)hipFree(P->spec32);
   if (P->tw_r32) (void)hipFree(P->tw_r32);
   if (P->tw_c32) (void)hipFree(P->tw_c32);
+  if (P->dct_r) (void)hipFree(P->dct_r);
+  if (P->dct_c) (void)hipFree(P->dct_c);
+  if (P->dct_r32) (void)hipFree(P->dct_r32);
+  if (P->dct_c32) (void)hipFree(P->dct_c32);
   if (P->ghat) (void)hipFree(P->ghat);
   if (P->ghatN) (void)hipFree(P->ghatN);
   if (P->cosX) (void)hipFree(P->cosX);
@@ -1344,7 +1504,7 @@ static ColParams col_params(const cup2d_ctx* c, bool apply, int* mode) {
   if (P->cs) {  // FFTW_dirichlet.h:47-48
     cp.waveFactX = M_PI / NX;
     cp.waveFactY = M_PI / NY;
-    cp.norm = 0.25 / ((double)NX * NY);
+    cp.norm = 1.0 / ((double)NX * NY);
     cp.cosX = P->cosX;
     cp.cosY = P->cosY;
     *mode = apply ? 5 : 3;
@@ -1363,10 +1523,17 @@ static ColParams col_params(const cup2d_ctx* c, bool apply, int* mode) {
 }
 
 template <typename S>
+static const cplx<S>* dct_table(double2* d, void* f) {
+  if constexpr (sizeof(S) == 8) return d;
+  else return reinterpret_cast<const cplx<S>*>(f);
+}
+
+template <typename S>
 static int cols_solve(cup2d_ctx* c, cplx<S>* spec, const cplx<S>* tw) {
   int mode;
-  const ColParams cp = col_params(c, false, &mode);
+  ColParams cp = col_params(c, false, &mode);
   const FFTPlan* P = c->fft;
+  cp.dct = dct_table<S>(P->dct_c, P->dct_c32);
   if (mode == 3) return cols<3, S>(c, P->Lc, spec, P->ncg, cp, tw);
   if (mode == 0) return cols<0, S>(c, P->Lc, spec, P->ncg, cp, tw);
   return cols<1, S>(c, P->Lc, spec, P->ncg, cp, tw);
@@ -1387,7 +1554,7 @@ int enqueue_rows_early(cup2d_ctx* c, hipStream_t s) {
     const int rf = enqueue_fade_reduce_on(c, s);
     if (rf) return rf;
   }
-  const RowSource fd{c->g, npart, c->rhs, c->st, c->u, c->v, nullptr, P->cs, c->f32 ? 1 : 0};
+  const RowSource fd{c->g, npart, c->rhs, c->st, c->u, c->v, nullptr, nullptr, c->f32 ? 1 : 0};
   int rc;
   {
     KernelTimer kt(c, T_FFT_ROWS_FWD);
@@ -1402,6 +1569,26 @@ int enqueue_rows_early(cup2d_ctx* c, hipStream_t s) {
   if (rc) return rc;
   c->rows_early = true;
   return launch_check(c, "early row pass");
+}
+
+// The grid's forward and inverse row passes with this plan's kind of rows.
+template <typename S>
+static int grid_rows_fwd(cup2d_ctx* c, const S* in, cplx<S>* spec, const cplx<S>* tw, int src,
+                         const RowSource& fd) {
+  const FFTPlan* P = c->fft;
+  const int NX = c->g.NX, NY = c->g.NY;
+  return P->cs ? rows_fwd<S, KIND_COS>(c, P->Lr, in, NX, NX, NY, spec, P->NYs, tw, src, fd)
+               : rows_fwd<S>(c, P->Lr, in, NX, NX, NY, spec, P->NYs, tw, src, fd);
+}
+template <typename S, int OUT>
+static int grid_rows_inv(cup2d_ctx* c, const cplx<S>* spec, void* out, const float* bres,
+                         const cplx<S>* tw, const double* mean = nullptr) {
+  const FFTPlan* P = c->fft;
+  const int NX = c->g.NX, NY = c->g.NY;
+  return P->cs ? rows_inv<S, OUT, KIND_COS>(c, P->Lr, spec, P->NYs, out, bres, NX, NX, NY, tw,
+                                            mean, nullptr, nullptr,
+                                            dct_table<S>(P->dct_r, P->dct_r32))
+               : rows_inv<S, OUT>(c, P->Lr, spec, P->NYs, out, bres, NX, NX, NY, tw, mean);
 }
 
 // src: SRC_PLAIN (rhs as given), SRC_FADE (rhs is the grid RHS: apply
@@ -1426,8 +1613,8 @@ int enqueue_poisson_fft(cup2d_ctx* c, double* rhs, double* sol, int src) {
     {
       KernelTimer kt(c, patch ? T_RHS_OBST : T_FFT_ROWS_FWD);
       RowSource fd{c->g, c->band_nblocks > 0 ? fade_partials(c) : 0, rhs, c->st,
-                   c->u, c->v, c->obmap, P->cs, 0, c->red};
-      rc = rows_fwd<double>(c, P->Lr, rhs, NX, NX, NY, P->spec, P->NYs, P->tw_r, src, fd);
+                   c->u, c->v, c->obmap, P->dct_r, P->cs && src == SRC_DIV ? 1 : 0, c->red};
+      rc = grid_rows_fwd<double>(c, rhs, P->spec, P->tw_r, src, fd);
     }
     if (rc) return rc;
     {
@@ -1441,8 +1628,7 @@ int enqueue_poisson_fft(cup2d_ctx* c, double* rhs, double* sol, int src) {
       rc = join_forces(c);
       if (rc) return rc;
       KernelTimer kt(c, T_FFT_ROWS_INV);
-      rc = rows_inv<double, OUT_SET>(c, P->Lr, P->spec, P->NYs, sol, nullptr, NX, NX, NY,
-                                     P->tw_r);
+      rc = grid_rows_inv<double, OUT_SET>(c, P->spec, sol, nullptr, P->tw_r);
     }
     if (rc) return rc;
     return launch_check(c, "poisson_fft");
@@ -1455,8 +1641,8 @@ int enqueue_poisson_fft(cup2d_ctx* c, double* rhs, double* sol, int src) {
   {
     KernelTimer kt(c, patch ? T_RHS_OBST : T_FFT_ROWS_FWD);
     RowSource fd{c->g, c->band_nblocks > 0 ? fade_partials(c) : 0, rhs, c->st,
-                 c->u, c->v, c->obmap, P->cs, src != SRC_PLAIN ? 1 : 0, c->red};
-    rc = rows_fwd<float>(c, P->Lr, b, NX, NX, NY, s32, P->NYs, twr32, src, fd);
+                 c->u, c->v, c->obmap, P->dct_r32, src != SRC_PLAIN ? 1 : 0, c->red};
+    rc = grid_rows_fwd<float>(c, b, s32, twr32, src, fd);
   }
   if (rc) return rc;
   {
@@ -1468,7 +1654,7 @@ int enqueue_poisson_fft(cup2d_ctx* c, double* rhs, double* sol, int src) {
   if (rc) return rc;
   {
     KernelTimer kt(c, T_FFT_ROWS_INV);
-    rc = rows_inv<float, OUT_SET>(c, P->Lr, s32, P->NYs, sol, nullptr, NX, NX, NY, twr32);
+    rc = grid_rows_inv<float, OUT_SET>(c, s32, sol, nullptr, twr32);
   }
   if (rc) return rc;
   const int sweeps = P->fs ? 0 : c->refine_sweeps;
@@ -1476,33 +1662,35 @@ int enqueue_poisson_fft(cup2d_ctx* c, double* rhs, double* sol, int src) {
   float* res = tp<float>(c->rres);
   for (int k = 0; k < sweeps; ++k) {
     TimerScope ts(c, T_REFINE);
-    const RowSource plain{c->g, 0, nullptr, c->st, nullptr, nullptr, nullptr, P->cs, 0};
-    rc = rows_fwd<double>(c, P->Lr, sol, NX, NX, NY, P->spec, P->NYs, P->tw_r, SRC_PLAIN, plain);
+    const RowSource plain{c->g, 0, nullptr, c->st, nullptr, nullptr, nullptr, P->dct_r, 0};
+    rc = grid_rows_fwd<double>(c, sol, P->spec, P->tw_r, SRC_PLAIN, plain);
     if (rc) return rc;
     int mode;
     ColParams ca = col_params(c, true, &mode);
     ca.dc_out = &c->st->pmean;
+    ca.dct = P->dct_c;
     rc = mode == 5 ? cols<5, double>(c, P->Lc, P->spec, P->ncg, ca, P->tw_c)
                    : cols<4, double>(c, P->Lc, P->spec, P->ncg, ca, P->tw_c);
     if (rc) return rc;
-    if (!P->cs && P->Lr == NX) {  // the residual's forward rows fused into its pass
+    if (!P->cs) {  // the residual's forward rows fused into its pass
       rc = rows_inv<double, OUT_RES_FWD>(c, P->Lr, P->spec, P->NYs, nullptr, b, NX, NX, NY,
                                          P->tw_r, nullptr, s32, twr32);
       if (rc) return rc;
       hipLaunchKernelGGL(k_res_reduce, dim3(1), dim3(256), 0, c->stream, c->respart,
                          c->rows_inv_wgs, &c->st->res[k]);
     } else {
-      rc = rows_inv<double, OUT_RES>(c, P->Lr, P->spec, P->NYs, res, b, NX, NX, NY, P->tw_r);
+      rc = rows_inv<double, OUT_RES, KIND_COS>(c, P->Lr, P->spec, P->NYs, res, b, NX, NX, NY,
+                                               P->tw_r, nullptr, nullptr, nullptr, P->dct_r);
       if (rc) return rc;
       hipLaunchKernelGGL(k_res_reduce, dim3(1), dim3(256), 0, c->stream, c->respart,
                          c->rows_inv_wgs, &c->st->res[k]);
-      rc = rows_fwd<float>(c, P->Lr, res, NX, NX, NY, s32, P->NYs, twr32, SRC_PLAIN, plain);
+      const RowSource plain32{c->g, 0, nullptr, c->st, nullptr, nullptr, nullptr, P->dct_r32, 0};
+      rc = grid_rows_fwd<float>(c, res, s32, twr32, SRC_PLAIN, plain32);
       if (rc) return rc;
     }
     rc = cols_solve<float>(c, s32, twc32);
     if (rc) return rc;
-    rc = rows_inv<float, OUT_ADD>(c, P->Lr, s32, P->NYs, sol, nullptr, NX, NX, NY, twr32,
-                                  &c->st->pmean);
+    rc = grid_rows_inv<float, OUT_ADD>(c, s32, sol, nullptr, twr32, &c->st->pmean);
     if (rc) return rc;
   }
   return launch_check(c, "poisson_fft");

@@ -87,6 +87,7 @@ struct Grid {
   int NX, NY, bpdx, bpdy;
   double h, hb, extent0, extent1;
   double nu, CFL, lambda, fadeLenX, fadeLenY;
+  double invFadeX, invFadeY;  // 1 / max(fadeLen, eps) (PoissonSolver.cpp:88-93)
   int implicit_penal, nshapes, nfish;
 };
 

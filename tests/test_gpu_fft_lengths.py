@@ -69,3 +69,37 @@ def test_freespace_lengths(cup, bpdx, bpdy):
     G[0, 0] = (2 * np.log(h / np.sqrt(np.pi)) - 1) / (4 * np.pi)
     P = np.fft.rfft2(r, s=G.shape) * np.fft.rfft2(G)
     assert rel(p, np.fft.irfft2(P, s=G.shape)[:NY, :NX]) < TOL
+
+
+def test_cosine_step_leaves_whole_rhs(cup):
+    """A whole step with the cosine solver forms the right-hand side inside the row pass; the
+    RHS plane afterwards holds it on every cell (faded), as the operators leave it.  Both form
+    the same cells with the same operations; only the fade factor's sums may differ by rounding:
+    a relative 1e-13 covers 4096-term sums at 16 eps."""
+    kw = dict(extent=1.0, nu=1e-3, fadeLen=0.05, poisson="cosine")
+    d = cup.disk(0.06, 0.4, 0.25, xvel=0.2, bFixed=True, bForced=True)
+    a, b = (cup.Simulation(16, 8, shapes=[d], **kw) for _ in range(2))
+    for s in (a, b):
+        s.reset()
+        s.simulate(3)
+    dt = a.calc_max_timestep()
+    a.advance(dt)
+    b.put_objects(dt)
+    b.advdiff(dt)
+    b.pressure_rhs(dt)
+    b.poisson_solve()
+    ra, rb = a.get_field(cup.TMP), b.get_field(cup.TMP)
+    assert rel(ra, rb) < 1e-13 and rel(a.get_field(cup.PRES), b.get_field(cup.PRES)) < TOL
+
+
+def test_cosine_fade_repeatable(cup):
+    """The row pass fades the band cells in place: the same right-hand side gives the same
+    solution and the same faded plane every time."""
+    sim = cup.Simulation(64, 8, extent=1.0, nu=1e-3, fadeLen=0.02, poisson="cosine")
+    r = np.random.default_rng(5).normal(size=(256, 2048))
+    got = set()
+    for _ in range(20):
+        sim.set_field(cup.TMP, r)
+        sim.poisson_solve()
+        got.add((sim.get_field(cup.TMP).tobytes(), sim.get_field(cup.PRES).tobytes()))
+    assert len(got) == 1
