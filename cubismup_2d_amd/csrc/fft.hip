@@ -243,13 +243,15 @@ __device__ __forceinline__ void dft_tw(V* v, V b) {
 // Elements per thread of the FFT core (the first pass is radix E), by
 // transform length.  With 8 the kernels are held to 128 VGPRs (4 waves per
 // SIMD, min_waves below) and two 8-wave workgroups share a CU; with 16 they
-// take up to 256 VGPRs.  Measured on MI355X (µs per pass, 8 vs 16): rows of
+// take up to 256 VGPRs.  Measured on MI355X (us per pass, 8 vs 16): rows of
 // 4096 63.8 vs 67.5, columns of 2048 41.5 vs 42.6; rows of 8192 382 vs 350,
-// inverse rows of 8192 157 vs 144, columns of 4096 205 vs 193.
+// inverse rows of 8192 157 vs 144; columns of 4096, one per workgroup
+// (col_cw): periodic 162 vs 171, free-space, whose symbol is loaded from a
+// table, 126 vs 114 (MODE 1).
 template <int L>
 constexpr int row_e() { return L >= 8192 ? 16 : 8; }
-template <int LC>
-constexpr int col_e() { return LC >= 4096 ? 16 : 8; }
+template <int LC, int MODE>
+constexpr int col_e() { return LC >= 4096 && MODE == 1 ? 16 : 8; }
 template <int E>
 constexpr int min_waves() { return E == 8 ? 4 : 1; }
 
@@ -1001,38 +1003,41 @@ __device__ __forceinline__ double col_symbol(int kx, int cg, int c, int ky, cons
   }
 }
 
-// Columns per workgroup (CW) of a column group of G: CW = G/2 halves the LDS
-// of a whole group so two workgroups share a CU.  The two halves of a group
-// run on the same XCD (block b runs on XCD b % 8) so the second half of each
-// 64 B chunk is an L2 hit.
-constexpr int CW = 2;
-static_assert(G % CW == 0, "CW");
+// Columns per workgroup of a column group of G: two, or one where two would
+// leave one workgroup per CU, whose load, transform and store phases overlap
+// nothing (columns of 4096, two -> one: 8192 x 4096 periodic 172 -> 162 us
+// with 8 elements per thread, 4000 x 2016 free-space 119 -> 114 us).  The parts of a group
+// run on the same XCD (block b runs on XCD b % 8) so the other parts of each
+// 64 B chunk are L2 hits.
+template <int LC>
+constexpr int col_cw() { return LC >= 4096 ? 1 : 2; }
 
-__device__ __forceinline__ void col_group_of_block(int b, int nblocks, int* cg, int* half) {
+template <int CW>
+__device__ __forceinline__ void col_group_of_block(int b, int nblocks, int* cg, int* part) {
   constexpr int H = G / CW;
   if (H == 1 || nblocks % (8 * H) != 0) {
     *cg = b / H;
-    *half = b % H;
+    *part = b % H;
     return;
   }
   const int xcd = b % 8, local = b / 8;        // consecutive locals share an XCD
   const int per_xcd = nblocks / 8;             // blocks per XCD
   const int lin = xcd * per_xcd + local;       // XCD-contiguous numbering
   *cg = lin / H;
-  *half = lin % H;
+  *part = lin % H;
 }
 
 template <int LC, int MODE, int E, typename S>
-__global__ __launch_bounds__(CW * LC / E, min_waves<E>()) void k_cols(cplx<S>* __restrict__ spec, ColParams P,
+__global__ __launch_bounds__(col_cw<LC>() * LC / E, min_waves<E>()) void k_cols(cplx<S>* __restrict__ spec, ColParams P,
                                                       const cplx<S>* __restrict__ tw) {
   using V = cplx<S>;
-  constexpr int NT = LC / E;
+  constexpr int NT = LC / E, CW = col_cw<LC>();
   static_assert(MODE != 3 && MODE != 5, "k_cols_cos");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   V* lds = reinterpret_cast<V*>(smem_raw);
   const int cl = threadIdx.x % CW, t = threadIdx.x / CW;
   int cg, half;
-  col_group_of_block(blockIdx.x, gridDim.x, &cg, &half);
+  col_group_of_block<CW>(blockIdx.x, gridDim.x, &cg, &half);
   const int c = half * CW + cl;  // column inside the group
   V* col = spec + (size_t)cg * P.stride * G;
   V w[TwCount<LC, E, E>::n];
@@ -1116,15 +1121,15 @@ __global__ __launch_bounds__(CW * LC / E, min_waves<E>()) void k_cols(cplx<S>* _
 // of the lower half and takes N-j from LDS, so each pair's symbols and
 // products are formed once.
 template <int N, int E, int MODE, typename S>
-__global__ __launch_bounds__(CW * N / E, min_waves<E>()) void k_cols_cos(
+__global__ __launch_bounds__(col_cw<N>() * N / E, min_waves<E>()) void k_cols_cos(
     cplx<S>* __restrict__ spec, ColParams P, const cplx<S>* __restrict__ tw) {
   using V = cplx<S>;
-  constexpr int NT = N / E;
+  constexpr int NT = N / E, CW = col_cw<N>();
   extern __shared__ __align__(16) unsigned char smem_raw[];
   V* lds = reinterpret_cast<V*>(smem_raw);
   const int cl = threadIdx.x % CW, t = threadIdx.x / CW;
   int cg, half;
-  col_group_of_block(blockIdx.x, gridDim.x, &cg, &half);
+  col_group_of_block<CW>(blockIdx.x, gridDim.x, &cg, &half);
   const int c = half * CW + cl, kx = cg * G + c;
   const V* dct = static_cast<const V*>(P.dct);
   V* col = spec + (size_t)cg * P.stride * G + c;
@@ -1245,7 +1250,7 @@ static void launch_rows_inv(cup2d_ctx* c, const cplx<S>* spec, int spec_rows, vo
 template <int LC, int MODE, typename S>
 static int launch_cols(cup2d_ctx* c, cplx<S>* spec, int ncg, const ColParams& P,
                        const cplx<S>* tw) {
-  constexpr int CE = col_e<LC>();
+  constexpr int CE = col_e<LC, MODE>(), CW = col_cw<LC>();
   if (MODE == 1 && 2 * P.rows > LC) return CUP2D_ERR_ARG;  // k_cols reads rows < LC/2 only
   const size_t shm = (size_t)lds_len<LC, CE>() * CW * sizeof(cplx<S>);
   const dim3 grid(ncg * (G / CW)), block(CW * LC / CE);
@@ -1324,21 +1329,27 @@ static void set_rows_attr() {
   set_rows_attr_S<L, KIND, double>();
   set_rows_attr_S<L, KIND, float>();
 }
+template <int LC, int MODE, typename S>
+static void set_cols_attr_M() {
+  constexpr int CE = col_e<LC, MODE>(), CW = col_cw<LC>();
+  const int shm = lds_len<LC, CE>() * CW * (int)sizeof(cplx<S>);
+  if constexpr (MODE == 3 || MODE == 5)
+    set_shm((const void*)k_cols_cos<LC, CE, MODE, S>, shm);
+  else
+    set_shm((const void*)k_cols<LC, MODE, CE, S>, shm);
+}
 template <int LC>
 static void set_cols_attr() {
-  constexpr int CE = col_e<LC>();
-  const int shm = lds_len<LC, CE>() * CW * (int)sizeof(double2);
-  const int shm32 = lds_len<LC, CE>() * CW * (int)sizeof(float2);
-  set_shm((const void*)k_cols<LC, 0, CE, double>, shm);
-  set_shm((const void*)k_cols<LC, 1, CE, double>, shm);
-  set_shm((const void*)k_cols<LC, 2, CE, double>, shm);
-  set_shm((const void*)k_cols<LC, 4, CE, double>, shm);
-  set_shm((const void*)k_cols<LC, 0, CE, float>, shm32);
-  set_shm((const void*)k_cols<LC, 1, CE, float>, shm32);
+  set_cols_attr_M<LC, 0, double>();
+  set_cols_attr_M<LC, 1, double>();
+  set_cols_attr_M<LC, 2, double>();
+  set_cols_attr_M<LC, 4, double>();
+  set_cols_attr_M<LC, 0, float>();
+  set_cols_attr_M<LC, 1, float>();
   if constexpr (2 * LC <= MAX_LC) {
-    set_shm((const void*)k_cols_cos<LC, CE, 3, double>, shm);
-    set_shm((const void*)k_cols_cos<LC, CE, 5, double>, shm);
-    set_shm((const void*)k_cols_cos<LC, CE, 3, float>, shm32);
+    set_cols_attr_M<LC, 3, double>();
+    set_cols_attr_M<LC, 5, double>();
+    set_cols_attr_M<LC, 3, float>();
   }
 }
 // the kernels of one plan's lengths and kind
