@@ -183,13 +183,15 @@ int pressure_single(cup2d_ctx* c, int fused) {
   if (fused && c->flux_deferred) {
     RC(join_obstacles(c));
     RC(enqueue_rhs_obstacles(c, 1));
-    // after an early row pass the fade factor is already reduced (the patch
-    // pass reduces the final one itself when it has to redo the pass)
-    if (c->rows_early)
+    // after an early row pass, or with the fused front, the fade factor is
+    // already reduced (the row pass reduces the final one itself when an
+    // obstacle block lies in the fade band)
+    if (c->rows_early || c->front_fused)
       c->fade_early = false;
     else
       RC(enqueue_fade_sums(c, 1));
     RC(enqueue_poisson_fft(c, c->rhs, c->pres, 2));
+    c->front_fused = false;
   } else {
     // the side stream may still be writing the advDiff output that the RHS
     // reads (swimmer layout: advDiff runs beside the placement chain)
@@ -252,14 +254,26 @@ int advance_enqueued(cup2d_ctx* c, int compute_dt) {
   // (with overlap, also the swimmers' time-only midline part of the next
   // step, off the critical path).  With swimmers the placement chain is
   // longer than advDiff: it keeps the main stream and advDiff goes beside it.
-  const bool chain_main = !c->hfish.empty() && !c->cfg.iterative_penal;
-  RC(enqueue_put_objects(c, compute_dt, chain_main ? 2 : 1));
+  // With disks only, placement, advDiff and the previous step's forces share
+  // launches on the main stream.
+  const bool fish = !c->hfish.empty(), chain_main = fish && !c->cfg.iterative_penal;
+  const bool front = !fish && c->g.nshapes > 0;
+  if (front)
+    RC(enqueue_step_front(c, compute_dt));
+  else
+    RC(enqueue_put_objects(c, compute_dt, chain_main ? 2 : (fish ? 1 : 0)));
   if (c->cfg.iterative_penal) {
-    RC(enqueue_advdiff(c, 0));
+    if (front) {
+      c->front_fused = false;
+      RC(flush_commit(c));
+      RC(enqueue_flux_fix(c, c->stream));
+    } else {
+      RC(enqueue_advdiff(c, 0));
+    }
     RC(pressure_iterator(c, nullptr, nullptr));
     RC(enqueue_find_max_u_partials(c));  // for the next step's dt
   } else {
-    if (!chain_main) RC(enqueue_advdiff(c, 1));
+    if (!front && !chain_main) RC(enqueue_advdiff(c, 1));
     RC(pressure_single(c, 1));
   }
   RC(enqueue_forces(c, 1, 1));

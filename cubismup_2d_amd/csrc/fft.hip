@@ -426,7 +426,9 @@ struct RowSource {
   const unsigned char* obmap;
   const void* dct;      // KIND_COS: w_k = exp(-i pi k / 2L), k <= L/2 (cplx<S>)
   int store_all;
-  const double* fadepart;  // SRC_PATCH redo: the fade sums' partials (npart x 3)
+  // the fade sums' partials (npart x 3): summed here when rows_redo is set
+  // (SRC_PATCH; SRC_DIV after enqueue_step_front, else nullptr)
+  const double* fadepart;
 };
 
 // Forward transform of a packed row pair held in x (x[q] = element t + q*NT
@@ -517,13 +519,13 @@ __device__ __forceinline__ void rows_fwd_group(int wg, const S* in, int in_pitch
       if (!__syncthreads_or(any)) return;
     }
   }
-  // the fade factor: k_fade_reduce's, or with a redo of the early pass the
-  // final one (the obstacle RHS kernel replaced the partials of the obstacle
-  // blocks in the band), reduced here in one fixed order by every workgroup
+  // the fade factor: the one reduced before, or with an obstacle block in the
+  // band (rows_redo) the final one (the obstacle RHS kernel replaced that
+  // block's partial), reduced here in one fixed order by every workgroup
   double fcorr = 0;
   if constexpr (SRC != SRC_PLAIN) fcorr = fd.st->fade_corr;
-  if constexpr (SRC == SRC_PATCH) {
-    if (fd.st->rows_redo != 0 && fd.npart > 0) {
+  if constexpr (DIV) {
+    if (fd.fadepart && fd.st->rows_redo != 0 && fd.npart > 0) {
       __shared__ double s_corr;
       if (threadIdx.x < 64) {
         double sums[3];
@@ -1624,7 +1626,8 @@ int enqueue_poisson_fft(cup2d_ctx* c, double* rhs, double* sol, int src) {
     {
       KernelTimer kt(c, patch ? T_RHS_OBST : T_FFT_ROWS_FWD);
       RowSource fd{c->g, c->band_nblocks > 0 ? fade_partials(c) : 0, rhs, c->st,
-                   c->u, c->v, c->obmap, P->dct_r, P->cs && src == SRC_DIV ? 1 : 0, c->red};
+                   c->u, c->v, c->obmap, P->dct_r, P->cs && src == SRC_DIV ? 1 : 0,
+                   patch || c->front_fused ? c->red : nullptr};
       rc = grid_rows_fwd<double>(c, rhs, P->spec, P->tw_r, src, fd);
     }
     if (rc) return rc;
@@ -1652,7 +1655,8 @@ int enqueue_poisson_fft(cup2d_ctx* c, double* rhs, double* sol, int src) {
   {
     KernelTimer kt(c, patch ? T_RHS_OBST : T_FFT_ROWS_FWD);
     RowSource fd{c->g, c->band_nblocks > 0 ? fade_partials(c) : 0, rhs, c->st,
-                 c->u, c->v, c->obmap, P->dct_r32, src != SRC_PLAIN ? 1 : 0, c->red};
+                 c->u, c->v, c->obmap, P->dct_r32, src != SRC_PLAIN ? 1 : 0,
+                   patch || c->front_fused ? c->red : nullptr};
     rc = grid_rows_fwd<float>(c, b, s32, twr32, src, fd);
   }
   if (rc) return rc;

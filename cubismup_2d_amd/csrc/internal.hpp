@@ -168,6 +168,7 @@ struct cup2d_ctx {
   hipEvent_t ev_mid = nullptr;
   bool obst_pending = false;
   bool commit_pending = false;  // the placement commit rides in the next obstacle RHS launch
+  bool front_fused = false;     // enqueue_step_front ran: the obstacle RHS launches take the fade sums
   // ComputeForces and the step end (time += dt) of the last whole step, not
   // enqueued yet.  The next whole step applies the step end in its list
   // builder and runs ComputeForces on the side stream after its obstacle
@@ -342,6 +343,7 @@ int enqueue_find_max_u_partials(cup2d_ctx* c);
 int enqueue_dt(cup2d_ctx* c);
 int enqueue_advdiff(cup2d_ctx* c, int defer_fix);
 int enqueue_advdiff_on(cup2d_ctx* c, int defer_fix, hipStream_t s);
+int enqueue_flux_fix(cup2d_ctx* c, hipStream_t s);
 int enqueue_pressure_rhs(cup2d_ctx* c);
 int stencil_edge_count(const cup2d_ctx* c);
 int enqueue_fade_sums(cup2d_ctx* c, int compute = 0);
@@ -381,6 +383,9 @@ int obstacles_alloc(cup2d_ctx* c);
 void obstacles_free(cup2d_ctx* c);
 constexpr int OBST_LIST_CAP = 2048;  // slots handled by the list builder
 int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap = 0);
+// The head of a whole step with disks only (PutObjectsOnGrid, advDiff and the
+// previous step's ComputeForces) in three launches on the main stream.
+int enqueue_step_front(cup2d_ctx* c, int compute_dt);
 int join_obstacles(cup2d_ctx* c);
 int flush_commit(cup2d_ctx* c);
 // compute: form the RHS of the obstacle blocks from the advDiff output first

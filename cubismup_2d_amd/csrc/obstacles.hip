@@ -13,6 +13,9 @@
 // Shape::computeForces (Shape.cpp:260-271).  Every workgroup that needs a
 // shape total recomputes it from the partials in the same order, so all of
 // them see bit-identical values.
+#include <type_traits>
+
+#include "advdiff.hpp"
 #include "device_util.hpp"
 #include "fish.hpp"
 
@@ -606,20 +609,17 @@ __device__ inline double grid_sdf(const Grid& g, const DiskLds& D, const Obstacl
 // distance evaluated once and shared through LDS instead of five times per
 // cell, and a thread's four cells in flight together, 13.4 -> 7.1 us at
 // 512 x 256 and 58 -> 27 us at 8192 x 4096 with 20 bodies.
-__global__ __launch_bounds__(NT) void k_obst_place(Grid g, const ShapeParams* __restrict__ sp,
-                                                   const cup2d_shape_state* __restrict__ ss,
-                                                   Obstacles ob, Obstacles pv,
-                                                   const unsigned char* __restrict__ obmap,
-                                                   const int* __restrict__ ubidx,
-                                                   double* __restrict__ chi,
-                                                   double* __restrict__ udx,
-                                                   double* __restrict__ udy,
-                                                   double* __restrict__ invrho) {
+__device__ void obst_place_wg(int w, const Grid& g, const ShapeParams* __restrict__ sp,
+                              const cup2d_shape_state* __restrict__ ss, const Obstacles& ob,
+                              const Obstacles& pv, const unsigned char* __restrict__ obmap,
+                              const int* __restrict__ ubidx, double* __restrict__ chi,
+                              double* __restrict__ udx, double* __restrict__ udy,
+                              double* __restrict__ invrho) {
   __shared__ double lds[LDS_RED];
   __shared__ int s_nbs[4][MAX_FISH];  // swimmer slots of the E, W, N, S neighbour blocks
   __shared__ int s_nbn[4];
   __shared__ DiskLds D;
-  const int nub = ob.cnt[1], w = blockIdx.x;
+  const int nub = ob.cnt[1];
   if (w >= nub) {
     if (w >= nub + pv.cnt[1]) return;
     const int b = pv.ub_block[w - nub];
@@ -762,6 +762,18 @@ __global__ __launch_bounds__(NT) void k_obst_place(Grid g, const ShapeParams* __
   }
 }
 
+__global__ __launch_bounds__(NT) void k_obst_place(Grid g, const ShapeParams* __restrict__ sp,
+                                                   const cup2d_shape_state* __restrict__ ss,
+                                                   Obstacles ob, Obstacles pv,
+                                                   const unsigned char* __restrict__ obmap,
+                                                   const int* __restrict__ ubidx,
+                                                   double* __restrict__ chi,
+                                                   double* __restrict__ udx,
+                                                   double* __restrict__ udy,
+                                                   double* __restrict__ invrho) {
+  obst_place_wg(blockIdx.x, g, sp, ss, ob, pv, obmap, ubidx, chi, udx, udy, invrho);
+}
+
 // centre of mass after putChiOnGrid (PutObjectsOnGrid.cpp:118-122) from the
 // totals t[0..3) of the COM partials, without touching the stored state
 __device__ inline void com_from_sums(const cup2d_shape_state* ss, int k, const double* t,
@@ -786,19 +798,19 @@ __device__ inline void shape_com(const Obstacles& ob, const cup2d_shape_state* s
 
 // Shape::integrateObstBlock (Shape.cpp:117-155): per-slot partials about the
 // updated centre of mass.
-__device__ void obst_moments_wg(const Grid& g, const cup2d_shape_state* __restrict__ ss,
+__device__ void obst_moments_wg(int s, const Grid& g, const cup2d_shape_state* __restrict__ ss,
                                 const Obstacles& ob, double* lds);
 
 __global__ __launch_bounds__(NT) void k_obst_moments(Grid g, const cup2d_shape_state* __restrict__ ss,
                                                      const StepState* __restrict__ st,
                                                      Obstacles ob) {
   __shared__ double lds[LDS_RED];
-  if ((int)blockIdx.x < ob.cnt[0]) obst_moments_wg(g, ss, ob, lds);
+  if ((int)blockIdx.x < ob.cnt[0]) obst_moments_wg(blockIdx.x, g, ss, ob, lds);
 }
 
-__device__ void obst_moments_wg(const Grid& g, const cup2d_shape_state* __restrict__ ss,
+__device__ void obst_moments_wg(int s, const Grid& g, const cup2d_shape_state* __restrict__ ss,
                                 const Obstacles& ob, double* lds) {
-  const int s = blockIdx.x, k = ob.slot_shape[s], b = ob.slot_block[s];
+  const int k = ob.slot_shape[s], b = ob.slot_block[s];
   const int bx = b % g.bpdx, by = b / g.bpdx;
   SlotView o = slot(ob, s);
   const double hsq = g.h * g.h;
@@ -934,10 +946,10 @@ static int launch_forces(cup2d_ctx* c, hipStream_t s, const Obstacles& lists, in
 // How much of the placement chain runs on the main stream before advDiff when
 // the chain runs beside it on the side stream (stages of enqueue_put_objects:
 // midline + list builder, PutFishOnBlocks, placement, moments, removeMoments,
-// commit): with swimmers the midline and list builder, with disks nothing.
+// commit; swimmers with the iterative penalization): the midline and list builder.
 // Beside advDiff, which saturates HBM, these latency-bound kernels run 2-3x
 // slower than alone; the split balances that against the main stream's wait.
-constexpr int SPLIT_FISH = 1, SPLIT_DISKS = 0;
+constexpr int SPLIT_FISH = 1;
 
 int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
   const int G = grid_cap(c);
@@ -982,7 +994,7 @@ int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
   // The chain's stages in order; the first `split` of them run on the main
   // stream before advDiff, the rest on the side stream beside it.
   enum { ST_MIDLINE, ST_FISH_PLACE, ST_PLACE, ST_MOMENTS, ST_UDEF, ST_COMMIT, ST_N };
-  const int split = !overlap || chain_main ? ST_N : (fish ? SPLIT_FISH : SPLIT_DISKS);
+  const int split = !overlap || chain_main ? ST_N : SPLIT_FISH;
   bool on_aux = false;
   auto stream_for = [&](int stage) -> hipStream_t {
     if (stage < split) return c->stream;
@@ -1061,10 +1073,8 @@ int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
     RC_OB(enqueue_fish_mid_next(c, c->host_step & 1, c->ev_begin, true));
     if (defer_forces)  // the previous step's ComputeForces, on its own lists
       RC_OB(launch_forces(c, c->aux, c->ob_prev, 0, u_prev, v_prev, 1));
-    if (defer_forces || !c->hfish.empty()) {
-      CUP2D_HIP_CHECK(c, hipEventRecord(c->ev_frc, c->aux));
-      c->frc_join = true;
-    }
+    CUP2D_HIP_CHECK(c, hipEventRecord(c->ev_frc, c->aux));
+    c->frc_join = true;
   }
   return launch_check(c, "put_objects");
 }
@@ -1123,21 +1133,14 @@ struct CellStage {
 // RT: the type of the RHS and velocity planes (double, or float at FP32
 // precision); the corrections are computed in double and stored rounded.
 template <typename RT>
-__global__ __launch_bounds__(NT) void k_rhs_obst1(Grid g, StepState* __restrict__ st,
-                                                  Obstacles ob, const double* __restrict__ chi,
-                                                  RT* __restrict__ r,
-                                                  const RT* __restrict__ u,
-                                                  const RT* __restrict__ v,
-                                                  cup2d_shape_state* __restrict__ commit_ss) {
-  __shared__ double lds[LDS_RED];
-  // k_rhs_obst2 sets it again when an obstacle block lies in the fade band
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->rows_redo = 0;
-  if (commit_ss && blockIdx.x == gridDim.x - 1) {  // the placement commit (k_obst_commit)
-    obst_commit_wg(g, commit_ss, ob);
-    return;
-  }
-  if ((int)blockIdx.x >= ob.cnt[1]) return;
-  const int b = ob.ub_block[blockIdx.x];
+__device__ void rhs_obst1_wg(int w, const Grid& g, StepState* __restrict__ st,
+                             const Obstacles& ob, const double* __restrict__ chi,
+                             RT* __restrict__ r, const RT* __restrict__ u,
+                             const RT* __restrict__ v, double* lds) {
+  // rhs_obst2_wg sets it again when an obstacle block lies in the fade band
+  if (w == 0 && threadIdx.x == 0) st->rows_redo = 0;
+  if (w >= ob.cnt[1]) return;
+  const int b = ob.ub_block[w];
   const int bx = b % g.bpdx, by = b / g.bpdx;
   if (u) {
     const RT corr = (RT)st->flux_corr;  // deferred advDiff flux correction
@@ -1147,7 +1150,7 @@ __global__ __launch_bounds__(NT) void k_rhs_obst1(Grid g, StepState* __restrict_
       r[(size_t)y * g.NX + x] = rhs_cell<RT>(u, v, g.NX, g.NY, x, y, corr, facDiv);
     }
   }
-  const int s0 = ob.ub_start[blockIdx.x], cnt = ob.ub_count[blockIdx.x];
+  const int s0 = ob.ub_start[w], cnt = ob.ub_count[w];
   for (int q = 0; q < cnt; ++q) {
     const int s = ob.ub_slots[s0 + q];
     SlotView o = slot(ob, s);
@@ -1175,21 +1178,33 @@ __global__ __launch_bounds__(NT) void k_rhs_obst1(Grid g, StepState* __restrict_
   }
 }
 
+template <typename RT>
+__global__ __launch_bounds__(NT) void k_rhs_obst1(Grid g, StepState* __restrict__ st,
+                                                  Obstacles ob, const double* __restrict__ chi,
+                                                  RT* __restrict__ r,
+                                                  const RT* __restrict__ u,
+                                                  const RT* __restrict__ v,
+                                                  cup2d_shape_state* __restrict__ commit_ss) {
+  __shared__ double lds[LDS_RED];
+  if (commit_ss && blockIdx.x == gridDim.x - 1)  // the placement commit (k_obst_commit)
+    obst_commit_wg(g, commit_ss, ob);
+  else
+    rhs_obst1_wg<RT>(blockIdx.x, g, st, ob, chi, r, u, v, lds);
+}
+
 // band_index != nullptr: the fade sums were formed from the advDiff output
 // before the obstacle RHS; the partial of an obstacle block in the fade band
 // is formed again here from its final RHS.
 template <typename RT>
-__global__ __launch_bounds__(NT) void k_rhs_obst2(Grid g, StepState* __restrict__ st,
-                                                  Obstacles ob, const double* __restrict__ chi,
-                                                  RT* __restrict__ r,
-                                                  const int* __restrict__ band_index,
-                                                  double* __restrict__ fadepart) {
+__device__ void rhs_obst2_wg(int w, const Grid& g, StepState* __restrict__ st,
+                             const Obstacles& ob, const double* __restrict__ chi,
+                             RT* __restrict__ r, const int* __restrict__ band_index,
+                             double* __restrict__ fadepart, double* lds) {
   static_assert(NT == 256, "fade_block_sums is a 256-thread reduction");
-  __shared__ double lds[12];
-  if ((int)blockIdx.x >= ob.cnt[1]) return;
-  const int b = ob.ub_block[blockIdx.x];
+  if (w >= ob.cnt[1]) return;
+  const int b = ob.ub_block[w];
   const int bx = b % g.bpdx, by = b / g.bpdx;
-  const int s0 = ob.ub_start[blockIdx.x], cnt = ob.ub_count[blockIdx.x];
+  const int s0 = ob.ub_start[w], cnt = ob.ub_count[w];
   for (int q = 0; q < cnt; ++q) {
     const int s = ob.ub_slots[s0 + q], k = ob.slot_shape[s];
     SlotView o = slot(ob, s);
@@ -1224,8 +1239,85 @@ __global__ __launch_bounds__(NT) void k_rhs_obst2(Grid g, StepState* __restrict_
   }
 }
 
+template <typename RT>
+__global__ __launch_bounds__(NT) void k_rhs_obst2(Grid g, StepState* __restrict__ st,
+                                                  Obstacles ob, const double* __restrict__ chi,
+                                                  RT* __restrict__ r,
+                                                  const int* __restrict__ band_index,
+                                                  double* __restrict__ fadepart) {
+  __shared__ double lds[12];
+  rhs_obst2_wg<RT>(blockIdx.x, g, st, ob, chi, r, band_index, fadepart, lds);
+}
+
+// The obstacle RHS launches of a step whose front was enqueue_step_front
+// (disks only): beside the G obstacle workgroups one takes the placement
+// commit and one per band block the fade sums, every block from the advDiff
+// output; then one reduces the fade factor, unless an obstacle block lies in
+// the fade band (its partial is being replaced, rows_redo is set and the row
+// pass reduces the final sums itself).
+template <typename RT>
+__global__ __launch_bounds__(NT) void k_step_rhs1(Grid g, StepState* __restrict__ st,
+                                                  Obstacles ob, int G,
+                                                  const double* __restrict__ chi,
+                                                  RT* __restrict__ r, const RT* __restrict__ u,
+                                                  const RT* __restrict__ v,
+                                                  cup2d_shape_state* __restrict__ commit_ss,
+                                                  const int* __restrict__ band_blocks,
+                                                  double* __restrict__ fadepart) {
+  __shared__ double lds[LDS_RED];
+  const int w = blockIdx.x;
+  if (w < G) {
+    rhs_obst1_wg<RT>(w, g, st, ob, chi, r, u, v, lds);
+  } else if (w == G) {
+    obst_commit_wg(g, commit_ss, ob);
+  } else {
+    const int j = w - G - 1;
+    const RT corr = (RT)st->flux_corr, facDiv = (RT)(0.5 * g.h / st->dt);
+    double a[3];
+    fade_block_sums<RT>(g, band_blocks[j], r, u, v, false, corr, facDiv, a, lds);
+    if (threadIdx.x == 0)
+      for (int q = 0; q < 3; ++q) fadepart[3 * j + q] = a[q];
+  }
+}
+template <typename RT>
+__global__ __launch_bounds__(NT) void k_step_rhs2(Grid g, StepState* __restrict__ st,
+                                                  Obstacles ob, int G,
+                                                  const double* __restrict__ chi,
+                                                  RT* __restrict__ r,
+                                                  const int* __restrict__ band_index,
+                                                  double* __restrict__ fadepart, int npart) {
+  __shared__ double lds[64];
+  const int w = blockIdx.x;
+  if (w < G) {
+    rhs_obst2_wg<RT>(w, g, st, ob, chi, r, band_index, fadepart, lds);
+    return;
+  }
+  int hit = 0;
+  for (int u = threadIdx.x; u < ob.cnt[1]; u += NT) hit |= band_index[ob.ub_block[u]] >= 0;
+  if (__syncthreads_or(hit)) return;
+  double sums[3];
+  block_sum_table<NT, 3>(fadepart, npart, 3, sums, lds);
+  if (threadIdx.x == 0) st->fade_corr = fade_corr_factor(sums[0], sums[1], sums[2]);
+}
+
+static int enqueue_step_rhs(cup2d_ctx* c) {
+  const int G = grid_cap(c), nb = c->band_nblocks;
+  TimerScope ts(c, T_RHS_OBST);
+  CUP2D_REAL_DISPATCH(c, hipLaunchKernelGGL(k_step_rhs1<T>, dim3(G + 1 + nb), dim3(NT), 0,
+                                            c->stream, c->g, c->st, c->ob, G, c->chi,
+                                            tp<T>(c->rhs), tp<T>(c->u), tp<T>(c->v), c->ss,
+                                            c->band_blocks, c->red));
+  CUP2D_REAL_DISPATCH(c, hipLaunchKernelGGL(k_step_rhs2<T>, dim3(nb > 0 ? G + 1 : G), dim3(NT), 0,
+                                            c->stream, c->g, c->st, c->ob, G, c->chi,
+                                            tp<T>(c->rhs), nb > 0 ? c->band_index : nullptr,
+                                            c->red, nb));
+  c->commit_pending = false;
+  return launch_check(c, "rhs_obstacles");
+}
+
 int enqueue_rhs_obstacles(cup2d_ctx* c, int compute) {
   if (c->g.nshapes == 0) return CUP2D_OK;
+  if (compute && c->front_fused) return enqueue_step_rhs(c);
   const int G = grid_cap(c);
   TimerScope ts(c, T_RHS_OBST);
   // a pending placement commit takes one more workgroup
@@ -1883,10 +1975,11 @@ __device__ void forces_fin_wg(const Grid& g, cup2d_shape_state* __restrict__ ss,
 
 // ComputeForces.cpp:16-107, per slot; surface points are the cells with D>0.
 template <typename RT>
-__device__ void forces_wg(const Grid& g, const ForceSnap* __restrict__ snap, const Obstacles& ob,
-                          const RT* __restrict__ u, const RT* __restrict__ v,
-                          const double* __restrict__ p, double* lds, const SurfVel& surf) {
-  const int s = blockIdx.x, k = ob.slot_shape[s], b = ob.slot_block[s];
+__device__ void forces_wg(int s, const Grid& g, const ForceSnap* __restrict__ snap,
+                          const Obstacles& ob, const RT* __restrict__ u,
+                          const RT* __restrict__ v, const double* __restrict__ p, double* lds,
+                          const SurfVel& surf) {
+  const int k = ob.slot_shape[s], b = ob.slot_block[s];
   const int bx = b % g.bpdx, by = b / g.bpdx;
   SlotView o = slot(ob, s);
   const double NUoH = g.nu / g.h;
@@ -1959,7 +2052,7 @@ __global__ __launch_bounds__(NT) void k_forces(Grid g, const ForceSnap* __restri
                                                const RT* __restrict__ v,
                                                const double* __restrict__ p, SurfVel sv) {
   __shared__ double lds[LDS_RED];
-  if ((int)blockIdx.x < ob.cnt[0]) forces_wg(g, snap, ob, u, v, p, lds, sv);
+  if ((int)blockIdx.x < ob.cnt[0]) forces_wg(blockIdx.x, g, snap, ob, u, v, p, lds, sv);
 }
 
 // shape totals (Shape::computeForces, Shape.cpp:252-300) and, with end_step,
@@ -1981,6 +2074,108 @@ static int launch_forces(cup2d_ctx* c, hipStream_t s, const Obstacles& lists, in
   hipLaunchKernelGGL(k_forces_fin, dim3(1), dim3(NT), 0, s, c->g, c->ss, lists, c->st, end_step,
                      c->fsnap, flog, deferred);
   return launch_check(c, "forces");
+}
+
+// ------------------------------------------------------- whole-step front
+// With disks only, the head of a whole step takes three launches on the main
+// stream: the list builder; then advDiff, the placement of every obstacle
+// block and the previous step's ComputeForces side by side in one grid; then
+// the moments, the flux reduction and the force totals.  (As kernels on two
+// streams the same work needed three cross-stream events per step, 6-9 us
+// each, and the totals waited for launches of one workgroup: whole step at
+// 512 x 256 107 -> 72 us, one disk on 4096 x 2048 317 -> 285 us.)  The parts of a launch touch disjoint data: the
+// placement writes this step's slots and the dense obstacle planes, the forces
+// read the previous step's lists, velocity and pressure.  The latency-bound
+// workgroups come first, so they start at once and the strips fill the rest.
+template <typename T, bool RAGGED>
+__global__ __launch_bounds__(256, 4) void k_step_place(
+    Grid g, const ShapeParams* __restrict__ sp, const cup2d_shape_state* __restrict__ ss,
+    Obstacles ob, Obstacles pv, const unsigned char* __restrict__ obmap,
+    const int* __restrict__ ubidx, double* __restrict__ chi, double* __restrict__ udx,
+    double* __restrict__ udy, double* __restrict__ invrho, int nplace, int nforces, int nfront,
+    const ForceSnap* __restrict__ snap, const double* __restrict__ p, SurfVel sv,
+    const T* __restrict__ u, const T* __restrict__ v, T* __restrict__ uo, T* __restrict__ vo,
+    const StepState* __restrict__ st, double* __restrict__ fluxpart, int gx, int gy) {
+  __shared__ double lds[LDS_RED];
+  int w = blockIdx.x;
+  if (w < nplace) {
+    obst_place_wg(w, g, sp, ss, ob, pv, obmap, ubidx, chi, udx, udy, invrho);
+    return;
+  }
+  if (w < nfront) {  // nfront: nplace + nforces rounded up to a multiple of 8
+    w -= nplace;
+    if (w < nforces && w < pv.cnt[0]) forces_wg(w, g, snap, pv, u, v, p, lds, sv);
+    return;
+  }
+  // the strips, each XCD's a contiguous band (workgroup b runs on XCD b % 8)
+  const int n = gx * gy, id = w - nfront;
+  const int t = (n % 8 == 0) ? (id % 8) * (n / 8) + id / 8 : id;
+  advdiff_strip<STENCIL_RY, RAGGED, T>(u, v, uo, vo, g, st, fluxpart, t % gx, t / gx, gx, gy, lds);
+}
+
+// G workgroups of moments, then the flux reduction, then (forces) the totals
+// of the previous step's ComputeForces.
+__global__ __launch_bounds__(NT) void k_step_moments(Grid g, cup2d_shape_state* __restrict__ ss,
+                                                     StepState* __restrict__ st, Obstacles ob,
+                                                     Obstacles pv, int G,
+                                                     const double* __restrict__ fluxpart, int gx,
+                                                     int gy, const ForceSnap* __restrict__ snap,
+                                                     ForceLog flog) {
+  __shared__ double lds[LDS_RED];
+  const int w = blockIdx.x;
+  if (w < G) {
+    if (w < ob.cnt[0]) obst_moments_wg(w, g, ss, ob, lds);
+  } else if (w == G) {
+    const double corr = flux_corr(fluxpart, edge_count(gx, gy), g, lds);
+    if (threadIdx.x == 0) st->flux_corr = corr;
+  } else {
+    forces_fin_wg(g, ss, pv, st, 0, snap, flog, 1);
+  }
+}
+
+int enqueue_step_front(cup2d_ctx* c, int compute_dt) {
+  const int G = grid_cap(c);
+  const bool forces = c->forces_pending;
+  const int end_prev = c->end_pending ? 1 : 0;
+  c->forces_pending = false;
+  c->end_pending = false;
+  RC_OB(join_forces(c));
+  std::swap(c->ob, c->ob_prev);
+  {
+    TimerScope ts(c, T_PUT_OBJECTS);
+    hipLaunchKernelGGL(k_obst_begin, dim3(1), dim3(NT), 0, c->stream, c->g, c->sp, c->ss, c->st,
+                       c->ob, c->ob_prev, c->obmap, c->ubidx, c->fishd, c->maxpart, c->nwg,
+                       c->ramp, compute_dt, c->graph_capture ? -1 : c->host_step, 0, end_prev);
+  }
+  const int NX = c->g.NX, gx = strips_x(NX), gy = c->g.NY / STENCIL_RY;
+  const int nplace = 2 * G, nforces = forces ? G : 0, nfront = (nplace + nforces + 7) / 8 * 8;
+  {
+    KernelTimer kt(c, T_ADVDIFF);
+    // strips narrower than a workgroup (NX < 256) are ragged ones of it
+    auto launch = [&](auto rg) {
+      constexpr bool RAGGED = rg();
+      CUP2D_REAL_DISPATCH(
+          c, CUP2D_TIMED_LAUNCH(c, (k_step_place<T, RAGGED>), dim3(nfront + gx * gy), dim3(256), 0,
+                                c->stream, c->g, (const ShapeParams*)c->sp,
+                                (const cup2d_shape_state*)c->ss, c->ob, c->ob_prev,
+                                (const unsigned char*)c->obmap, (const int*)c->ubidx, c->chi,
+                                c->udx, c->udy, c->invrho, nplace, nforces, nfront,
+                                (const ForceSnap*)c->fsnap, (const double*)c->pres, surf_of(c),
+                                tp<T>(c->u), tp<T>(c->v), tp<T>(c->tu), tp<T>(c->tv),
+                                (const StepState*)c->st, c->fluxpart, gx, gy));
+    };
+    if (NX % 256 != 0) launch(std::true_type{});
+    else launch(std::false_type{});
+  }
+  std::swap(c->u, c->tu);  // advDiff.cpp:81-87 copy tmpV -> vel
+  std::swap(c->v, c->tv);
+  c->flux_deferred = true;
+  const ForceLog flog{c->flog, c->flog_cnt, c->flog_cap};
+  hipLaunchKernelGGL(k_step_moments, dim3(forces ? G + 2 : G + 1), dim3(NT), 0, c->stream, c->g,
+                     c->ss, c->st, c->ob, c->ob_prev, G, c->fluxpart, gx, gy, c->fsnap, flog);
+  c->commit_pending = true;
+  c->front_fused = true;
+  return launch_check(c, "step front");
 }
 
 // ComputeForces::operator() + the step end.  on_aux: defer it to the side
