@@ -144,22 +144,42 @@ int ensure_frozen(cup2d_ctx* c) {
   return CUP2D_OK;
 }
 
-int sync_all(cup2d_ctx* c) {
+// everything pending enqueued and the main stream behind the side streams
+int enqueue_pending(cup2d_ctx* c) {
   RC(join_obstacles(c));
   RC(flush_commit(c));
   RC(flush_forces(c));
   RC(join_obstacles(c));
-  RC(join_forces(c));
-  CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->mids));
-  CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->aux));
+  return join_forces(c);
+}
+int wait_streams(cup2d_ctx* c) {
+  if (c->side_used) {
+    CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->mids));
+    CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->aux));
+    c->side_used = false;
+  }
   CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->stream));
   return CUP2D_OK;
 }
+int sync_all(cup2d_ctx* c) {
+  RC(enqueue_pending(c));
+  return wait_streams(c);
+}
+
+// The step scalars (and one shape's state) after everything enqueued so far,
+// in c->mail: a kernel of one wave writes them to pinned host memory, so one
+// stream wait replaces a wait and a device-to-host copy, which took about as
+// long as a small step's whole solve (a cosine solve of 1024 x 512 through
+// cup2d_poisson_solve 43 -> 33 us).
+int fetch_state(cup2d_ctx* c, int shape = -1) {
+  RC(enqueue_pending(c));
+  RC(enqueue_publish(c, shape));
+  return wait_streams(c);
+}
 
 int sync_and_check(cup2d_ctx* c) {
-  RC(sync_all(c));
-  int err = 0;
-  CUP2D_HIP_CHECK(c, hipMemcpy(&err, &c->st->error, sizeof(int), hipMemcpyDeviceToHost));
+  RC(fetch_state(c));
+  const int err = c->mail->st.error;
   if (err == CUP2D_ERR_BODY_OUT) return fail(c, err, "a body left the domain");
   if (err == CUP2D_ERR_CAPACITY) return fail(c, err, "obstacle-block pool exhausted");
   if (err == CUP2D_ERR_NONFINITE)
@@ -211,20 +231,18 @@ int pressure_single(cup2d_ctx* c, int fused) {
 int pressure_iterator(cup2d_ctx* c, int* iters_out, double* reldf_out) {
   RC(need_fft(c));
   RC(join_obstacles(c));
-  double* d_reldf = c->red + 4096 - 8;
   RC(enqueue_copy_vel_to_tmpv(c));
   int iter;
   double relDF = 1e3;
   for (iter = 0; iter < 1000; ++iter) {
     RC(enqueue_iter_project(c));
     RC(enqueue_iter_body(c));
-    RC(enqueue_iter_penalize(c, d_reldf));
+    RC(enqueue_iter_penalize(c, &c->mail_dev->reldf));
     RC(enqueue_iter_rhs(c));
     RC(enqueue_fade_sums(c));
     RC(enqueue_poisson_fft(c, c->rhs, c->pres, 1));
-    CUP2D_HIP_CHECK(c, hipMemcpyAsync(&relDF, d_reldf, sizeof(double), hipMemcpyDeviceToHost,
-                                      c->stream));
     CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->stream));
+    relDF = c->mail->reldf;
     const bool conv = relDF < c->iter_target || iter > 100 || iter > 2 * c->iter_old_nsteps;
     if (conv) {
       RC(enqueue_pressure_correction(c, 0));  // finalizePressure (:186-212)
@@ -557,6 +575,8 @@ int cup2d_create(const cup2d_cfg* cfg, cup2d_ctx** out) {
       hipEventCreateWithFlags(&c->ev_fork, CUP2D_SYNC_EVENT_FLAGS) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_qaux, CUP2D_SYNC_EVENT_FLAGS) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_qmid, CUP2D_SYNC_EVENT_FLAGS) != hipSuccess ||
+      hipHostMalloc((void**)&c->mail, sizeof(HostMail), hipHostMallocMapped) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&c->mail_dev, c->mail, 0) != hipSuccess ||
       hipMalloc(&c->fsnap, sizeof(ForceSnap) * MAX_SHAPES) != hipSuccess ||
       hipMalloc(&c->surf_coef, sizeof(double) * 4 * SURF_MAX_MODES) != hipSuccess) {
     c->err = "side stream creation failed";
@@ -668,6 +688,7 @@ int cup2d_destroy(cup2d_ctx* c) {
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_qaux) (void)hipEventDestroy(c->ev_qaux);
   if (c->ev_qmid) (void)hipEventDestroy(c->ev_qmid);
+  if (c->mail) (void)hipHostFree(c->mail);
   if (c->fsnap) (void)hipFree(c->fsnap);
   if (c->surf_coef) (void)hipFree(c->surf_coef);
   adjoint_free(c);
@@ -797,9 +818,8 @@ int cup2d_field_device_ptr(cup2d_ctx* c, int f, int comp, void** dptr) {
 int cup2d_get_scalars(cup2d_ctx* c, double* time, double* dt, int* step, double uinf[2],
                       double* h) {
   CHECK_CTX(c);
-  RC(sync_all(c));
-  StepState s;
-  CUP2D_HIP_CHECK(c, hipMemcpy(&s, c->st, sizeof(s), hipMemcpyDeviceToHost));
+  RC(fetch_state(c));
+  const StepState& s = c->mail->st;
   if (time) *time = s.time;
   if (dt) *dt = s.dt;
   if (step) *step = s.step;
@@ -823,8 +843,8 @@ int cup2d_set_scalars(cup2d_ctx* c, double time, int step, double uinfx, double 
 int cup2d_get_shape(cup2d_ctx* c, int i, cup2d_shape_state* out) {
   CHECK_CTX(c);
   if (i < 0 || i >= c->g.nshapes || !out) return fail(c, CUP2D_ERR_ARG, "bad shape id");
-  RC(sync_all(c));
-  CUP2D_HIP_CHECK(c, hipMemcpy(out, c->ss + i, sizeof(*out), hipMemcpyDeviceToHost));
+  RC(fetch_state(c, i));
+  *out = c->mail->ss;
   return CUP2D_OK;
 }
 
@@ -863,21 +883,17 @@ int cup2d_reset(cup2d_ctx* c) {
 int cup2d_find_max_u(cup2d_ctx* c, double* maxU) {
   CHECK_CTX(c);
   RC(enqueue_find_max_u(c));
-  CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-  StepState s;
-  CUP2D_HIP_CHECK(c, hipMemcpy(&s, c->st, sizeof(s), hipMemcpyDeviceToHost));
-  if (maxU) *maxU = s.maxU;
-  return sync_and_check(c);
+  const int rc = sync_and_check(c);
+  if (maxU && rc != CUP2D_ERR_HIP) *maxU = c->mail->st.maxU;
+  return rc;
 }
 
 int cup2d_calc_max_timestep(cup2d_ctx* c, double* dt) {
   CHECK_CTX(c);
   RC(enqueue_dt(c));
-  CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-  StepState s;
-  CUP2D_HIP_CHECK(c, hipMemcpy(&s, c->st, sizeof(s), hipMemcpyDeviceToHost));
-  if (dt) *dt = s.dt;
-  return sync_and_check(c);
+  const int rc = sync_and_check(c);
+  if (dt && rc != CUP2D_ERR_HIP) *dt = c->mail->st.dt;
+  return rc;
 }
 
 int cup2d_put_objects(cup2d_ctx* c, double dt) {

@@ -899,6 +899,7 @@ int enqueue_fish_midline(cup2d_ctx* c, hipStream_t s) {
 // otherwise the caller orders the main stream after the midline stream.
 int enqueue_fish_mid_next(cup2d_ctx* c, int parity, hipEvent_t after, bool join_aux) {
   if (c->hfish.empty()) return CUP2D_OK;
+  c->side_used = true;
   // `after` follows this step's midline kernels, which share the work arrays
   CUP2D_HIP_CHECK(c, hipStreamWaitEvent(c->mids, after, 0));
   hipLaunchKernelGGL(k_fish_mid_a, dim3((int)c->hfish.size()), dim3(NT), 0, c->mids, c->fishd,

@@ -132,6 +132,14 @@ struct Obstacles {
 
 struct FFTPlan;  // fft.hip
 
+// Host memory that kernels write: the step scalars, one shape's state and the
+// iterative penalization's relDF, read by the host after a stream wait.
+struct HostMail {
+  StepState st;
+  cup2d_shape_state ss;
+  double reldf;
+};
+
 // Per-kernel HIP-event timers (the role of SimulationData::startProfiler /
 // stopProfiler, SimulationData.cpp:187-205): when enabled, every launch of
 // the kernel is bracketed by two events on the context's stream.
@@ -161,6 +169,9 @@ struct cup2d_ctx {
   hipStream_t aux = nullptr;
   hipEvent_t ev_begin = nullptr, ev_obst = nullptr, ev_pen = nullptr, ev_frc = nullptr;
   hipEvent_t ev_lists = nullptr;  // this step's midline and lists done (main stream)
+  bool side_used = false;  // work enqueued on aux or mids since the host last waited for them
+  cup2d::HostMail* mail = nullptr;      // pinned host memory
+  cup2d::HostMail* mail_dev = nullptr;  // the same in the device's address space
   // third stream: the swimmers' time-only midline part of the next step runs
   // there beside advDiff (a kernel with many workgroups, so one more resident
   // workgroup costs it nothing); the side stream joins it (ev_mid) while idle
@@ -355,6 +366,7 @@ int enqueue_set_dt(cup2d_ctx* c, double dt);
 int enqueue_ic(cup2d_ctx* c);
 int enqueue_apply_obj_vel(cup2d_ctx* c);
 int enqueue_step_end(cup2d_ctx* c);
+int enqueue_publish(cup2d_ctx* c, int shape);  // st (and shape >= 0) to the host mailbox
 // f32: the planes hold float (the velocity and RHS planes at FP32 precision)
 int enqueue_blocks_to_dense(cup2d_ctx* c, const double* stage, double* a, double* b, int nc,
                             bool f32 = false);

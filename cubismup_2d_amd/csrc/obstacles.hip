@@ -981,6 +981,7 @@ int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
   auto launch_side = [&]() -> int {
     CUP2D_HIP_CHECK(c, hipEventRecord(c->ev_begin, c->stream));
     CUP2D_HIP_CHECK(c, hipStreamWaitEvent(c->aux, c->ev_begin, 0));
+    c->side_used = true;
     RC_OB(enqueue_advdiff_on(c, 1, c->aux));
     RC_OB(enqueue_fade_sums_early(c, c->aux));
     // the forward row FFT of the RHS without the obstacle correction, which
@@ -1000,6 +1001,7 @@ int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
     if (stage < split) return c->stream;
     if (!on_aux) {  // first side-stream stage: the side stream joins here
       on_aux = true;
+      c->side_used = true;
       if (hipEventRecord(c->ev_begin, c->stream) != hipSuccess ||
           hipStreamWaitEvent(c->aux, c->ev_begin, 0) != hipSuccess)
         return nullptr;

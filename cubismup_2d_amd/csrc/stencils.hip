@@ -114,6 +114,24 @@ __global__ void k_step_end(StepState* st) {
   st->time += st->dt;
   st->step += 1;
 }
+// The step scalars, and with s != nullptr a shape's state, to the host mailbox.
+__global__ void k_publish(const StepState* __restrict__ st,
+                          const cup2d_shape_state* __restrict__ s, HostMail* __restrict__ m) {
+  static_assert(sizeof(StepState) % 8 == 0 && sizeof(cup2d_shape_state) % 8 == 0, "64-bit words");
+  const unsigned long long* a = reinterpret_cast<const unsigned long long*>(st);
+  unsigned long long* b = reinterpret_cast<unsigned long long*>(&m->st);
+  for (int i = threadIdx.x; i < (int)(sizeof(*st) / 8); i += 64) b[i] = a[i];
+  if (!s) return;
+  a = reinterpret_cast<const unsigned long long*>(s);
+  b = reinterpret_cast<unsigned long long*>(&m->ss);
+  for (int i = threadIdx.x; i < (int)(sizeof(*s) / 8); i += 64) b[i] = a[i];
+}
+int enqueue_publish(cup2d_ctx* c, int shape) {
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, c->stream, c->st,
+                     shape >= 0 ? c->ss + shape : nullptr, c->mail_dev);
+  return launch_check(c, "publish");
+}
+
 int enqueue_step_end(cup2d_ctx* c) {
   hipLaunchKernelGGL(k_step_end, dim3(1), dim3(1), 0, c->stream, c->st);
   return launch_check(c, "step_end");
