@@ -508,6 +508,41 @@ __global__ void k_adj_acc_drag(const cup2d_shape_state* __restrict__ ss, int sha
   if (threadIdx.x == 0) *J += w * ss[shape].drag;
 }
 
+// The stored copies of a recomputed step, two cells per thread and iteration
+// (NX is even): the advDiff output with the deferred boundary-flux correction
+// (advDiff.cpp:107-115), and the step's velocity and pressure.
+__global__ __launch_bounds__(ANT) void k_adj_record_w(Grid g, const StepState* __restrict__ st,
+                                                      const double* __restrict__ u,
+                                                      const double* __restrict__ v,
+                                                      double* __restrict__ wu,
+                                                      double* __restrict__ wv) {
+  const double corr = st->flux_corr;
+  const size_t n2 = (size_t)g.NX * g.NY / 2;
+  for (size_t j = (size_t)blockIdx.x * ANT + threadIdx.x; j < n2; j += (size_t)gridDim.x * ANT) {
+    double2 a = reinterpret_cast<const double2*>(u)[j], b = reinterpret_cast<const double2*>(v)[j];
+    const int x = (int)(2 * j % g.NX), y = (int)(2 * j / g.NX);
+    a.x = flux_fixed<double>(a.x, x, g.NX, corr);
+    a.y = flux_fixed<double>(a.y, x + 1, g.NX, corr);
+    b.x = flux_fixed<double>(b.x, y, g.NY, corr);
+    b.y = flux_fixed<double>(b.y, y, g.NY, corr);
+    reinterpret_cast<double2*>(wu)[j] = a;
+    reinterpret_cast<double2*>(wv)[j] = b;
+  }
+}
+__global__ __launch_bounds__(ANT) void k_adj_record(size_t n2, const double2* __restrict__ u,
+                                                    const double2* __restrict__ v,
+                                                    const double2* __restrict__ p,
+                                                    double2* __restrict__ cu,
+                                                    double2* __restrict__ cv,
+                                                    double2* __restrict__ cp) {
+  for (size_t j = (size_t)blockIdx.x * ANT + threadIdx.x; j < n2; j += (size_t)gridDim.x * ANT) {
+    const double2 a = u[j], b = v[j];
+    cu[j] = a;
+    cv[j] = b;
+    if (cp) cp[j] = p[j];
+  }
+}
+
 __global__ __launch_bounds__(ANT) void k_adj_fill(double* a, size_t n, double val) {
   for (size_t j = (size_t)blockIdx.x * ANT + threadIdx.x; j < n; j += (size_t)gridDim.x * ANT)
     a[j] = val;
@@ -520,6 +555,18 @@ namespace cup2d {
 int enqueue_adjoint_fill(cup2d_ctx* c, double* a, size_t n, double val) {
   hipLaunchKernelGGL(k_adj_fill, dim3(1024), dim3(ANT), 0, c->stream, a, n, val);
   return launch_check(c, "adjoint fill");
+}
+
+int enqueue_adjoint_record_w(cup2d_ctx* c, double* wu, double* wv) {
+  hipLaunchKernelGGL(k_adj_record_w, dim3(1024), dim3(ANT), 0, c->stream, c->g, c->st, c->u, c->v,
+                     wu, wv);
+  return launch_check(c, "adjoint record");
+}
+int enqueue_adjoint_record(cup2d_ctx* c, double* u, double* v, double* p) {
+  hipLaunchKernelGGL(k_adj_record, dim3(1024), dim3(ANT), 0, c->stream,
+                     (size_t)c->g.NX * c->g.NY / 2, (const double2*)c->u, (const double2*)c->v,
+                     (const double2*)c->pres, (double2*)u, (double2*)v, (double2*)p);
+  return launch_check(c, "adjoint record");
 }
 
 int enqueue_adjoint_acc_drag(cup2d_ctx* c, int shape, double w, double* J) {

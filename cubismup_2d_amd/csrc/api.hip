@@ -413,6 +413,8 @@ struct AdjointState {
   double* theta_part = nullptr;
   double* theta = nullptr;             // [4M]
   double* scal = nullptr;              // J, flux sum
+  double* dts_dev = nullptr;           // [dts_cap] the forward run's time steps
+  int dts_cap = 0;
   bool ready = false;                  // a forward run whose backward may follow
 };
 
@@ -421,7 +423,7 @@ void adjoint_free(cup2d_ctx* c) {
   AdjointState* a = c->adj;
   if (!a) return;
   for (double* p : a->ck) (void)hipFree(p);
-  for (double* p : {a->seg, a->work, a->part, a->theta_part, a->theta, a->scal})
+  for (double* p : {a->seg, a->work, a->part, a->theta_part, a->theta, a->scal, a->dts_dev})
     if (p) (void)hipFree(p);
   delete a;
   c->adj = nullptr;
@@ -445,23 +447,18 @@ int adjoint_eligible(cup2d_ctx* c) {
   return need_fft(c);
 }
 
-// one forward step at fixed dt, operator by operator on the main stream
-// (put objects, advDiff with its flux correction, PressureSingle, forces and
-// the step end); rec != nullptr stores the flux-corrected advDiff output and
-// the pressure there.
-int adjoint_fwd_step(cup2d_ctx* c, double dt, double* rec_w, double* rec_p) {
+// One step of a recomputed segment at its recorded dt: Simulation::advance
+// without ComputeForces (the objective is known, the shape state is restored
+// afterwards); stores the flux-corrected advDiff output, the step's velocity
+// and its pressure.
+int adjoint_recompute_step(cup2d_ctx* c, double dt, double* w, double* u1, double* p) {
   const size_t n = (size_t)c->g.NX * c->g.NY;
   RC(enqueue_set_dt(c, dt));
-  RC(enqueue_put_objects(c, 0, 0));
-  RC(enqueue_advdiff(c, 0));
-  if (rec_w) {
-    CUP2D_HIP_CHECK(c, hipMemcpyAsync(rec_w, c->u, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-    CUP2D_HIP_CHECK(c, hipMemcpyAsync(rec_w + n, c->v, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-  }
-  RC(pressure_single(c, 0));
-  RC(enqueue_forces(c, 1, 0));
-  if (rec_p)
-    CUP2D_HIP_CHECK(c, hipMemcpyAsync(rec_p, c->pres, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
+  RC(enqueue_step_front(c, 0));
+  RC(enqueue_adjoint_record_w(c, w, w + n));
+  RC(pressure_single(c, 1));
+  RC(enqueue_adjoint_record(c, u1, u1 + n, p));
+  c->end_pending = true;
   return CUP2D_OK;
 }
 
@@ -1047,6 +1044,13 @@ int cup2d_adjoint_forward(cup2d_ctx* c, int nsteps, int every, const double* dts
     CUP2D_HIP_CHECK(c, hipMalloc(&a->theta, sizeof(double) * 4 * SURF_MAX_MODES));
     CUP2D_HIP_CHECK(c, hipMalloc(&a->scal, sizeof(double) * 4));
   }
+  if (a->dts_cap < nsteps) {
+    if (a->dts_dev) (void)hipFree(a->dts_dev);
+    a->dts_dev = nullptr;
+    a->dts_cap = 0;
+    CUP2D_HIP_CHECK(c, hipMalloc(&a->dts_dev, sizeof(double) * nsteps));
+    a->dts_cap = nsteps;
+  }
   a->ck_st.assign(nseg + 1, StepState{});
   a->ck_ss.assign(nseg + 1, {});
   a->nsteps = nsteps;
@@ -1056,24 +1060,25 @@ int cup2d_adjoint_forward(cup2d_ctx* c, int nsteps, int every, const double* dts
   RC(enqueue_adjoint_fill(c, a->scal, 1, 0.0));
   RC(adjoint_save(c, 0));
   const double wJ = 1.0 / nsteps;
+  // whole steps as Simulation::simulate takes them, dt on the device (from
+  // the findMaxU partials) unless given; a step's drag is added by the next
+  // step's front or behind the forces flushed for a checkpoint
+  if (!dts_in) RC(enqueue_find_max_u_partials(c));
   for (int k = 0; k < nsteps; ++k) {
-    double dt;
-    if (dts_in) {
-      dt = dts_in[k];
-    } else {  // Simulation::calcMaxTimestep
-      RC(enqueue_dt(c));
-      StepState s;
-      CUP2D_HIP_CHECK(c, hipMemcpyAsync(&s, c->st, sizeof(s), hipMemcpyDeviceToHost, c->stream));
-      CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-      dt = s.dt;
-    }
-    a->dts[k] = dt;
-    RC(adjoint_fwd_step(c, dt, nullptr, nullptr));
+    if (dts_in) RC(enqueue_set_dt(c, dts_in[k]));
+    RC(enqueue_step_front(c, dts_in ? 0 : 1, FrontAcc{a->scal, wJ, a->dts_dev, k}));
+    RC(pressure_single(c, 1));
+    RC(enqueue_forces(c, 1, 1));
     c->host_step += 1;
-    RC(enqueue_adjoint_acc_drag(c, 0, wJ, a->scal));
-    if ((k + 1) % every == 0 && k + 1 < nsteps) RC(adjoint_save(c, (k + 1) / every));
+    if ((k + 1) % every == 0 || k + 1 == nsteps) {
+      RC(flush_forces(c));
+      RC(enqueue_adjoint_acc_drag(c, 0, wJ, a->scal));
+      // (k + 1 == nsteps: the final state, restored after the backward sweep)
+      RC(adjoint_save(c, k + 1 == nsteps ? nseg : (k + 1) / every));
+    }
   }
-  RC(adjoint_save(c, nseg));  // the final state, restored after the backward sweep
+  CUP2D_HIP_CHECK(c, hipMemcpy(a->dts.data(), a->dts_dev, sizeof(double) * nsteps,
+                               hipMemcpyDeviceToHost));
   {
     const StepState& s = a->ck_st[nseg];
     a->uinf0 = s.uinf[0];
@@ -1118,13 +1123,13 @@ int cup2d_adjoint_backward(cup2d_ctx* c, double* grad) {
     const int k0 = sgi * K, len = std::min(K, N - k0);
     RC(adjoint_restore(c, sgi));
     // recompute the segment, storing each step's input, advDiff output and pressure
+    RC(enqueue_adjoint_record(c, segU, segU + n, nullptr));
     for (int j = 0; j < len; ++j) {
-      CUP2D_HIP_CHECK(c, hipMemcpyAsync(segU + 2 * n * j, c->u, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-      CUP2D_HIP_CHECK(c, hipMemcpyAsync(segU + 2 * n * j + n, c->v, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-      RC(adjoint_fwd_step(c, a->dts[k0 + j], segW + 2 * n * j, segP + n * j));
+      RC(adjoint_recompute_step(c, a->dts[k0 + j], segW + 2 * n * j, segU + 2 * n * (j + 1),
+                                segP + n * j));
+      c->host_step += 1;
     }
-    CUP2D_HIP_CHECK(c, hipMemcpyAsync(segU + 2 * n * len, c->u, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
-    CUP2D_HIP_CHECK(c, hipMemcpyAsync(segU + 2 * n * len + n, c->v, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
+    RC(flush_forces(c));  // the last step's end
     for (int j = len - 1; j >= 0; --j) {
       AdjStep s{};
       s.shape = 0;

@@ -422,6 +422,8 @@ __device__ inline void surf_vel(const SurfVel& sv, double p0, double p1, double*
   const double zr = r > 0 ? p0 / r : 1.0, zi = r > 0 ? p1 / r : 0.0;
   double wr = 1, wi = 0, un = 0, ut = 0;
   const int M = sv.M;
+  // (unrolled so that the coefficients of four modes are loaded together)
+#pragma unroll 4
   for (int m = 0; m < M; ++m) {
     const double tr = wr * zr - wi * zi;
     wi = wr * zi + wi * zr;

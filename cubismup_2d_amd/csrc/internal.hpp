@@ -397,7 +397,15 @@ constexpr int OBST_LIST_CAP = 2048;  // slots handled by the list builder
 int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap = 0);
 // The head of a whole step with disks only (PutObjectsOnGrid, advDiff and the
 // previous step's ComputeForces) in three launches on the main stream.
-int enqueue_step_front(cup2d_ctx* c, int compute_dt);
+// acc (the adjoint's forward run): dts[k] receives this step's dt, and *J the
+// weighted drag of the previous step if its forces are part of the launches.
+struct FrontAcc {
+  double* J;     // nullptr: none
+  double w;
+  double* dts;
+  int k;
+};
+int enqueue_step_front(cup2d_ctx* c, int compute_dt, const FrontAcc& acc = FrontAcc{});
 int join_obstacles(cup2d_ctx* c);
 int flush_commit(cup2d_ctx* c);
 // compute: form the RHS of the obstacle blocks from the advDiff output first
@@ -432,6 +440,10 @@ struct AdjStep {
 int enqueue_adjoint_step(cup2d_ctx* c, const AdjStep& a);
 int enqueue_adjoint_fill(cup2d_ctx* c, double* a, size_t n, double val);
 int enqueue_adjoint_acc_drag(cup2d_ctx* c, int shape, double w, double* J);
+// copies of the velocity, with the deferred flux correction applied (w), or of
+// the velocity and the pressure
+int enqueue_adjoint_record_w(cup2d_ctx* c, double* wu, double* wv);
+int enqueue_adjoint_record(cup2d_ctx* c, double* u, double* v, double* p);
 
 // fish.hip
 // FishData::FishData + width table (FishLibrary.cpp:14-38); returns Nm or -1

@@ -2122,20 +2122,25 @@ __global__ __launch_bounds__(NT) void k_step_moments(Grid g, cup2d_shape_state* 
                                                      Obstacles pv, int G,
                                                      const double* __restrict__ fluxpart, int gx,
                                                      int gy, const ForceSnap* __restrict__ snap,
-                                                     ForceLog flog) {
+                                                     ForceLog flog, FrontAcc acc) {
   __shared__ double lds[LDS_RED];
   const int w = blockIdx.x;
   if (w < G) {
     if (w < ob.cnt[0]) obst_moments_wg(w, g, ss, ob, lds);
   } else if (w == G) {
     const double corr = flux_corr(fluxpart, edge_count(gx, gy), g, lds);
-    if (threadIdx.x == 0) st->flux_corr = corr;
+    if (threadIdx.x == 0) {
+      st->flux_corr = corr;
+      if (acc.J) acc.dts[acc.k] = st->dt;
+    }
   } else {
     forces_fin_wg(g, ss, pv, st, 0, snap, flog, 1);
+    // (thread 0 has just written shape 0's drag)
+    if (acc.J && threadIdx.x == 0) *acc.J += acc.w * ss[0].drag;
   }
 }
 
-int enqueue_step_front(cup2d_ctx* c, int compute_dt) {
+int enqueue_step_front(cup2d_ctx* c, int compute_dt, const FrontAcc& acc) {
   const int G = grid_cap(c);
   const bool forces = c->forces_pending;
   const int end_prev = c->end_pending ? 1 : 0;
@@ -2174,7 +2179,7 @@ int enqueue_step_front(cup2d_ctx* c, int compute_dt) {
   c->flux_deferred = true;
   const ForceLog flog{c->flog, c->flog_cnt, c->flog_cap};
   hipLaunchKernelGGL(k_step_moments, dim3(forces ? G + 2 : G + 1), dim3(NT), 0, c->stream, c->g,
-                     c->ss, c->st, c->ob, c->ob_prev, G, c->fluxpart, gx, gy, c->fsnap, flog);
+                     c->ss, c->st, c->ob, c->ob_prev, G, c->fluxpart, gx, gy, c->fsnap, flog, acc);
   c->commit_pending = true;
   c->front_fused = true;
   return launch_check(c, "step front");
