@@ -43,6 +43,44 @@ namespace {
 constexpr int ANT = 256;
 constexpr double EPSD = 2.220446049250313e-16;
 constexpr int BC_KILL = 100;  // Definitions.h:38
+constexpr int ADJ_CPT = BS * BS / ANT;  // cells per thread of a block
+static_assert(BS * BS % ANT == 0, "whole cells per thread");
+
+// Sums of NV values per thread (a power of two <= 32) over the workgroup: each
+// butterfly step halves the values a lane still carries, 32 exchanges per
+// wave for 32 values where a butterfly per value takes 192 (k_adj_penalize 18.7
+// -> 10.0 us).  The total of value k is returned to
+// thread k < NV; lds holds ANT/64 * NV.
+template <int NV, int O = 32>
+__device__ inline void scatter_step(double* a) {
+  const bool hi = threadIdx.x & O;
+  constexpr int H = NV / 2;
+  if constexpr (H >= 1) {
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const double keep = hi ? a[i + H] : a[i], send = hi ? a[i] : a[i + H];
+      a[i] = keep + __shfl_xor(send, O, 64);
+    }
+    if constexpr (O > 1) scatter_step<H, O / 2>(a);
+  } else {
+    a[0] += __shfl_xor(a[0], O, 64);
+    if constexpr (O > 1) scatter_step<1, O / 2>(a);
+  }
+}
+template <int NV>
+__device__ inline double block_sum_scatter(double* a, double* lds) {
+  static_assert(NV == 32, "five halvings, one plain step");
+  scatter_step<NV>(a);
+  const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
+  __syncthreads();
+  // the lane's bits 5..1 chose its value from the top bit down
+  if ((lane & 1) == 0) lds[wv * NV + (lane >> 1)] = a[0];
+  __syncthreads();
+  double s = 0;
+  if (threadIdx.x < NV)
+    for (int w = 0; w < ANT / 64; ++w) s += lds[w * NV + threadIdx.x];
+  return s;
+}
 
 __device__ inline size_t cidx(const Grid& g, int x, int y) {
   x = x < 0 ? 0 : (x >= g.NX ? g.NX - 1 : x);
@@ -96,16 +134,30 @@ __global__ __launch_bounds__(ANT) void k_adj_forces(Grid g, Obstacles ob, int sh
   const int b = ob.slot_block[s], bx = b % g.bpdx, by = b / g.bpdx;
   const ASlot o = aslot(ob, s);
   const double NUoH = g.nu / g.h;
-  for (int i = threadIdx.x; i < BS * BS; i += ANT) {
-    if (!(o.sd[i] > 0)) continue;
+  // every load of the thread's cells first (one memory round trip), surface
+  // points or not
+  double sd[ADJ_CPT], sx[ADJ_CPT], sy[ADJ_CPT], d11[ADJ_CPT], d22[ADJ_CPT], d12[ADJ_CPT],
+      pc[ADJ_CPT];
+#pragma unroll
+  for (int j = 0; j < ADJ_CPT; ++j) {
+    const int i = threadIdx.x + j * ANT, gx = bx * BS + i % BS, gy = by * BS + i / BS;
+    sd[j] = o.sd[i];
+    sx[j] = o.sx[i];
+    sy[j] = o.sy[i];
+    d11[j] = u[cidx(g, gx + 1, gy)] - u[cidx(g, gx - 1, gy)];
+    d22[j] = v[cidx(g, gx, gy + 1)] - v[cidx(g, gx, gy - 1)];
+    d12[j] = u[cidx(g, gx, gy + 1)] - u[cidx(g, gx, gy - 1)] + v[cidx(g, gx + 1, gy)] -
+             v[cidx(g, gx - 1, gy)];
+    pc[j] = p[(size_t)gy * g.NX + gx];
+  }
+#pragma unroll
+  for (int j = 0; j < ADJ_CPT; ++j) {
+    const int i = threadIdx.x + j * ANT;
+    if (!(sd[j] > 0)) continue;
     const int gx = bx * BS + i % BS, gy = by * BS + i / BS;
-    const double D11 = NUoH * (u[cidx(g, gx + 1, gy)] - u[cidx(g, gx - 1, gy)]);
-    const double D22 = NUoH * (v[cidx(g, gx, gy + 1)] - v[cidx(g, gx, gy - 1)]);
-    const double D12 = NUoH / 2 *
-                       (u[cidx(g, gx, gy + 1)] - u[cidx(g, gx, gy - 1)] +
-                        v[cidx(g, gx + 1, gy)] - v[cidx(g, gx - 1, gy)]);
-    const double nX = o.sx[i], nY = o.sy[i];
-    const double Pc = p[(size_t)gy * g.NX + gx];
+    const double D11 = NUoH * d11[j], D22 = NUoH * d22[j], D12 = NUoH / 2 * d12[j];
+    const double nX = sx[j], nY = sy[j];
+    const double Pc = pc[j];
     const double fXT = D11 * nX + D12 * nY - Pc * nX;
     const double fYT = D12 * nX + D22 * nY - Pc * nY;
     const double fp = fXT * vu0 + fYT * vu1;
@@ -128,14 +180,13 @@ __global__ __launch_bounds__(ANT) void k_adj_forces(Grid g, Obstacles ob, int sh
 
 // explicit penalization u <- (1 - chi) u + chi (U_s + udef): the adjoint of
 // the penalized cells scales by 1 - chi; the surface-velocity coefficients
-// receive chi (ub, vb) . d(udef)/d(coef), per workgroup into part[wg][4M].
+// receive chi (ub, vb) . d(udef)/d(coef), per workgroup added to part[wg][4M]
+// over the steps (k_adj_theta sums them once at the end).
 // One workgroup per distinct obstacle block.
 // Modes per accumulation pass of k_adj_penalize: its 4 x ADJ_MCH sums stay
 // in registers (4 x SURF_MAX_MODES indexed by a run-time mode would live in
 // scratch memory).
 constexpr int ADJ_MCH = 8;
-constexpr int ADJ_CPT = BS * BS / ANT;  // cells per thread of a block
-static_assert(BS * BS % ANT == 0, "whole cells per thread");
 
 __global__ __launch_bounds__(ANT) void k_adj_penalize(Grid g, Obstacles ob, int shape,
                                                       const double* __restrict__ chi,
@@ -152,10 +203,7 @@ __global__ __launch_bounds__(ANT) void k_adj_penalize(Grid g, Obstacles ob, int 
     for (int q = 0; q < cnt; ++q)
       if (ob.slot_shape[ob.ub_slots[s0 + q]] == shape) s = ob.ub_slots[s0 + q];
   }
-  if (s < 0) {  // no cell of the shape: zero partials
-    for (int k = threadIdx.x; k < 4 * M; k += ANT) out[k] = 0;
-    return;
-  }
+  if (s < 0) return;  // no cell of the shape
   // per cell: the weights of the normal and tangential parts and the unit
   // direction z from the centre of mass, whose powers z^(m+1) carry mode m;
   // the adjoint velocity is scaled by (1 - chi) on the way
@@ -203,26 +251,22 @@ __global__ __launch_bounds__(ANT) void k_adj_penalize(Grid g, Obstacles ob, int 
         acc[3 * ADJ_MCH + mm] += gt[j] * wi[j];
       }
     }
-    block_sum_multi<ANT, 4 * ADJ_MCH>(acc, lds);
-    if (threadIdx.x == 0) {
-#pragma unroll
-      for (int mm = 0; mm < ADJ_MCH; ++mm) {
-        if (m0 + mm >= M) continue;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) out[q * M + m0 + mm] = acc[q * ADJ_MCH + mm];
-      }
+    const double sum = block_sum_scatter<4 * ADJ_MCH>(acc, lds);
+    if (threadIdx.x < 4 * ADJ_MCH) {
+      const int q = threadIdx.x / ADJ_MCH, m = m0 + (int)threadIdx.x % ADJ_MCH;
+      if (m < M) out[q * M + m] += sum;
     }
   }
 }
 
-// the parameter gradient += sum over workgroups of the partials: one
-// workgroup per parameter, the sum in a fixed order (block_sum_array)
+// the parameter gradient: the sum over workgroups of the partials, one
+// workgroup per parameter, in a fixed order (block_sum_array)
 __global__ __launch_bounds__(ANT) void k_adj_theta(const double* __restrict__ part, int nwg,
                                                    int n4, double* __restrict__ theta) {
   __shared__ double lds[ANT / 64];
   const int k = blockIdx.x;
   const double s = block_sum_array<ANT>(part + k, nwg, n4, lds);
-  if (threadIdx.x == 0) theta[k] += s;
+  if (threadIdx.x == 0) theta[k] = s;
 }
 
 // projection z = wf + pFac grad p: pb += pFac (Gx^T ub + Gy^T vb)
@@ -240,18 +284,12 @@ __global__ __launch_bounds__(ANT) void k_adj_project(Grid g, double pFac,
 // cub2rhs fade, pass 1: per band block, the forward sums of f = r fa^2
 // (total, positive and negative parts) and the adjoint sums
 // sum rb max(f,0) and sum rb (-min(f,0)); r recomputed from wf.
-__global__ __launch_bounds__(ANT) void k_adj_fade1(Grid g, const int* __restrict__ blocks,
-                                                   int nblocks, double facDiv,
-                                                   const double* __restrict__ wu,
-                                                   const double* __restrict__ wv,
-                                                   const double* __restrict__ rb,
-                                                   double* __restrict__ part) {
-  __shared__ double lds[(ANT / 64) * 5];
-  const int j = blockIdx.x;
-  if (j >= nblocks) return;
+__device__ void adj_fade1_wg(int wg, const Grid& g, const int* __restrict__ blocks, int nblocks, double facDiv, const double* __restrict__ wu, const double* __restrict__ wv, const double* __restrict__ rb, double* __restrict__ part, double* lds) {
+  const int j = wg;
   const int b = blocks[j], bx = b % g.bpdx, by = b / g.bpdx;
   double a[5] = {0, 0, 0, 0, 0};
-  for (int i = threadIdx.x; i < BS * BS; i += ANT) {
+#pragma unroll
+  for (int it = 0, i = threadIdx.x; it < ADJ_CPT; ++it, i += ANT) {
     const int ix = i % BS, iy = i / BS, x = bx * BS + ix, y = by * BS + iy;
     const double fa = fade_arg(g, cell_pos(bx, ix, g.hb, g.h), cell_pos(by, iy, g.hb, g.h));
     const double f = rhs_raw(g, wu, wv, x, y, facDiv) * (fa * fa);
@@ -267,15 +305,8 @@ __global__ __launch_bounds__(ANT) void k_adj_fade1(Grid g, const int* __restrict
 
 // cub2rhs fade, pass 2: every workgroup sums the partials (same order), forms
 // corr = Sr / (Sr > 0 ? P : N) and applies the transposed fade to its block.
-__global__ __launch_bounds__(ANT) void k_adj_fade2(Grid g, const int* __restrict__ blocks,
-                                                   int nblocks, double facDiv,
-                                                   const double* __restrict__ wu,
-                                                   const double* __restrict__ wv,
-                                                   const double* __restrict__ part,
-                                                   double* __restrict__ rb) {
-  __shared__ double lds[(ANT / 64) * 5];
-  const int j = blockIdx.x;
-  if (j >= nblocks) return;
+__device__ void adj_fade2_wg(int wg, const Grid& g, const int* __restrict__ blocks, int nblocks, double facDiv, const double* __restrict__ wu, const double* __restrict__ wv, const double* __restrict__ part, double* __restrict__ rb, double* lds) {
+  const int j = wg;
   double tot[5];
   block_sum_table<ANT, 5>(part, nblocks, 5, tot, lds);  // the same order in every workgroup
   const double Sr = tot[0], P = dmax(tot[1], EPSD), Nn = dmax(tot[2], EPSD);
@@ -284,7 +315,8 @@ __global__ __launch_bounds__(ANT) void k_adj_fade2(Grid g, const int* __restrict
   // a denominator held at epsilon (fade_corr_factor's clamp) has no derivative
   const double kP = tot[1] < EPSD ? 0.0 : 1.0, kN = tot[2] < EPSD ? 0.0 : 1.0;
   const int b = blocks[j], bx = b % g.bpdx, by = b / g.bpdx;
-  for (int i = threadIdx.x; i < BS * BS; i += ANT) {
+#pragma unroll
+  for (int it = 0, i = threadIdx.x; it < ADJ_CPT; ++it, i += ANT) {
     const int ix = i % BS, iy = i / BS, x = bx * BS + ix, y = by * BS + iy;
     const double fa = fade_arg(g, cell_pos(bx, ix, g.hb, g.h), cell_pos(by, iy, g.hb, g.h));
     const double fa2 = fa * fa;
@@ -300,56 +332,53 @@ __global__ __launch_bounds__(ANT) void k_adj_fade2(Grid g, const int* __restrict
 // the shape (S = sum -chi r, positive and negative perimeter parts of
 // T = r (1 - chi)) and the adjoint sums for both signs of corr:
 // sum rb (-T) [perimeter, T > 0] and sum rb T [perimeter, T < 0].
-__global__ __launch_bounds__(ANT) void k_adj_obst1(Grid g, Obstacles ob, int shape,
-                                                   double facDiv,
-                                                   const double* __restrict__ chi,
-                                                   const double* __restrict__ wu,
-                                                   const double* __restrict__ wv,
-                                                   const double* __restrict__ rb,
-                                                   double* __restrict__ part) {
-  __shared__ double lds[(ANT / 64) * 5];
+__device__ void adj_obst1_wg(int wg, const Grid& g, const Obstacles& ob, int shape, double facDiv, const double* __restrict__ chi, const double* __restrict__ wu, const double* __restrict__ wv, const double* __restrict__ rb, double* __restrict__ part, double* lds) {
   double a[5] = {0, 0, 0, 0, 0};
   const int nub = ob.cnt[1];
-  if ((int)blockIdx.x < nub) {
-    const int b = ob.ub_block[blockIdx.x], bx = b % g.bpdx, by = b / g.bpdx;
-    const int s0 = ob.ub_start[blockIdx.x], cnt = ob.ub_count[blockIdx.x];
+  if (wg < nub) {
+    const int b = ob.ub_block[wg], bx = b % g.bpdx, by = b / g.bpdx;
+    const int s0 = ob.ub_start[wg], cnt = ob.ub_count[wg];
     for (int q = 0; q < cnt; ++q) {
       const int s = ob.ub_slots[s0 + q];
       if (ob.slot_shape[s] != shape) continue;
       const ASlot o = aslot(ob, s);
-      for (int i = threadIdx.x; i < BS * BS; i += ANT) {
-        const int x = bx * BS + i % BS, y = by * BS + i / BS;
+      // every load of the thread's cells first (one memory round trip)
+      double cX[ADJ_CPT], cO[ADJ_CPT], cg[ADJ_CPT], cr[ADJ_CPT], cb[ADJ_CPT];
+#pragma unroll
+      for (int it = 0; it < ADJ_CPT; ++it) {
+        const int i = threadIdx.x + it * ANT, x = bx * BS + i % BS, y = by * BS + i / BS;
         const size_t d = (size_t)y * g.NX + x;
-        if (chi[d] > o.chi[i]) continue;
+        cX[it] = chi[d];
+        cO[it] = o.chi[i];
         const double gx = chi[cidx(g, x + 1, y)] - chi[cidx(g, x - 1, y)];
         const double gy = chi[cidx(g, x, y + 1)] - chi[cidx(g, x, y - 1)];
-        const bool perim = gx * gx + gy * gy > 0;
-        const double rr = rhs_raw(g, wu, wv, x, y, facDiv);
-        const double src = -o.chi[i] * rr;
+        cg[it] = gx * gx + gy * gy;
+        cr[it] = rhs_raw(g, wu, wv, x, y, facDiv);
+        cb[it] = rb[d];
+      }
+#pragma unroll
+      for (int it = 0; it < ADJ_CPT; ++it) {
+        if (cX[it] > cO[it]) continue;
+        const bool perim = cg[it] > 0;
+        const double rr = cr[it];
+        const double src = -cO[it] * rr;
         const double T = rr + src;
         a[0] += src;
-        if (perim && T > 0) { a[1] += T; a[3] -= rb[d] * T; }
-        if (perim && T < 0) { a[2] -= T; a[4] += rb[d] * T; }
+        if (perim && T > 0) { a[1] += T; a[3] -= cb[it] * T; }
+        if (perim && T < 0) { a[2] -= T; a[4] += cb[it] * T; }
       }
     }
   }
   block_sum_multi<ANT, 5>(a, lds);
   if (threadIdx.x == 0)
-    for (int k = 0; k < 5; ++k) part[5 * blockIdx.x + k] = a[k];
+    for (int k = 0; k < 5; ++k) part[5 * wg + k] = a[k];
 }
 
 // obstacle RHS correction, pass 2: totals (in order), corr = S / D, and the
 // transposed correction and source term on the block's cells.
-__global__ __launch_bounds__(ANT) void k_adj_obst2(Grid g, Obstacles ob, int shape,
-                                                   double facDiv,
-                                                   const double* __restrict__ chi,
-                                                   const double* __restrict__ wu,
-                                                   const double* __restrict__ wv,
-                                                   const double* __restrict__ part,
-                                                   double* __restrict__ rb) {
-  __shared__ double lds[(ANT / 64) * 5];
+__device__ void adj_obst2_wg(int wg, const Grid& g, const Obstacles& ob, int shape, double facDiv, const double* __restrict__ chi, const double* __restrict__ wu, const double* __restrict__ wv, const double* __restrict__ part, double* __restrict__ rb, double* lds) {
   const int nub = ob.cnt[1];
-  if ((int)blockIdx.x >= nub) return;
+  if (wg >= nub) return;
   double tot[5];
   block_sum_table<ANT, 5>(part, nub, 5, tot, lds);  // the same order in every workgroup
   const double S = tot[0];
@@ -358,21 +387,33 @@ __global__ __launch_bounds__(ANT) void k_adj_obst2(Grid g, Obstacles ob, int sha
   const double kD = Draw < EPSD ? 0.0 : 1.0;  // a clamped denominator has no derivative
   const double corr = S / D;
   const double Cbar = corr > 0 ? tot[3] : (corr < 0 ? tot[4] : 0.0);
-  const int b = ob.ub_block[blockIdx.x], bx = b % g.bpdx, by = b / g.bpdx;
-  const int s0 = ob.ub_start[blockIdx.x], cnt = ob.ub_count[blockIdx.x];
+  const int b = ob.ub_block[wg], bx = b % g.bpdx, by = b / g.bpdx;
+  const int s0 = ob.ub_start[wg], cnt = ob.ub_count[wg];
   for (int q = 0; q < cnt; ++q) {
     const int s = ob.ub_slots[s0 + q];
     if (ob.slot_shape[s] != shape) continue;
     const ASlot o = aslot(ob, s);
-    for (int i = threadIdx.x; i < BS * BS; i += ANT) {
-      const int x = bx * BS + i % BS, y = by * BS + i / BS;
+    // every load of the thread's cells first (one memory round trip)
+    double cX[ADJ_CPT], cO[ADJ_CPT], cg[ADJ_CPT], cr[ADJ_CPT], cb[ADJ_CPT];
+#pragma unroll
+    for (int it = 0; it < ADJ_CPT; ++it) {
+      const int i = threadIdx.x + it * ANT, x = bx * BS + i % BS, y = by * BS + i / BS;
       const size_t d = (size_t)y * g.NX + x;
-      if (chi[d] > o.chi[i]) continue;
+      cX[it] = chi[d];
+      cO[it] = o.chi[i];
       const double gx = chi[cidx(g, x + 1, y)] - chi[cidx(g, x - 1, y)];
       const double gy = chi[cidx(g, x, y + 1)] - chi[cidx(g, x, y - 1)];
-      const bool perim = gx * gx + gy * gy > 0;
-      const double X = o.chi[i];
-      const double rr = rhs_raw(g, wu, wv, x, y, facDiv);
+      cg[it] = gx * gx + gy * gy;
+      cr[it] = rhs_raw(g, wu, wv, x, y, facDiv);
+      cb[it] = rb[d];
+    }
+#pragma unroll
+    for (int it = 0; it < ADJ_CPT; ++it) {
+      const int i = threadIdx.x + it * ANT;
+      const size_t d = (size_t)(by * BS + i / BS) * g.NX + bx * BS + i % BS;
+      if (cX[it] > cO[it]) continue;
+      const bool perim = cg[it] > 0;
+      const double X = cO[it], rr = cr[it];
       const double T = rr + (-X * rr);
       double sigma = 0;
       if (perim && T > 0 && corr > 0) sigma = 1;
@@ -380,10 +421,40 @@ __global__ __launch_bounds__(ANT) void k_adj_obst2(Grid g, Obstacles ob, int sha
       double dcorr = 0;  // d corr / d T through the denominator
       if (S > 0 && perim && T > 0) dcorr = -kD * corr / D;
       if (!(S > 0) && perim && T < 0) dcorr = kD * corr / D;
-      const double Tbar = rb[d] * (1 - sigma * corr) + Cbar * dcorr;
+      const double Tbar = cb[it] * (1 - sigma * corr) + Cbar * dcorr;
       rb[d] = Tbar * (1 - X) + (Cbar / D) * (-X);
     }
   }
+}
+
+// The two passes of the fade's and of the obstacle correction's adjoint side
+// by side: nb band blocks, then the obstacle blocks (the disk's blocks lie
+// outside the band, so the two touch different cells).
+__global__ __launch_bounds__(ANT) void k_adj_rhs1(Grid g, const int* __restrict__ blocks, int nb,
+                                                  Obstacles ob, int shape, double facDiv,
+                                                  const double* __restrict__ chi,
+                                                  const double* __restrict__ wu,
+                                                  const double* __restrict__ wv,
+                                                  const double* __restrict__ rb,
+                                                  double* __restrict__ fpart,
+                                                  double* __restrict__ opart) {
+  __shared__ double lds[(ANT / 64) * 5];
+  const int w = blockIdx.x;
+  if (w < nb) adj_fade1_wg(w, g, blocks, nb, facDiv, wu, wv, rb, fpart, lds);
+  else adj_obst1_wg(w - nb, g, ob, shape, facDiv, chi, wu, wv, rb, opart, lds);
+}
+__global__ __launch_bounds__(ANT) void k_adj_rhs2(Grid g, const int* __restrict__ blocks, int nb,
+                                                  Obstacles ob, int shape, double facDiv,
+                                                  const double* __restrict__ chi,
+                                                  const double* __restrict__ wu,
+                                                  const double* __restrict__ wv,
+                                                  const double* __restrict__ fpart,
+                                                  const double* __restrict__ opart,
+                                                  double* __restrict__ rb) {
+  __shared__ double lds[(ANT / 64) * 5];
+  const int w = blockIdx.x;
+  if (w < nb) adj_fade2_wg(w, g, blocks, nb, facDiv, wu, wv, fpart, rb, lds);
+  else adj_obst2_wg(w - nb, g, ob, shape, facDiv, chi, wu, wv, opart, rb, lds);
 }
 
 // divergence r = facDiv div(wf): wb = ub + facDiv Gx^T rb, vb' = vb + facDiv Gy^T rb
@@ -447,7 +518,8 @@ __global__ __launch_bounds__(ANT) void k_adj_advdiff(Grid g, double dt, double U
                                                      const double* __restrict__ wbv,
                                                      const double* __restrict__ fluxsum,
                                                      double* __restrict__ ub,
-                                                     double* __restrict__ vb) {
+                                                     double* __restrict__ vb,
+                                                     double* __restrict__ pb) {
   const int NX = g.NX, NY = g.NY;
   const double h = g.h;
   const double dfac = (g.nu / h) * (dt / h), afac = -0.5 * dt / h;
@@ -499,6 +571,7 @@ __global__ __launch_bounds__(ANT) void k_adj_advdiff(Grid g, double dt, double U
     }
     ub[j] = gu;
     vb[j] = gv;
+    pb[j] = 0;  // for the next step's forces
   }
 }
 
@@ -574,43 +647,42 @@ int enqueue_adjoint_acc_drag(cup2d_ctx* c, int shape, double w, double* J) {
   return launch_check(c, "adjoint drag");
 }
 
+// theta = the sums of the steps' partials (theta_part) over the workgroups
+int enqueue_adjoint_theta(cup2d_ctx* c, const double* theta_part, double* theta) {
+  if (c->surf_modes == 0) return CUP2D_OK;
+  hipLaunchKernelGGL(k_adj_theta, dim3(4 * c->surf_modes), dim3(ANT), 0, c->stream, theta_part,
+                     c->ob.cap > 0 ? c->ob.cap : 1, 4 * c->surf_modes, theta);
+  return launch_check(c, "adjoint gradient");
+}
+
 // One step of the adjoint, backwards: on entry (a.ub, a.vb) is the adjoint
-// of the step's output velocity; on exit that of its input velocity, and the
-// surface-velocity gradient a.theta has this step's share added.
+// of the step's output velocity and a.pb is zero; on exit that of its input
+// velocity, a.pb zero again, and a.theta_part has this step's share added.
 int enqueue_adjoint_step(cup2d_ctx* c, const AdjStep& a) {
   const Grid& g = c->g;
-  const size_t n = (size_t)g.NX * g.NY;
   const int G = c->ob.cap > 0 ? c->ob.cap : 1;
   const double facDiv = 0.5 * g.h / a.dt, pFac = -0.5 * a.dt / g.h;
   hipStream_t s = c->stream;
-  hipLaunchKernelGGL(k_adj_fill, dim3(1024), dim3(ANT), 0, s, a.pb, n, 0.0);
   hipLaunchKernelGGL(k_adj_forces, dim3(G), dim3(ANT), 0, s, g, c->ob, a.shape, a.u1, a.v1, a.p1,
                      a.vu0, a.vu1, a.wJ, a.ub, a.vb, a.pb);
   hipLaunchKernelGGL(k_adj_penalize, dim3(G), dim3(ANT), 0, s, g, c->ob, a.shape, c->chi, c->ss,
                      surf_of(c), a.ub, a.vb, a.theta_part);
-  if (c->surf_modes > 0)
-    hipLaunchKernelGGL(k_adj_theta, dim3(4 * c->surf_modes), dim3(ANT), 0, s, a.theta_part, G,
-                       4 * c->surf_modes, a.theta);
   hipLaunchKernelGGL(k_adj_project, dim3(2048), dim3(ANT), 0, s, g, pFac, a.ub, a.vb, a.pb);
   int rc = launch_check(c, "adjoint: forces, penalization, projection");
   if (rc) return rc;
   rc = enqueue_poisson_fft(c, a.pb, a.rb, 0);  // the solve is symmetric
   if (rc) return rc;
-  if (c->band_nblocks > 0) {
-    hipLaunchKernelGGL(k_adj_fade1, dim3(c->band_nblocks), dim3(ANT), 0, s, g, c->band_blocks,
-                       c->band_nblocks, facDiv, a.wu, a.wv, a.rb, a.part);
-    hipLaunchKernelGGL(k_adj_fade2, dim3(c->band_nblocks), dim3(ANT), 0, s, g, c->band_blocks,
-                       c->band_nblocks, facDiv, a.wu, a.wv, a.part, a.rb);
-  }
-  hipLaunchKernelGGL(k_adj_obst1, dim3(G), dim3(ANT), 0, s, g, c->ob, a.shape, facDiv, c->chi,
-                     a.wu, a.wv, a.rb, a.part);
-  hipLaunchKernelGGL(k_adj_obst2, dim3(G), dim3(ANT), 0, s, g, c->ob, a.shape, facDiv, c->chi,
-                     a.wu, a.wv, a.part, a.rb);
+  const int nb = c->band_nblocks;
+  double* opart = a.part + 5 * nb;
+  hipLaunchKernelGGL(k_adj_rhs1, dim3(nb + G), dim3(ANT), 0, s, g, c->band_blocks, nb, c->ob,
+                     a.shape, facDiv, c->chi, a.wu, a.wv, a.rb, a.part, opart);
+  hipLaunchKernelGGL(k_adj_rhs2, dim3(nb + G), dim3(ANT), 0, s, g, c->band_blocks, nb, c->ob,
+                     a.shape, facDiv, c->chi, a.wu, a.wv, a.part, opart, a.rb);
   hipLaunchKernelGGL(k_adj_div, dim3(2048), dim3(ANT), 0, s, g, facDiv, a.ub, a.vb, a.rb, a.wbu,
                      a.wbv);
   hipLaunchKernelGGL(k_adj_flux_sum, dim3(1), dim3(ANT), 0, s, g, a.wbu, a.wbv, a.fluxsum);
   hipLaunchKernelGGL(k_adj_advdiff, dim3(2048), dim3(ANT), 0, s, g, a.dt, a.uinf0, a.uinf1, a.u0,
-                     a.v0, a.wbu, a.wbv, a.fluxsum, a.ub, a.vb);
+                     a.v0, a.wbu, a.wbv, a.fluxsum, a.ub, a.vb, a.pb);
   return launch_check(c, "adjoint: fade, obstacle RHS, divergence, advDiff");
 }
 

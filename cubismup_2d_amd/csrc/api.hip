@@ -408,7 +408,7 @@ struct AdjointState {
   std::vector<StepState> ck_st;
   std::vector<std::vector<cup2d_shape_state>> ck_ss;
   double* seg = nullptr;               // (every + 1) (u, v), every (wu, wv), every p
-  double* work = nullptr;              // ub vb pb rb wbu wbv ub2 vb2
+  double* work = nullptr;              // ub vb pb rb wbu wbv
   double* part = nullptr;              // 5 per block
   double* theta_part = nullptr;
   double* theta = nullptr;             // [4M]
@@ -1036,9 +1036,9 @@ int cup2d_adjoint_forward(cup2d_ctx* c, int nsteps, int every, const double* dts
     a->ck.assign(nseg + 1, nullptr);
     for (double*& p : a->ck) CUP2D_HIP_CHECK(c, hipMalloc(&p, sizeof(double) * 2 * n));
     CUP2D_HIP_CHECK(c, hipMalloc(&a->seg, sizeof(double) * n * (2 * (every + 1) + 3 * every)));
-    CUP2D_HIP_CHECK(c, hipMalloc(&a->work, sizeof(double) * n * 8));
+    CUP2D_HIP_CHECK(c, hipMalloc(&a->work, sizeof(double) * n * 6));
     const int G = c->ob.cap > 0 ? c->ob.cap : 1;
-    const int nblk = std::max(G, c->band_nblocks);
+    const int nblk = G + c->band_nblocks;
     CUP2D_HIP_CHECK(c, hipMalloc(&a->part, sizeof(double) * 5 * (size_t)(nblk + 1)));
     CUP2D_HIP_CHECK(c, hipMalloc(&a->theta_part, sizeof(double) * 4 * SURF_MAX_MODES * (size_t)G));
     CUP2D_HIP_CHECK(c, hipMalloc(&a->theta, sizeof(double) * 4 * SURF_MAX_MODES));
@@ -1110,14 +1110,12 @@ int cup2d_adjoint_backward(cup2d_ctx* c, double* grad) {
   double* rb = pb + n;
   double* wbu = rb + n;
   double* wbv = wbu + n;
-  double* ub2 = wbv + n;
-  double* vb2 = ub2 + n;
   double* segU = a->seg;                       // (K + 1) x (u, v)
   double* segW = segU + 2 * n * (K + 1);       // K x (wu, wv)
   double* segP = segW + 2 * n * K;             // K x p
   const int M = c->surf_modes;
-  RC(enqueue_adjoint_fill(c, ub, 2 * n, 0.0));
-  RC(enqueue_adjoint_fill(c, a->theta, 4 * M, 0.0));
+  RC(enqueue_adjoint_fill(c, ub, 3 * n, 0.0));  // ub, vb, pb
+  RC(enqueue_adjoint_fill(c, a->theta_part, (size_t)4 * M * (c->ob.cap > 0 ? c->ob.cap : 1), 0.0));
   const int nseg = (N + K - 1) / K;
   for (int sgi = nseg - 1; sgi >= 0; --sgi) {
     const int k0 = sgi * K, len = std::min(K, N - k0);
@@ -1149,12 +1147,11 @@ int cup2d_adjoint_backward(cup2d_ctx* c, double* grad) {
       s.ub = ub; s.vb = vb; s.pb = pb; s.rb = rb; s.wbu = wbu; s.wbv = wbv;
       s.part = a->part;
       s.theta_part = a->theta_part;
-      s.theta = a->theta;
       s.fluxsum = a->scal + 1;
-      (void)ub2; (void)vb2;
       RC(enqueue_adjoint_step(c, s));
     }
   }
+  RC(enqueue_adjoint_theta(c, a->theta_part, a->theta));
   CUP2D_HIP_CHECK(c, hipMemcpyAsync(grad, a->theta, sizeof(double) * 4 * M, hipMemcpyDeviceToHost, c->stream));
   RC(adjoint_restore(c, nseg));  // back to the state after the forward run
   return sync_and_check(c);

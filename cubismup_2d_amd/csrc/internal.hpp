@@ -432,12 +432,12 @@ struct AdjStep {
   const double* p1;        // its pressure
   double *ub, *vb;         // in: adjoint of the output velocity; out: of the input
   double *pb, *rb, *wbu, *wbv;  // work planes
-  double* part;            // work partials (5 per block)
-  double* theta_part;      // [obstacle slots][4M]
-  double* theta;           // [4M] gradient, accumulated
+  double* part;            // work partials (5 per band and obstacle block)
+  double* theta_part;      // [obstacle slots][4M], accumulated over the steps
   double* fluxsum;         // one double
 };
 int enqueue_adjoint_step(cup2d_ctx* c, const AdjStep& a);
+int enqueue_adjoint_theta(cup2d_ctx* c, const double* theta_part, double* theta);
 int enqueue_adjoint_fill(cup2d_ctx* c, double* a, size_t n, double val);
 int enqueue_adjoint_acc_drag(cup2d_ctx* c, int shape, double w, double* J);
 // copies of the velocity, with the deferred flux correction applied (w), or of
