@@ -509,6 +509,47 @@ union PlaceLds {
 };
 }  // namespace
 
+namespace {
+// The threads' indices i with hit set, in thread order, to list[]; returns
+// their number (every thread; ends with a barrier).
+__device__ inline int block_compact(bool hit, int i, int* list, int* tmp) {
+  const unsigned long long m = __ballot(hit);
+  const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
+  if (lane == 0) tmp[wv] = __popcll(m);
+  __syncthreads();
+  int base = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) {
+    const int x = tmp[w];
+    base += w < wv ? x : 0;
+    total += x;
+  }
+  if (hit) list[base + __popcll(m & ((1ull << lane) - 1))] = i;
+  __syncthreads();
+  return total;
+}
+// out[t] = the inclusive sum of v over threads 0 .. t (ends with a barrier)
+__device__ inline void block_inscan(int v, int* out, int* tmp) {
+  const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int o = __shfl_up(v, off, 64);
+    v += lane >= off ? o : 0;
+  }
+  if (lane == 63) tmp[wv] = v;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) v += w < wv ? tmp[w] : 0;
+  out[threadIdx.x] = v;
+  __syncthreads();
+}
+}  // namespace
+
+// One chunk of surface points (the usual case: up to SEG_PER_CHUNK segments
+// meet a block) keeps every pair's distance in registers between the two
+// passes and takes the winners' points from LDS; scans and compactions go by
+// shuffles and ballots instead of log-step LDS scans (16 barriers each):
+// 26 -> TODO us alone at 4096 x 2048.
 __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __restrict__ sp,
                                                    const cup2d_shape_state* __restrict__ ss,
                                                    const FishDev* __restrict__ fd,
@@ -519,6 +560,7 @@ __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __
   __shared__ int s_win[BS * BS];
   __shared__ unsigned long long s_qw[BS * BS], s_qu[BS * BS], s_qv[BS * BS];
   __shared__ int s_touch[BS * BS];
+  __shared__ int s_wsum[NT / 64];
   __shared__ PlaceLds U;
   const int s = blockIdx.x;
   if (s >= ob.cnt[0]) return;
@@ -536,28 +578,15 @@ __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __
     s_best[i] = ONE;  // |dist| starts at 1 (dist = -1)
     s_win[i] = 0x7fffffff;
   }
-  // segments meeting this block, in segment order (Fish.cpp:158-173)
+  // segments meeting this block, in segment order (Fish.cpp:158-173): a
+  // segment per thread, compacted by wave ballots
+  static_assert(FISH_MAX_SEG <= NT, "a segment per thread");
   int nsl;
   {
     double start[2], end[2];
     block_corners(g, bx, by, start, end);
-    int cnt = 0;
-    const int per = (F.Nseg + NT - 1) / NT;  // consecutive segments per thread
-    const int i0 = t * per, i1 = i0 + per < F.Nseg ? i0 + per : F.Nseg;
-    for (int i = i0; i < i1; ++i) cnt += seg_intersects(F.seg + (size_t)i * FISH_SEGD, start, end);
-    s_tmp[t] = cnt;
-    __syncthreads();
-    for (int off = 1; off < NT; off <<= 1) {
-      const int v = t >= off ? s_tmp[t - off] : 0;
-      __syncthreads();
-      s_tmp[t] += v;
-      __syncthreads();
-    }
-    int pos = t == 0 ? 0 : s_tmp[t - 1];
-    nsl = s_tmp[NT - 1];
-    for (int i = i0; i < i1; ++i)
-      if (seg_intersects(F.seg + (size_t)i * FISH_SEGD, start, end)) sl[pos++] = i;
-    __syncthreads();
+    const bool hit = t < F.Nseg && seg_intersects(F.seg + (size_t)t * FISH_SEGD, start, end);
+    nsl = block_compact(hit, t, sl, s_tmp);
   }
   const cup2d_shape_state& S = ss[k];
   Frame Fr;
@@ -570,29 +599,61 @@ __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __
   }
   // ---- constructSurface
   const int nchunk = (nsl + SEG_PER_CHUNK - 1) / SEG_PER_CHUNK;
+  // the surface points of the chunk from segment j0 (np of them) to U.pts
+  auto load_points = [&](int j0, int np) {
+    if (t < np) {
+      const int j = j0 + t / PTS_PER_SEG, r = t % PTS_PER_SEG;
+      const int s0 = 8 * sl[j], s1 = 8 * sl[j] + 8;
+      const int first = s0 > 1 ? s0 : 1, last = s1 < Nm - 2 ? s1 : Nm - 2;
+      const int sidx = first + r / 2, signp = (r & 1) ? 1 : -1;
+      SurfPt P;
+      if (sidx <= last) {
+        surf_point(F, M, Fr, sidx, signp, org0, org1, invh, P);
+        P.valid = 1;
+      } else {
+        P.valid = 0;
+      }
+      U.pts[t] = P;
+    }
+    __syncthreads();
+  };
+  if (nchunk <= 1) {
+    const int np = nsl * PTS_PER_SEG;
+    load_points(0, np);
+    constexpr int PAIRS = SEG_PER_CHUNK * PTS_PER_SEG * 16;
+    constexpr int PER = (PAIRS + NT - 1) / NT;
+    constexpr unsigned long long NONE = ~0ull;
+    unsigned long long bits[PER];
+    int cell[PER];
+#pragma unroll
+    for (int it = 0; it < PER; ++it) {
+      const int idx = t + it * NT, p = idx >> 4, q = idx & 15;
+      bits[it] = NONE;
+      cell[it] = 0;
+      if (p >= np || !U.pts[p].valid) continue;
+      const int sx = U.pts[p].iap[0] - 1 + (q & 3), sy = U.pts[p].iap[1] - 1 + (q >> 2);
+      if (sx < 0 || sx >= BS || sy < 0 || sy >= BS) continue;
+      const double pc[2] = {cell_pos(bx, sx, g.hb, h), cell_pos(by, sy, g.hb, h)};
+      const double d1 = dmin(dmin(dist_sq(pc, U.pts[p].myP), dist_sq(pc, U.pts[p].pP)),
+                             dist_sq(pc, U.pts[p].pM));
+      bits[it] = (unsigned long long)__double_as_longlong(d1);
+      cell[it] = sy * BS + sx;
+      atomicMin(&s_best[cell[it]], bits[it]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < PER; ++it)  // (bits < ONE: d1 < 1)
+      if (bits[it] < ONE && bits[it] == s_best[cell[it]])
+        atomicMin(&s_win[cell[it]], (t + it * NT) >> 4);
+    __syncthreads();
+  } else
   for (int pass = 0; pass < 2; ++pass) {
     for (int ch = 0; ch < nchunk; ++ch) {
       const int j0 = ch * SEG_PER_CHUNK;
       const int nj = nsl - j0 < SEG_PER_CHUNK ? nsl - j0 : SEG_PER_CHUNK;
       const int np = nj * PTS_PER_SEG;
-      if (pass == 0 || nchunk > 1) {  // (one chunk: pass 1 reuses the points)
-        __syncthreads();
-        if (t < np) {
-          const int j = j0 + t / PTS_PER_SEG, r = t % PTS_PER_SEG;
-          const int s0 = 8 * sl[j], s1 = 8 * sl[j] + 8;
-          const int first = s0 > 1 ? s0 : 1, last = s1 < Nm - 2 ? s1 : Nm - 2;
-          const int sidx = first + r / 2, signp = (r & 1) ? 1 : -1;
-          SurfPt P;
-          if (sidx <= last) {
-            surf_point(F, M, Fr, sidx, signp, org0, org1, invh, P);
-            P.valid = 1;
-          } else {
-            P.valid = 0;
-          }
-          U.pts[t] = P;
-        }
-        __syncthreads();
-      }
+      __syncthreads();
+      load_points(j0, np);
       for (int idx = t; idx < np * 16; idx += NT) {
         const int p = idx >> 4, q = idx & 15;
         if (!U.pts[p].valid) continue;
@@ -625,7 +686,8 @@ __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __
     const int first = s0 > 1 ? s0 : 1;
     const int sidx = first + r / 2, signp = (r & 1) ? 1 : -1;
     SurfPt P;
-    surf_point(F, M, Fr, sidx, signp, org0, org1, invh, P);
+    if (nchunk <= 1) P = U.pts[win];
+    else surf_point(F, M, Fr, sidx, signp, org0, org1, invh, P);
     double p[2] = {cell_pos(bx, cx, g.hb, h), cell_pos(by, cy0 + c, g.hb, h)};
     const double dist0 = dist_sq(p, P.myP), distP = dist_sq(p, P.pP), distM = dist_sq(p, P.pM);
     Fr.from_comp(p);
@@ -698,14 +760,7 @@ __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __
         E[E_VNX] = M.vNorX[sidx]; E[E_VNY] = M.vNorY[sidx];
       }
     }
-    s_tmp[t] = npts;
-    __syncthreads();
-    for (int off = 1; off < NT; off <<= 1) {  // inclusive scan of the point counts
-      const int v = t >= off ? s_tmp[t - off] : 0;
-      __syncthreads();
-      s_tmp[t] += v;
-      __syncthreads();
-    }
+    block_inscan(npts, s_tmp, s_wsum);  // inclusive scan of the point counts
     const int P = s_tmp[NT - 1];
     for (int idx = t; idx < P; idx += NT) {
       int lo = 0, hi = ne - 1;  // first entry whose inclusive count exceeds idx
@@ -764,6 +819,41 @@ __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __
     ob.rho[base + i] = 1;
     ob.chi[base + i] = 0;
   }
+}
+
+// Does any segment of swimmer blockIdx.y meet a candidate block of the list
+// builder (AreaSegment::isIntersectingWithAABB, Fish.cpp:158-173)?  A wave per
+// candidate, its lanes taking the segments; the answers go to
+// touch[swimmer][block].  With several swimmers the list builder, one
+// workgroup, spent most of its time on these tests one swimmer after another
+// (8192 x 4096 with four: TODO us); with one, its own prefiltered tests take
+// less than another launch.
+__global__ __launch_bounds__(NT) void k_fish_touch(Grid g, const FishDev* __restrict__ fd,
+                                                   unsigned char* __restrict__ touch) {
+  const int f = blockIdx.y, lane = threadIdx.x % 64;
+  const FishDev& F = fd[f];
+  const int nseg = F.Nseg;
+  const double box[4] = {F.box[0], F.box[1], F.box[2], F.box[3]};
+  int r[4];  // bx0, by0, width, height
+  candidate_range(g, box, r);
+  unsigned char* out = touch + (size_t)f * g.bpdx * g.bpdy;
+  for (int c = blockIdx.x * (NT / 64) + threadIdx.x / 64; c < r[2] * r[3];
+       c += gridDim.x * (NT / 64)) {
+    const int bx = r[0] + c % r[2], by = r[1] + c / r[2];
+    double start[2], end[2];
+    block_corners(g, bx, by, start, end);
+    bool hit = false;
+    for (int i = lane; i < nseg; i += 64)
+      hit |= seg_intersects(F.seg + (size_t)i * FISH_SEGD, start, end);
+    const unsigned long long m = __ballot(hit);
+    if (lane == 0) out[bx + g.bpdx * by] = m != 0;
+  }
+}
+
+int enqueue_fish_touch(cup2d_ctx* c, hipStream_t s) {
+  hipLaunchKernelGGL(k_fish_touch, dim3(64, (int)c->hfish.size()), dim3(NT), 0, s, c->g, c->fishd,
+                     c->fish_touch);
+  return launch_check(c, "fish touch");
 }
 
 // ------------------------------------------------------------------- host
@@ -871,6 +961,8 @@ void fish_free_all(cup2d_ctx* c) {
   c->hfish.clear();
   if (c->fishd) (void)hipFree(c->fishd);
   c->fishd = nullptr;
+  if (c->fish_touch) (void)hipFree(c->fish_touch);
+  c->fish_touch = nullptr;
 }
 
 // The time-only part lives in buffer host_step & 1: computed here when it is

@@ -46,6 +46,29 @@ __device__ inline void block_corners(const Grid& g, int bx, int by, double start
   end[1] = cell_pos(by, BS - 1, g.hb, g.h);
 }
 
+// The candidate blocks of a bounding box x0 x1 y0 y1: first block and extent
+// in x and y (out = bx0, by0, width, height).  A box that is not finite (a body
+// moved by a non-finite velocity or dt; CUP2D_ERR_NONFINITE is raised by the
+// dt part) selects no block: the range is clamped in floating point before any
+// integer conversion.
+__device__ inline void candidate_range(const Grid& g, const double box[4], int out[4]) {
+  bool fin = true;
+  double bb[4];
+  for (int q = 0; q < 4; ++q) {
+    const double x = box[q] / g.hb;
+    fin = fin && x == x && fabs(x) < 1e9;
+    bb[q] = fin ? x : 0.0;
+  }
+  int bx0 = (int)floor(bb[0]) - 1, bx1 = (int)floor(bb[1]) + 1;
+  int by0 = (int)floor(bb[2]) - 1, by1 = (int)floor(bb[3]) + 1;
+  bx0 = bx0 < 0 ? 0 : bx0; by0 = by0 < 0 ? 0 : by0;
+  bx1 = bx1 >= g.bpdx ? g.bpdx - 1 : bx1; by1 = by1 >= g.bpdy ? g.bpdy - 1 : by1;
+  out[0] = bx0;
+  out[1] = by0;
+  out[2] = fin && bx1 >= bx0 ? bx1 - bx0 + 1 : 0;
+  out[3] = fin && by1 >= by0 ? by1 - by0 + 1 : 0;
+}
+
 // Fish::create steps 6-7 (Fish.cpp:158-185): does any segment of swimmer F
 // meet block (bx, by)?
 __device__ inline bool fish_touching(const Grid& g, const FishDev& F, int bx, int by) {

@@ -54,6 +54,34 @@ __device__ inline SlotView slot(const Obstacles& ob, int s) {
   return v;
 }
 
+// A workgroup's slot s, or its distinct block u with the block's first slot
+// (the only one unless shapes overlap): the list entries are loaded together
+// with the count they are tested against (the lists hold at least gridDim
+// entries, so the loads are in bounds), one memory round trip instead of two
+// or three in kernels of a few microseconds.
+struct SlotHead {
+  int n, k, b;
+  __device__ SlotHead(const Obstacles& ob, int s) {
+    const int i = s < ob.cap ? s : ob.cap - 1;
+    n = ob.cnt[0];
+    k = ob.slot_shape[i];
+    b = ob.slot_block[i];
+    asm volatile("" ::"s"(n), "s"(k), "s"(b));
+  }
+};
+struct BlockHead {
+  int n, b, start, count, first;
+  __device__ BlockHead(const Obstacles& ob, int u) {
+    const int i = u < ob.cap ? u : ob.cap - 1;
+    n = ob.cnt[1];
+    b = ob.ub_block[i];
+    start = ob.ub_start[i];
+    count = ob.ub_count[i];
+    first = ob.ub_first[i];
+    asm volatile("" ::"s"(n), "s"(b), "s"(start), "s"(count), "s"(first));
+  }
+};
+
 // value of a dense field at global cell (gx, gy) with BlockLabOpen ghosts
 // (zero-gradient at the four domain faces, Definitions.h:125-157)
 template <typename RT>
@@ -163,7 +191,8 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
                                                    int nmaxpart,
                                                    const double* __restrict__ ramp,
                                                    int compute_dt, int step_idx, int phase,
-                                                   int end_prev) {
+                                                   int end_prev,
+                                                   const unsigned char* __restrict__ touch) {
   __shared__ int s_a[LCAP], s_b[LCAP], s_c[LCAP], s_d[LCAP];
   __shared__ int s_tmp[NT];
   __shared__ int s_cstart[MAX_SHAPES + 1];
@@ -182,7 +211,10 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
   __shared__ int s_fix[MAX_SHAPES][2];
   __shared__ double s_step[3];  // dt, U_inf
   // Every global value of the dt / motion part is loaded first, so the
-  // kernel waits for one round trip instead of one per dependent step.
+  // kernel waits for one round trip instead of one per dependent step (and
+  // the first NT blocks of the previous lists, tested against their count
+  // when they are cleared).
+  const int pvb = phase != 1 ? pv.ub_block[t < pv.cap ? t : pv.cap - 1] : 0;
   double mA = 0;  // the max of the projection's partials (count known upfront)
   if (phase != 2 && compute_dt) mA = max_array<NT>(maxpart, nmaxpart);
   double Tu = 0, Tv = 0, Tom = 0, Tcm0 = 0, Tcm1 = 0, Tl0 = 0, Tl1 = 0, Tor = 0, Tg0 = 0, Tg1 = 0;
@@ -299,7 +331,7 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
       if (c0 < 0 || c0 > g.extent0 || c1 < 0 || c1 > g.extent1) st->error = CUP2D_ERR_BODY_OUT;
     }
   }
-  if (phase != 2) {
+  if (phase == 1) {  // (phase 0: no swimmers, no early row pass)
     // the early row pass of the pressure solve runs when the previous step's
     // obstacle blocks lie in at most a quarter of the block rows (its patch
     // transforms the rows that hold obstacle blocks); ub_block is ascending
@@ -315,8 +347,9 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
   }
   if (phase != 1)
     for (int u = t; u < nub_prev; u += NT) {
-      obmap[pv.ub_block[u]] = 0;
-      ubidx[pv.ub_block[u]] = -1;
+      const int b = u < NT ? pvb : pv.ub_block[u];
+      obmap[b] = 0;
+      ubidx[b] = -1;
     }
   __syncthreads();
   if (phase == 1) return;
@@ -329,22 +362,9 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
       s_box[k][0] = Cx - R - safety; s_box[k][1] = Cx + R + safety;
       s_box[k][2] = Cy - R - safety; s_box[k][3] = Cy + R + safety;
     }
-    // a box that is not finite (a body moved by a non-finite velocity or dt;
-    // CUP2D_ERR_NONFINITE is raised by the dt part) selects no block: the
-    // block range is clamped in floating point before any integer conversion
-    bool fin = true;
-    double bb[4];
-    for (int q = 0; q < 4; ++q) {
-      const double x = s_box[k][q] / g.hb;
-      fin = fin && x == x && fabs(x) < 1e9;
-      bb[q] = fin ? x : 0.0;
-    }
-    int bx0 = (int)floor(bb[0]) - 1, bx1 = (int)floor(bb[1]) + 1;
-    int by0 = (int)floor(bb[2]) - 1, by1 = (int)floor(bb[3]) + 1;
-    bx0 = bx0 < 0 ? 0 : bx0; by0 = by0 < 0 ? 0 : by0;
-    bx1 = bx1 >= g.bpdx ? g.bpdx - 1 : bx1; by1 = by1 >= g.bpdy ? g.bpdy - 1 : by1;
-    const int w = fin && bx1 >= bx0 ? bx1 - bx0 + 1 : 0;
-    const int hgt = fin && by1 >= by0 ? by1 - by0 + 1 : 0;
+    int r[4];
+    candidate_range(g, s_box[k], r);
+    const int bx0 = r[0], by0 = r[1], w = r[2], hgt = r[3];
     s_rng[k][0] = bx0; s_rng[k][1] = by0; s_rng[k][2] = w;
     s_tmp[k] = w * hgt;
   }
@@ -374,7 +394,11 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
       const int local = cidx - s_cstart[k], w = s_rng[k][2];
       const int bx = s_rng[k][0] + local % w, by = s_rng[k][1] + local / w;
       const double bbox[2][2] = {{s_box[k][0], s_box[k][1]}, {s_box[k][2], s_box[k][3]}};
-      s_a[c] = sp[k].kind == 0 && touching(g, bx, by, bbox) ? 1 : 0;
+      // (touch: the swimmers' tests are done, k_fish_touch)
+      s_a[c] = sp[k].kind == 0 ? (touching(g, bx, by, bbox) ? 1 : 0)
+                               : (touch ? touch[(size_t)sp[k].fish * g.bpdx * g.bpdy + bx +
+                                                g.bpdx * by]
+                                        : 0);
       s_b[c] = bx + g.bpdx * by;
       s_c[c] = k;
     }
@@ -384,7 +408,7 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
     // block's box (grown by the chunk's largest safe distance) cannot pass
     // the first test of any of its segments, so only the pairs that meet it
     // are listed, and their (candidate, segment) tests run in parallel.
-    for (int k = 0; k < ns; ++k) {
+    for (int k = 0; !touch && k < ns; ++k) {
       if (sp[k].kind != 1) continue;
       const int c0 = s_cstart[k] > w0 ? s_cstart[k] - w0 : 0;
       const int c1 = s_cstart[k + 1] - w0 < nw ? s_cstart[k + 1] - w0 : nw;
@@ -520,6 +544,7 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
       ob.ub_block[u] = s_d[s];
       ob.ub_start[u] = s_cnt[s];
       ob.ub_count[u] = s_n[s];
+      ob.ub_first[u] = s;
       obmap[s_d[s]] = 1;
       ubidx[s_d[s]] = u;
     }
@@ -619,14 +644,15 @@ __device__ void obst_place_wg(int w, const Grid& g, const ShapeParams* __restric
   __shared__ int s_nbs[4][MAX_FISH];  // swimmer slots of the E, W, N, S neighbour blocks
   __shared__ int s_nbn[4];
   __shared__ DiskLds D;
-  const int nub = ob.cnt[1];
+  const BlockHead head(ob, w);
+  const int nub = head.n;
   if (w >= nub) {
     if (w >= nub + pv.cnt[1]) return;
     const int b = pv.ub_block[w - nub];
     if (!obmap[b]) clear_block(g, b, chi, udx, udy, invrho);
     return;
   }
-  const int b = ob.ub_block[w];
+  const int b = head.b;
   const int bx = b % g.bpdx, by = b / g.bpdx;
   for (int k = threadIdx.x; k < g.nshapes; k += NT) {
     D.kind[k] = sp[k].kind;
@@ -661,7 +687,7 @@ __device__ void obst_place_wg(int w, const Grid& g, const ShapeParams* __restric
   // the shape's distances of the block and the grid SDF of the cells across
   // its E, W, N, S edges: each distance (a square root) is evaluated once
   __shared__ double s_d[BS * BS], s_h[4][BS];
-  const int s0 = ob.ub_start[w], cnt = ob.ub_count[w];
+  const int s0 = head.start, cnt = head.count;
   const double h = g.h, i2h = 0.5 / h, fac = 0.5 * h;
   {  // the same cells for every shape of the block
     const int d = threadIdx.x / BS, j = threadIdx.x % BS;
@@ -671,7 +697,7 @@ __device__ void obst_place_wg(int w, const Grid& g, const ShapeParams* __restric
     }
   }
   for (int q = 0; q < cnt; ++q) {
-    const int s = ob.ub_slots[s0 + q], k = ob.slot_shape[s];
+    const int s = q == 0 ? head.first : ob.ub_slots[s0 + q], k = ob.slot_shape[s];
     SlotView o = slot(ob, s);
     // swimmers: dist, udef and rho = 1 come from PutFishOnBlocks
     const bool fish = D.kind[k] == 1;
@@ -805,12 +831,14 @@ __global__ __launch_bounds__(NT) void k_obst_moments(Grid g, const cup2d_shape_s
                                                      const StepState* __restrict__ st,
                                                      Obstacles ob) {
   __shared__ double lds[LDS_RED];
-  if ((int)blockIdx.x < ob.cnt[0]) obst_moments_wg(blockIdx.x, g, ss, ob, lds);
+  obst_moments_wg(blockIdx.x, g, ss, ob, lds);
 }
 
 __device__ void obst_moments_wg(int s, const Grid& g, const cup2d_shape_state* __restrict__ ss,
                                 const Obstacles& ob, double* lds) {
-  const int k = ob.slot_shape[s], b = ob.slot_block[s];
+  const SlotHead head(ob, s);
+  if (s >= head.n) return;
+  const int k = head.k, b = head.b;
   const int bx = b % g.bpdx, by = b / g.bpdx;
   SlotView o = slot(ob, s);
   const double hsq = g.h * g.h;
@@ -854,13 +882,13 @@ __global__ __launch_bounds__(NT) void k_obst_udef(Grid g, cup2d_shape_state* __r
                                                   const double* __restrict__ chi,
                                                   double* __restrict__ udx,
                                                   double* __restrict__ udy) {
-  const int nub = ob.cnt[1];
-  if ((int)blockIdx.x < nub) {
-    const int b = ob.ub_block[blockIdx.x];
+  const BlockHead head(ob, blockIdx.x);
+  if ((int)blockIdx.x < head.n) {
+    const int b = head.b;
     const int bx = b % g.bpdx, by = b / g.bpdx;
-    const int s0 = ob.ub_start[blockIdx.x], cnt = ob.ub_count[blockIdx.x];
+    const int s0 = head.start, cnt = head.count;
     for (int q = 0; q < cnt; ++q) {
-      const int s = ob.ub_slots[s0 + q], k = ob.slot_shape[s];
+      const int s = q == 0 ? head.first : ob.ub_slots[s0 + q], k = ob.slot_shape[s];
       SlotView o = slot(ob, s);
       // the block's cells are loaded before the shape's sums are reduced,
       // so the two memory latencies overlap
@@ -970,7 +998,7 @@ int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
     hipLaunchKernelGGL(k_obst_begin, dim3(1), dim3(NT), 0, c->stream, c->g, c->sp, c->ss, c->st,
                        c->ob, c->ob_prev, c->obmap, c->ubidx, c->fishd, c->maxpart, c->nwg,
                        c->ramp, compute_dt, c->graph_capture ? -1 : c->host_step, fish ? 1 : 0,
-                       end_prev);
+                       end_prev, nullptr);
   }
   // overlap 2: advDiff needs only dt and U_inf from the first phase of the
   // list builder; it runs on the side stream beside the whole chain, which
@@ -1015,9 +1043,12 @@ int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
   if (fish) {
     if (!(s = stream_for(ST_MIDLINE))) return CUP2D_ERR_HIP;
     RC_OB(enqueue_fish_midline(c, s));
+    const bool several = c->hfish.size() > 1;
+    if (several) RC_OB(enqueue_fish_touch(c, s));
     hipLaunchKernelGGL(k_obst_begin, dim3(1), dim3(NT), 0, s, c->g, c->sp, c->ss, c->st, c->ob,
                        c->ob_prev, c->obmap, c->ubidx, c->fishd, c->maxpart, c->nwg, c->ramp, 0,
-                       c->graph_capture ? -1 : c->host_step, 2, 0);
+                       c->graph_capture ? -1 : c->host_step, 2, 0,
+                       several ? c->fish_touch : nullptr);
     if (chain_main && mid_a_here) CUP2D_HIP_CHECK(c, hipEventRecord(c->ev_lists, c->stream));
     if (!(s = stream_for(ST_FISH_PLACE))) return CUP2D_ERR_HIP;
     RC_OB(enqueue_fish_place(c, s));
@@ -1141,8 +1172,9 @@ __device__ void rhs_obst1_wg(int w, const Grid& g, StepState* __restrict__ st,
                              const RT* __restrict__ v, double* lds) {
   // rhs_obst2_wg sets it again when an obstacle block lies in the fade band
   if (w == 0 && threadIdx.x == 0) st->rows_redo = 0;
-  if (w >= ob.cnt[1]) return;
-  const int b = ob.ub_block[w];
+  const BlockHead head(ob, w);
+  if (w >= head.n) return;
+  const int b = head.b;
   const int bx = b % g.bpdx, by = b / g.bpdx;
   if (u) {
     const RT corr = (RT)st->flux_corr;  // deferred advDiff flux correction
@@ -1152,9 +1184,9 @@ __device__ void rhs_obst1_wg(int w, const Grid& g, StepState* __restrict__ st,
       r[(size_t)y * g.NX + x] = rhs_cell<RT>(u, v, g.NX, g.NY, x, y, corr, facDiv);
     }
   }
-  const int s0 = ob.ub_start[w], cnt = ob.ub_count[w];
+  const int s0 = head.start, cnt = head.count;
   for (int q = 0; q < cnt; ++q) {
-    const int s = ob.ub_slots[s0 + q];
+    const int s = q == 0 ? head.first : ob.ub_slots[s0 + q];
     SlotView o = slot(ob, s);
     double sum = 0, pos = 0, neg = 0;
     CellStage cs;
@@ -1203,12 +1235,13 @@ __device__ void rhs_obst2_wg(int w, const Grid& g, StepState* __restrict__ st,
                              RT* __restrict__ r, const int* __restrict__ band_index,
                              double* __restrict__ fadepart, double* lds) {
   static_assert(NT == 256, "fade_block_sums is a 256-thread reduction");
-  if (w >= ob.cnt[1]) return;
-  const int b = ob.ub_block[w];
+  const BlockHead head(ob, w);
+  if (w >= head.n) return;
+  const int b = head.b;
   const int bx = b % g.bpdx, by = b / g.bpdx;
-  const int s0 = ob.ub_start[w], cnt = ob.ub_count[w];
+  const int s0 = head.start, cnt = head.count;
   for (int q = 0; q < cnt; ++q) {
-    const int s = ob.ub_slots[s0 + q], k = ob.slot_shape[s];
+    const int s = q == 0 ? head.first : ob.ub_slots[s0 + q], k = ob.slot_shape[s];
     SlotView o = slot(ob, s);
     // the block's cells are loaded before the shape's sums are reduced, so
     // the two memory latencies overlap
@@ -1521,7 +1554,10 @@ __device__ void momenta_wg(const Grid& g, const cup2d_shape_state* __restrict__ 
                            const StepState* __restrict__ st, const Obstacles& ob,
                            const RT* __restrict__ u, const RT* __restrict__ v, double* lds,
                            const SurfVel& sv) {
-  const int s = blockIdx.x, k = ob.slot_shape[s], b = ob.slot_block[s];
+  const int s = blockIdx.x;
+  const SlotHead head(ob, s);
+  if (s >= head.n) return;
+  const int k = head.k, b = head.b;
   const int bx = b % g.bpdx, by = b / g.bpdx;
   SlotView o = slot(ob, s);
   const double hsq = g.h * g.h;
@@ -1608,7 +1644,7 @@ __global__ __launch_bounds__(NT) void k_momenta(Grid g, const ShapeParams* __res
                                                 const RT* __restrict__ u,
                                                 const RT* __restrict__ v, SurfVel sv) {
   __shared__ double lds[LDS_RED];
-  if ((int)blockIdx.x < ob.cnt[0]) momenta_wg(g, ss, st, ob, u, v, lds, sv);
+  momenta_wg(g, ss, st, ob, u, v, lds, sv);
 }
 
 int enqueue_body_update(cup2d_ctx* c) {
@@ -1644,19 +1680,20 @@ __global__ __launch_bounds__(NT) void k_penalize(Grid g, const ShapeParams* __re
                                                  ForceSnap* __restrict__ snap, SurfVel sv) {
   __shared__ double lds[LDS_RED];
   __shared__ double s_uvw[MAX_SHAPES][3];
-  const int nub = ob.cnt[1];
+  const BlockHead head(ob, blockIdx.x);
+  const int nub = head.n;
   if ((int)blockIdx.x >= nub && !(SOLVE && blockIdx.x == 0)) return;
   const double dt = st->dt;
   // the block's velocities and chi are loaded first, so that their memory
   // latency overlaps the solve's reduction of the partials
   const bool mine = (int)blockIdx.x < nub;
-  const int b = mine ? ob.ub_block[blockIdx.x] : 0;
+  const int b = mine ? head.b : 0;
   const int bx = b % g.bpdx, by = b / g.bpdx;
   constexpr int NC = BS * BS / NT;
   double uR[NC], vR[NC], cR[NC];
   // and the block's first slot (the only one unless shapes overlap)
-  const int s0 = mine ? ob.ub_start[blockIdx.x] : 0, cnt = mine ? ob.ub_count[blockIdx.x] : 0;
-  const int sf = mine ? ob.ub_slots[s0] : 0;
+  const int s0 = head.start, cnt = mine ? head.count : 0;
+  const int sf = mine ? head.first : 0;
   double fX[NC], fU[NC], fV[NC];
   if (mine) {
     const SlotView o = slot(ob, sf);
@@ -1800,8 +1837,10 @@ __global__ __launch_bounds__(NT) void k_iter_momenta(Grid g, const cup2d_shape_s
                                                      const double* __restrict__ fu,
                                                      const double* __restrict__ fv) {
   __shared__ double lds[LDS_RED];
-  if ((int)blockIdx.x >= ob.cnt[0]) return;
-  const int s = blockIdx.x, k = ob.slot_shape[s], b = ob.slot_block[s];
+  const int s = blockIdx.x;
+  const SlotHead head(ob, s);
+  if (s >= head.n) return;
+  const int k = head.k, b = head.b;
   const int bx = b % g.bpdx, by = b / g.bpdx;
   SlotView o = slot(ob, s);
   const double hsq = g.h * g.h;
@@ -1858,13 +1897,14 @@ __global__ __launch_bounds__(NT) void k_iter_penalize(Grid g, const cup2d_shape_
                                                       double* __restrict__ v,
                                                       double* __restrict__ part) {
   __shared__ double lds[LDS_RED];
-  if ((int)blockIdx.x >= ob.cnt[1]) return;
-  const int b = ob.ub_block[blockIdx.x];
+  const BlockHead head(ob, blockIdx.x);
+  if ((int)blockIdx.x >= head.n) return;
+  const int b = head.b;
   const int bx = b % g.bpdx, by = b / g.bpdx;
-  const int s0 = ob.ub_start[blockIdx.x], cnt = ob.ub_count[blockIdx.x];
+  const int s0 = head.start, cnt = head.count;
   double a[4] = {0, 0, 0, 0};
   for (int q = 0; q < cnt; ++q) {
-    const int s = ob.ub_slots[s0 + q], k = ob.slot_shape[s];
+    const int s = q == 0 ? head.first : ob.ub_slots[s0 + q], k = ob.slot_shape[s];
     SlotView o = slot(ob, s);
     const double u_s = ss[k].u, v_s = ss[k].v, omega_s = ss[k].omega;
     const double Cx = ss[k].centerOfMass[0], Cy = ss[k].centerOfMass[1];
@@ -1981,7 +2021,9 @@ __device__ void forces_wg(int s, const Grid& g, const ForceSnap* __restrict__ sn
                           const Obstacles& ob, const RT* __restrict__ u,
                           const RT* __restrict__ v, const double* __restrict__ p, double* lds,
                           const SurfVel& surf) {
-  const int k = ob.slot_shape[s], b = ob.slot_block[s];
+  const SlotHead head(ob, s);
+  if (s >= head.n) return;
+  const int k = head.k, b = head.b;
   const int bx = b % g.bpdx, by = b / g.bpdx;
   SlotView o = slot(ob, s);
   const double NUoH = g.nu / g.h;
@@ -2054,7 +2096,7 @@ __global__ __launch_bounds__(NT) void k_forces(Grid g, const ForceSnap* __restri
                                                const RT* __restrict__ v,
                                                const double* __restrict__ p, SurfVel sv) {
   __shared__ double lds[LDS_RED];
-  if ((int)blockIdx.x < ob.cnt[0]) forces_wg(blockIdx.x, g, snap, ob, u, v, p, lds, sv);
+  forces_wg(blockIdx.x, g, snap, ob, u, v, p, lds, sv);
 }
 
 // shape totals (Shape::computeForces, Shape.cpp:252-300) and, with end_step,
@@ -2106,7 +2148,7 @@ __global__ __launch_bounds__(256, 4) void k_step_place(
   }
   if (w < nfront) {  // nfront: nplace + nforces rounded up to a multiple of 8
     w -= nplace;
-    if (w < nforces && w < pv.cnt[0]) forces_wg(w, g, snap, pv, u, v, p, lds, sv);
+    if (w < nforces) forces_wg(w, g, snap, pv, u, v, p, lds, sv);
     return;
   }
   // the strips, each XCD's a contiguous band (workgroup b runs on XCD b % 8)
@@ -2126,7 +2168,7 @@ __global__ __launch_bounds__(NT) void k_step_moments(Grid g, cup2d_shape_state* 
   __shared__ double lds[LDS_RED];
   const int w = blockIdx.x;
   if (w < G) {
-    if (w < ob.cnt[0]) obst_moments_wg(w, g, ss, ob, lds);
+    obst_moments_wg(w, g, ss, ob, lds);
   } else if (w == G) {
     const double corr = flux_corr(fluxpart, edge_count(gx, gy), g, lds);
     if (threadIdx.x == 0) {
@@ -2152,7 +2194,8 @@ int enqueue_step_front(cup2d_ctx* c, int compute_dt, const FrontAcc& acc) {
     TimerScope ts(c, T_PUT_OBJECTS);
     hipLaunchKernelGGL(k_obst_begin, dim3(1), dim3(NT), 0, c->stream, c->g, c->sp, c->ss, c->st,
                        c->ob, c->ob_prev, c->obmap, c->ubidx, c->fishd, c->maxpart, c->nwg,
-                       c->ramp, compute_dt, c->graph_capture ? -1 : c->host_step, 0, end_prev);
+                       c->ramp, compute_dt, c->graph_capture ? -1 : c->host_step, 0, end_prev,
+                       nullptr);
   }
   const int NX = c->g.NX, gx = strips_x(NX), gy = c->g.NY / STENCIL_RY;
   const int nplace = 2 * G, nforces = forces ? G : 0, nfront = (nplace + nforces + 7) / 8 * 8;
@@ -2254,7 +2297,7 @@ int enqueue_shapes_reset(cup2d_ctx* c) {
 static int obstacles_alloc_one(cup2d_ctx* c, Obstacles& o, int cap) {
   o.cap = cap;
   const size_t cells = (size_t)cap * BS * BS;
-  const size_t ni = (size_t)6 * cap + 2 + MAX_SHAPES + 1;
+  const size_t ni = (size_t)7 * cap + 2 + MAX_SHAPES + 1;
   int* ibuf = nullptr;
   CUP2D_HIP_CHECK(c, hipMalloc(&ibuf, sizeof(int) * ni));
   CUP2D_HIP_CHECK(c, hipMemset(ibuf, 0, sizeof(int) * ni));
@@ -2264,8 +2307,9 @@ static int obstacles_alloc_one(cup2d_ctx* c, Obstacles& o, int cap) {
   o.ub_start = ibuf + 3 * cap;
   o.ub_count = ibuf + 4 * cap;
   o.ub_slots = ibuf + 5 * cap;
-  o.cnt = ibuf + 6 * cap;
-  o.slot_of_shape_start = ibuf + 6 * cap + 2;
+  o.ub_first = ibuf + 6 * cap;
+  o.cnt = ibuf + 7 * cap;
+  o.slot_of_shape_start = ibuf + 7 * cap + 2;
   double* dbuf = nullptr;
   const size_t nd = cells * 9 + (size_t)cap * SLOT_PART;
   CUP2D_HIP_CHECK(c, hipMalloc(&dbuf, sizeof(double) * nd));
@@ -2298,6 +2342,8 @@ int obstacles_alloc(cup2d_ctx* c) {
   // list builder holds while the actual obstacle blocks fit: the list
   // builder reports CUP2D_ERR_CAPACITY when they do not
   cap = cap > OBST_LIST_CAP ? OBST_LIST_CAP : cap;
+  if (c->hfish.size() > 1)
+    CUP2D_HIP_CHECK(c, hipMalloc(&c->fish_touch, c->hfish.size() * (size_t)nblocks));
   int rc = obstacles_alloc_one(c, c->ob, cap);
   if (rc) return rc;
   return obstacles_alloc_one(c, c->ob_prev, cap);
