@@ -1,6 +1,8 @@
 // advdiff.hpp -- the advection-diffusion strip of the full-grid stencil kernels.
 #pragma once
 
+#include <type_traits>
+
 #include "device_util.hpp"
 
 namespace cup2d {
@@ -23,6 +25,24 @@ static inline int strip_width(int NX) {
 }
 static inline int strips_x(int NX) { return (NX + strip_width(NX) - 1) / strip_width(NX); }
 static inline bool ragged(int NX) { return NX % strip_width(NX) != 0; }
+// fn(RAGGED, STREAM, T{}) as compile-time values: whether the grid's last
+// strips (of the given width) are ragged, whether its stores are streamed, and
+// the planes' type
+template <typename F>
+inline void strip_dispatch(const cup2d_ctx* c, int width, F&& fn) {
+  const bool rg = c->g.NX % width != 0;
+  if (c->f32) {
+    if (rg) fn(std::true_type{}, std::false_type{}, float{});
+    else fn(std::false_type{}, std::false_type{}, float{});
+  } else if (c->stream_stores) {
+    if (rg) fn(std::true_type{}, std::true_type{}, double{});
+    else fn(std::false_type{}, std::true_type{}, double{});
+  } else {
+    if (rg) fn(std::true_type{}, std::false_type{}, double{});
+    else fn(std::false_type{}, std::false_type{}, double{});
+  }
+}
+
 // the statement with RAGGED = whether the grid's last strips are ragged
 #define CUP2D_RAGGED_DISPATCH(NX, ...)  \
   do {                                  \
@@ -53,7 +73,8 @@ struct WaveEdges {
 // IF = sum_E u - sum_W u + sum_N v - sum_S v (advDiff.cpp:93-102).
 // T: the velocity planes' type; the stencil is evaluated in T (FP32 at
 // FP32 precision), the factors are formed in double and rounded once.
-template <int RY, bool RAGGED, typename T>
+// STREAM: the stores are non-temporal (cup2d_ctx::stream_stores).
+template <int RY, bool RAGGED, bool STREAM, typename T>
 __device__ inline void advdiff_strip(const T* __restrict__ u, const T* __restrict__ v,
                                      T* __restrict__ uo, T* __restrict__ vo,
                                      const Grid& g, const StepState* __restrict__ st,
@@ -129,8 +150,13 @@ __device__ inline void advdiff_strip(const T* __restrict__ u, const T* __restric
     const T v1 = vc + (afac * dVadv + dfac * dVdif);
     const size_t idx = i0 + (size_t)iy * NX;
     if (in) {
-      uo[idx] = u1;
-      vo[idx] = v1;
+      if constexpr (STREAM) {
+        __builtin_nontemporal_store(u1, uo + idx);
+        __builtin_nontemporal_store(v1, vo + idx);
+      } else {
+        uo[idx] = u1;
+        vo[idx] = v1;
+      }
     }
     // selects, not branches, so the row loop stays one basic block
     flux = x == 0 ? flux - u1 : flux;

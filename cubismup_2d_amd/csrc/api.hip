@@ -580,6 +580,7 @@ int cup2d_create(const cup2d_cfg* cfg, cup2d_ctx** out) {
     return bail(CUP2D_ERR_HIP);
   }
   const size_t n = (size_t)g.NX * g.NY;
+  c->stream_stores = !c->f32 && n * 6 * sizeof(double) > (size_t)256 << 20;
   double** planes[] = {&c->u, &c->v, &c->tu, &c->tv, &c->pres, &c->rhs,
                        &c->chi, &c->udx, &c->udy, &c->invrho, &c->vfu, &c->vfv};
   for (double** p : planes)

@@ -718,7 +718,8 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_fwd(
 // OUT_SET: out (double) = x; OUT_ADD: out (double) += x (the FP64 update of a
 // refinement sweep); OUT_RES: out (float) = b - x, b the float RHS plane
 // (the residual of a refinement sweep, x = the FP64 operator applied to p).
-// With S = double and OUT_SET the pass is the plain FP64 one.
+// With S = double and OUT_SET the pass is the plain FP64 one; stream: its
+// stores are non-temporal (cup2d_ctx::stream_stores).
 enum { OUT_SET = 0, OUT_ADD = 1, OUT_RES = 2, OUT_RES_FWD = 3 };
 // OUT_RES_FWD (FP64 transform, float residual): OUT_RES whose residual rows,
 // rounded to float as OUT_RES stores them, are transformed forward in FP32
@@ -741,7 +742,8 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
                                                          double* __restrict__ respart,
                                                          float2* __restrict__ spec32,
                                                          const float2* __restrict__ tw32,
-                                                         const cplx<S>* __restrict__ dct) {
+                                                         const cplx<S>* __restrict__ dct,
+                                                         int stream) {
   using V = cplx<S>;
   constexpr int NT = L / E, PADL = lds_len<L, E>();
   constexpr bool RES = OUT == OUT_RES || OUT == OUT_RES_FWD;
@@ -893,6 +895,9 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
         if constexpr (OUT == OUT_ADD) {
           o0[i] += (double)x[q].x - pm;
           o1[i] += (double)x[q].y - pm;
+        } else if (stream) {
+          __builtin_nontemporal_store((double)x[q].x, o0 + i);
+          __builtin_nontemporal_store((double)x[q].y, o1 + i);
         } else {
           o0[i] = (double)x[q].x;
           o1[i] = (double)x[q].y;
@@ -1247,7 +1252,8 @@ static void launch_rows_inv(cup2d_ctx* c, const cplx<S>* spec, int spec_rows, vo
   const int pairs = nrows / 2;
   CUP2D_TIMED_LAUNCH(c, (k_rows_inv<L, NP, RE, S, OUT, KIND>), dim3((pairs + NP - 1) / NP),
                      dim3(NP * L / RE), shm, c->stream, spec, spec_rows, out, bres, pitch,
-                     ncols, nrows, tw, mean, c->respart, spec32, tw32, dct);
+                     ncols, nrows, tw, mean, c->respart, spec32, tw32, dct,
+                     c->stream_stores ? 1 : 0);
 }
 template <int LC, int MODE, typename S>
 static int launch_cols(cup2d_ctx* c, cplx<S>* spec, int ncg, const ColParams& P,

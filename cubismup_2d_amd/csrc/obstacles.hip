@@ -2131,7 +2131,7 @@ static int launch_forces(cup2d_ctx* c, hipStream_t s, const Obstacles& lists, in
 // placement writes this step's slots and the dense obstacle planes, the forces
 // read the previous step's lists, velocity and pressure.  The latency-bound
 // workgroups come first, so they start at once and the strips fill the rest.
-template <typename T, bool RAGGED>
+template <typename T, bool RAGGED, bool STREAM>
 __global__ __launch_bounds__(256, 4) void k_step_place(
     Grid g, const ShapeParams* __restrict__ sp, const cup2d_shape_state* __restrict__ ss,
     Obstacles ob, Obstacles pv, const unsigned char* __restrict__ obmap,
@@ -2154,7 +2154,7 @@ __global__ __launch_bounds__(256, 4) void k_step_place(
   // the strips, each XCD's a contiguous band (workgroup b runs on XCD b % 8)
   const int n = gx * gy, id = w - nfront;
   const int t = (n % 8 == 0) ? (id % 8) * (n / 8) + id / 8 : id;
-  advdiff_strip<STENCIL_RY, RAGGED, T>(u, v, uo, vo, g, st, fluxpart, t % gx, t / gx, gx, gy, lds);
+  advdiff_strip<STENCIL_RY, RAGGED, STREAM, T>(u, v, uo, vo, g, st, fluxpart, t % gx, t / gx, gx, gy, lds);
 }
 
 // G workgroups of moments, then the flux reduction, then (forces) the totals
@@ -2202,20 +2202,16 @@ int enqueue_step_front(cup2d_ctx* c, int compute_dt, const FrontAcc& acc) {
   {
     KernelTimer kt(c, T_ADVDIFF);
     // strips narrower than a workgroup (NX < 256) are ragged ones of it
-    auto launch = [&](auto rg) {
-      constexpr bool RAGGED = rg();
-      CUP2D_REAL_DISPATCH(
-          c, CUP2D_TIMED_LAUNCH(c, (k_step_place<T, RAGGED>), dim3(nfront + gx * gy), dim3(256), 0,
-                                c->stream, c->g, (const ShapeParams*)c->sp,
-                                (const cup2d_shape_state*)c->ss, c->ob, c->ob_prev,
-                                (const unsigned char*)c->obmap, (const int*)c->ubidx, c->chi,
-                                c->udx, c->udy, c->invrho, nplace, nforces, nfront,
-                                (const ForceSnap*)c->fsnap, (const double*)c->pres, surf_of(c),
-                                tp<T>(c->u), tp<T>(c->v), tp<T>(c->tu), tp<T>(c->tv),
-                                (const StepState*)c->st, c->fluxpart, gx, gy));
-    };
-    if (NX % 256 != 0) launch(std::true_type{});
-    else launch(std::false_type{});
+    strip_dispatch(c, 256, [&](auto rg, auto stream, auto real) {
+      using T = decltype(real);
+      CUP2D_TIMED_LAUNCH(c, (k_step_place<T, rg(), stream()>), dim3(nfront + gx * gy), dim3(256), 0,
+                         c->stream, c->g, (const ShapeParams*)c->sp,
+                         (const cup2d_shape_state*)c->ss, c->ob, c->ob_prev,
+                         (const unsigned char*)c->obmap, (const int*)c->ubidx, c->chi, c->udx,
+                         c->udy, c->invrho, nplace, nforces, nfront, (const ForceSnap*)c->fsnap,
+                         (const double*)c->pres, surf_of(c), tp<T>(c->u), tp<T>(c->v),
+                         tp<T>(c->tu), tp<T>(c->tv), (const StepState*)c->st, c->fluxpart, gx, gy);
+    });
   }
   std::swap(c->u, c->tu);  // advDiff.cpp:81-87 copy tmpV -> vel
   std::swap(c->v, c->tv);

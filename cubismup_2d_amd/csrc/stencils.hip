@@ -154,7 +154,7 @@ __device__ inline void stencil_tile(int* bx, int* by) {
 // grid smaller than that each workgroup takes the strips id, id + gridDim.x,
 // ... (the grid is a multiple of 8, so a workgroup keeps its XCD), which
 // leaves workgroup slots free for the obstacle kernels of the side stream.
-template <int RY, bool RAGGED, typename T>
+template <int RY, bool RAGGED, bool STREAM, typename T>
 __global__ __launch_bounds__(256) void k_advdiff(const T* __restrict__ u,
                                                  const T* __restrict__ v,
                                                  T* __restrict__ uo, T* __restrict__ vo,
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void k_advdiff(const T* __restrict__ u,
   const int n = gx * gy;
   for (int id = blockIdx.x; id < n; id += gridDim.x) {
     const int t = (n % 8 == 0) ? (id % 8) * (n / 8) + id / 8 : id;
-    advdiff_strip<RY, RAGGED, T>(u, v, uo, vo, g, st, fluxpart, t % gx, t / gx, gx, gy, lds);
+    advdiff_strip<RY, RAGGED, STREAM, T>(u, v, uo, vo, g, st, fluxpart, t % gx, t / gx, gx, gy, lds);
   }
 }
 
@@ -212,9 +212,12 @@ int enqueue_advdiff_on(cup2d_ctx* c, int defer_fix, hipStream_t s) {
   {
     const int nwg = gx * gy;
     KernelTimer kt(c, T_ADVDIFF);
-    CUP2D_RAGGED_DISPATCH(c->g.NX, CUP2D_REAL_DISPATCH(c, CUP2D_TIMED_LAUNCH(
-        c, (k_advdiff<RYS, RAGGED, T>), dim3(nwg), dim3(tx), 0, s, tp<T>(c->u), tp<T>(c->v),
-        tp<T>(c->tu), tp<T>(c->tv), c->g, (const StepState*)c->st, c->fluxpart, gx, gy)));
+    strip_dispatch(c, tx, [&](auto rg, auto stream, auto real) {
+      using T = decltype(real);
+      CUP2D_TIMED_LAUNCH(c, (k_advdiff<RYS, rg(), stream(), T>), dim3(nwg), dim3(tx), 0, s,
+                         tp<T>(c->u), tp<T>(c->v), tp<T>(c->tu), tp<T>(c->tv), c->g,
+                         (const StepState*)c->st, c->fluxpart, gx, gy);
+    });
   }
   std::swap(c->u, c->tu);  // advDiff.cpp:81-87 copy tmpV -> vel
   std::swap(c->v, c->tv);
