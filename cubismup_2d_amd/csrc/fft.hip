@@ -24,10 +24,11 @@
 // pass transforms two real columns at once.  (Transforming the 2NX x 2NY
 // mirror image instead took twice the spectrum and four times the column
 // work: column pass at 2048 x 1024 36.2 us, solve at 1024 x 512 47 us.)
-// The FFT core is a radix-16 Stockham autosort (radix 2/4/8 for the last
-// pass), 16 complex values per thread in registers, LDS padded by one slot
-// every 16 entries so stride-16 stores are bank-conflict free.  Twiddles come
-// from per-length tables exp(-2 pi i k/L) built in long double on the host.
+// The FFT core is a Stockham autosort of radix E = 8 or 16 (row_e, col_e; a
+// smaller radix for the last pass), E complex values per thread in registers,
+// LDS padded by one slot every E entries so stride-E stores are bank-conflict
+// free.  Twiddles come from per-length tables exp(-2 pi i k/L) built in long
+// double on the host.
 #include <cmath>
 #include <type_traits>
 #include <utility>
@@ -365,6 +366,75 @@ __device__ __forceinline__ void fft_regs(V* x, V* lds, int base, int stride, int
   pass_first<L, E, FWD>(x, lds, base, stride, t);
   fft_tail<L, E, E, FWD>(lds, base, stride, t, w, x);
 }
+
+// The same transform with the real and imaginary parts exchanged one after
+// the other, so that the LDS holds reals: half the memory for twice the
+// barriers.  Every exchange reads the elements t + q*NT back.
+// The twiddle bases of a pass are loaded while the exchange before it holds
+// half of the registers' data in LDS; t is hidden from the compiler at each
+// exchange, which would otherwise keep every exchange's addresses at once.
+template <int L, int E, int NS, typename V, typename F>
+__device__ __forceinline__ void exchange_split(V* x, typename ScalarOf<V>::type* lds, int t,
+                                               const V* __restrict__ tw, V* w, F&& widx) {
+  constexpr int NT = L / E, R = TwCount<L, E, NS>::R;
+  asm volatile("" : "+v"(t));
+#pragma unroll
+  for (int r = 0; r < E; ++r) lds[padE<E>(widx(r))] = x[r].x;
+  __syncthreads();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int p = 0; p < E / R; ++p) w[p] = tw[((t + p * NT) % NS) * (L / (NS * R))];
+#pragma unroll
+  for (int q = 0; q < E; ++q) x[q].x = lds[padE<E>(t + q * NT)];
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < E; ++r) lds[padE<E>(widx(r))] = x[r].y;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < E; ++q) x[q].y = lds[padE<E>(t + q * NT)];
+  __syncthreads();
+}
+template <int L, int E, int NS, bool FWD, typename V>
+__device__ __forceinline__ void fft_tail_split(V* x, typename ScalarOf<V>::type* lds, int t,
+                                               const V* __restrict__ tw, const V* w) {
+  constexpr int R = TwCount<L, E, NS>::R, PER = E / R;
+  if constexpr (NS * R < L) {
+    static_assert(R == E, "only the last pass has a smaller radix");
+    dft_tw<E, FWD>(x, w[0]);
+    V wn[E / TwCount<L, E, NS * E>::R];
+    const int idxD = (t / NS) * NS * E + t % NS;
+    exchange_split<L, E, NS * E>(x, lds, t, tw, wn, [&](int r) { return idxD + r * NS; });
+    fft_tail_split<L, E, NS * E, FWD>(x, lds, t, tw, wn);
+  } else {  // butterfly p holds the elements p + PER r
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      V v[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = x[p + PER * r];
+      dft_tw<R, FWD>(v, w[p]);
+#pragma unroll
+      for (int r = 0; r < R; ++r) x[p + PER * r] = v[r];
+    }
+  }
+}
+template <int L, int E, bool FWD, typename V>
+__device__ __forceinline__ void fft_regs_split(V* x, typename ScalarOf<V>::type* lds, int t,
+                                               const V* __restrict__ tw) {
+  dft<E, FWD>(x);
+  V w[E / TwCount<L, E, E>::R];
+  exchange_split<L, E, E>(x, lds, t, tw, w, [&](int r) { return t * E + r; });
+  fft_tail_split<L, E, E, FWD>(x, lds, t, tw, w);
+}
+
+// FP64 inverse rows of 8192: a complex row pair fills the LDS of a CU, whose
+// one workgroup then loads, transforms and stores with nothing beside it; the
+// split exchange lets two share it, within 128 registers.  Inverse rows of
+// 8192 x 4096 132 -> 103 us, of the doubled 4000 x 2016 57 -> 49 us.  The
+// forward rows (57 -> 58 us; 271 -> 420 us with the RHS, whose source rows
+// spill) and columns of 4096 (periodic 162 -> 186 us, free-space 119 -> 118)
+// gain nothing and keep the complex exchange.
+template <int L, typename S, int OUT>
+constexpr bool row_split() { return L >= 8192 && sizeof(S) == 8 && OUT == 0; }
 
 template <int L, int E>
 constexpr int lds_len() { return L + L / E; }
@@ -733,7 +803,8 @@ enum { OUT_SET = 0, OUT_ADD = 1, OUT_RES = 2, OUT_RES_FWD = 3 };
 // sum (b - mean_wg b)^2 (the residual norm of the sweep without the mean,
 // which the operator does not see; k_res_reduce merges them).
 template <int L, int NP, int E, typename S, int OUT, int KIND = KIND_SEQ>
-__global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const cplx<S>* __restrict__ spec,
+__global__ __launch_bounds__(NP * L / E, (row_split<L, S, OUT>() ? 4 : min_waves<E>())) void k_rows_inv(
+                                                         const cplx<S>* __restrict__ spec,
                                                          int spec_rows, void* __restrict__ outv,
                                                          const float* __restrict__ bres,
                                                          int out_pitch, int ncols, int nrows,
@@ -747,6 +818,8 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
   using V = cplx<S>;
   constexpr int NT = L / E, PADL = lds_len<L, E>();
   constexpr bool RES = OUT == OUT_RES || OUT == OUT_RES_FWD;
+  constexpr bool SPLIT = row_split<L, S, OUT>();
+  constexpr int U0 = SPLIT ? L / 2 : 0;  // the partner's first element (half the LDS holds them)
   extern __shared__ __align__(16) unsigned char smem_raw[];
   V* lds = reinterpret_cast<V*>(smem_raw);
   const int f = threadIdx.x / NT, t = threadIdx.x % NT;
@@ -754,7 +827,7 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
   const bool valid = y0 < nrows;
   const int base = f * PADL;
   V w[TwCount<L, E, E>::n];
-  tw_load<L, E, E>(tw, t, w);
+  if constexpr (!SPLIT) tw_load<L, E, E>(tw, t, w);
   V x[E];
   // Z_k = A_k + i B_k and Z_{L-k} = conj(A_k) + i conj(B_k); DC and Nyquist
   // of both rows are packed in slot 0 (real parts only).  All loads are
@@ -791,17 +864,22 @@ __global__ __launch_bounds__(NP * L / E, min_waves<E>()) void k_rows_inv(const c
         B.y = -B.y;
       }
       x[q] = mk<V>(A.x - B.y, A.y + B.x);
-      lds[base + padE<E>(L - k)] = mk<V>(A.x + B.y, -A.y + B.x);
+      lds[base + padE<E>(L - k - U0)] = mk<V>(A.x + B.y, -A.y + B.x);
     }
   }
   __syncthreads();
 #pragma unroll
   for (int q = E / 2; q < E; ++q) {
     const int i = t + q * NT;
-    if (i != L / 2) x[q] = lds[base + padE<E>(i)];
+    if (i != L / 2) x[q] = lds[base + padE<E>(i - U0)];
   }
   __syncthreads();
-  fft_regs<L, E, false>(x, lds, base, 1, t, w);
+  if constexpr (SPLIT) {
+    static_assert(NP == 1 && KIND == KIND_SEQ, "one row pair, no reordering");
+    fft_regs_split<L, E, false>(x, reinterpret_cast<S*>(smem_raw), t, tw);
+  } else {
+    fft_regs<L, E, false>(x, lds, base, 1, t, w);
+  }
   if constexpr (KIND == KIND_COS) {  // back to the grid's order, through LDS
 #pragma unroll
     for (int q = 0; q < E; ++q)
@@ -1248,7 +1326,8 @@ static void launch_rows_inv(cup2d_ctx* c, const cplx<S>* spec, int spec_rows, vo
   constexpr int RE = row_e<L>();
   c->rows_inv_wgs = (nrows / 2 + rows_np<L, RE>() - 1) / rows_np<L, RE>();
   constexpr int NP = rows_np<L, RE>();
-  const size_t shm = (size_t)NP * lds_len<L, RE>() * sizeof(cplx<S>);
+  const size_t shm = (size_t)NP * lds_len<L, RE>() * sizeof(cplx<S>) /
+                     (row_split<L, S, OUT>() ? 2 : 1);
   const int pairs = nrows / 2;
   CUP2D_TIMED_LAUNCH(c, (k_rows_inv<L, NP, RE, S, OUT, KIND>), dim3((pairs + NP - 1) / NP),
                      dim3(NP * L / RE), shm, c->stream, spec, spec_rows, out, bres, pitch,
