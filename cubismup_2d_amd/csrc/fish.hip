@@ -549,7 +549,7 @@ __device__ inline void block_inscan(int v, int* out, int* tmp) {
 // meet a block) keeps every pair's distance in registers between the two
 // passes and takes the winners' points from LDS; scans and compactions go by
 // shuffles and ballots instead of log-step LDS scans (16 barriers each):
-// 26 -> TODO us alone at 4096 x 2048.
+// 39 -> 35 us beside advDiff at 4096 x 2048.
 __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __restrict__ sp,
                                                    const cup2d_shape_state* __restrict__ ss,
                                                    const FishDev* __restrict__ fd,
@@ -821,41 +821,6 @@ __global__ __launch_bounds__(NT) void k_fish_place(Grid g, const ShapeParams* __
   }
 }
 
-// Does any segment of swimmer blockIdx.y meet a candidate block of the list
-// builder (AreaSegment::isIntersectingWithAABB, Fish.cpp:158-173)?  A wave per
-// candidate, its lanes taking the segments; the answers go to
-// touch[swimmer][block].  With several swimmers the list builder, one
-// workgroup, spent most of its time on these tests one swimmer after another
-// (8192 x 4096 with four: TODO us); with one, its own prefiltered tests take
-// less than another launch.
-__global__ __launch_bounds__(NT) void k_fish_touch(Grid g, const FishDev* __restrict__ fd,
-                                                   unsigned char* __restrict__ touch) {
-  const int f = blockIdx.y, lane = threadIdx.x % 64;
-  const FishDev& F = fd[f];
-  const int nseg = F.Nseg;
-  const double box[4] = {F.box[0], F.box[1], F.box[2], F.box[3]};
-  int r[4];  // bx0, by0, width, height
-  candidate_range(g, box, r);
-  unsigned char* out = touch + (size_t)f * g.bpdx * g.bpdy;
-  for (int c = blockIdx.x * (NT / 64) + threadIdx.x / 64; c < r[2] * r[3];
-       c += gridDim.x * (NT / 64)) {
-    const int bx = r[0] + c % r[2], by = r[1] + c / r[2];
-    double start[2], end[2];
-    block_corners(g, bx, by, start, end);
-    bool hit = false;
-    for (int i = lane; i < nseg; i += 64)
-      hit |= seg_intersects(F.seg + (size_t)i * FISH_SEGD, start, end);
-    const unsigned long long m = __ballot(hit);
-    if (lane == 0) out[bx + g.bpdx * by] = m != 0;
-  }
-}
-
-int enqueue_fish_touch(cup2d_ctx* c, hipStream_t s) {
-  hipLaunchKernelGGL(k_fish_touch, dim3(64, (int)c->hfish.size()), dim3(NT), 0, s, c->g, c->fishd,
-                     c->fish_touch);
-  return launch_check(c, "fish touch");
-}
-
 // ------------------------------------------------------------------- host
 // FishData::FishData (FishLibrary.cpp:14-38, FishLibrary.h:44-60) and the
 // half-width table (AmplitudeFish::_width, CarlingFish.cpp:41-48, or the
@@ -961,8 +926,6 @@ void fish_free_all(cup2d_ctx* c) {
   c->hfish.clear();
   if (c->fishd) (void)hipFree(c->fishd);
   c->fishd = nullptr;
-  if (c->fish_touch) (void)hipFree(c->fish_touch);
-  c->fish_touch = nullptr;
 }
 
 // The time-only part lives in buffer host_step & 1: computed here when it is

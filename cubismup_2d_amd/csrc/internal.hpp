@@ -277,7 +277,6 @@ struct cup2d_ctx {
   int* ubidx = nullptr;                    // [blocks] distinct-block index this step, -1 if none
   cup2d::FishDev* fishd = nullptr;         // device [MAX_FISH]
   std::vector<cup2d::FishDev> hfish;       // host copy (device pointers)
-  unsigned char* fish_touch = nullptr;     // [swimmers][blocks], with more than one (k_fish_touch)
   int band_nblocks = 0;
   int* band_blocks = nullptr;              // blocks touched by the cub2rhs fade
   int* band_index = nullptr;               // [blocks] position in band_blocks, -1 if none
@@ -466,7 +465,6 @@ int enqueue_fish_midline(cup2d_ctx* c, hipStream_t s);
 // the time-only part of the next whole step's midline (time + dt)
 int enqueue_fish_mid_next(cup2d_ctx* c, int parity, hipEvent_t after, bool join_aux);
 int enqueue_fish_place(cup2d_ctx* c, hipStream_t s);
-int enqueue_fish_touch(cup2d_ctx* c, hipStream_t s);
 // PressureIterator_unif pieces (PressureIterator_unif.cpp)
 int enqueue_copy_vel_to_tmpv(cup2d_ctx* c);
 int enqueue_iter_project(cup2d_ctx* c);

@@ -191,8 +191,7 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
                                                    int nmaxpart,
                                                    const double* __restrict__ ramp,
                                                    int compute_dt, int step_idx, int phase,
-                                                   int end_prev,
-                                                   const unsigned char* __restrict__ touch) {
+                                                   int end_prev) {
   __shared__ int s_a[LCAP], s_b[LCAP], s_c[LCAP], s_d[LCAP];
   __shared__ int s_tmp[NT];
   __shared__ int s_cstart[MAX_SHAPES + 1];
@@ -394,11 +393,7 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
       const int local = cidx - s_cstart[k], w = s_rng[k][2];
       const int bx = s_rng[k][0] + local % w, by = s_rng[k][1] + local / w;
       const double bbox[2][2] = {{s_box[k][0], s_box[k][1]}, {s_box[k][2], s_box[k][3]}};
-      // (touch: the swimmers' tests are done, k_fish_touch)
-      s_a[c] = sp[k].kind == 0 ? (touching(g, bx, by, bbox) ? 1 : 0)
-                               : (touch ? touch[(size_t)sp[k].fish * g.bpdx * g.bpdy + bx +
-                                                g.bpdx * by]
-                                        : 0);
+      s_a[c] = sp[k].kind == 0 && touching(g, bx, by, bbox) ? 1 : 0;
       s_b[c] = bx + g.bpdx * by;
       s_c[c] = k;
     }
@@ -408,7 +403,7 @@ __global__ __launch_bounds__(NT) void k_obst_begin(Grid g, const ShapeParams* __
     // block's box (grown by the chunk's largest safe distance) cannot pass
     // the first test of any of its segments, so only the pairs that meet it
     // are listed, and their (candidate, segment) tests run in parallel.
-    for (int k = 0; !touch && k < ns; ++k) {
+    for (int k = 0; k < ns; ++k) {
       if (sp[k].kind != 1) continue;
       const int c0 = s_cstart[k] > w0 ? s_cstart[k] - w0 : 0;
       const int c1 = s_cstart[k + 1] - w0 < nw ? s_cstart[k + 1] - w0 : nw;
@@ -998,7 +993,7 @@ int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
     hipLaunchKernelGGL(k_obst_begin, dim3(1), dim3(NT), 0, c->stream, c->g, c->sp, c->ss, c->st,
                        c->ob, c->ob_prev, c->obmap, c->ubidx, c->fishd, c->maxpart, c->nwg,
                        c->ramp, compute_dt, c->graph_capture ? -1 : c->host_step, fish ? 1 : 0,
-                       end_prev, nullptr);
+                       end_prev);
   }
   // overlap 2: advDiff needs only dt and U_inf from the first phase of the
   // list builder; it runs on the side stream beside the whole chain, which
@@ -1043,12 +1038,9 @@ int enqueue_put_objects(cup2d_ctx* c, int compute_dt, int overlap) {
   if (fish) {
     if (!(s = stream_for(ST_MIDLINE))) return CUP2D_ERR_HIP;
     RC_OB(enqueue_fish_midline(c, s));
-    const bool several = c->hfish.size() > 1;
-    if (several) RC_OB(enqueue_fish_touch(c, s));
     hipLaunchKernelGGL(k_obst_begin, dim3(1), dim3(NT), 0, s, c->g, c->sp, c->ss, c->st, c->ob,
                        c->ob_prev, c->obmap, c->ubidx, c->fishd, c->maxpart, c->nwg, c->ramp, 0,
-                       c->graph_capture ? -1 : c->host_step, 2, 0,
-                       several ? c->fish_touch : nullptr);
+                       c->graph_capture ? -1 : c->host_step, 2, 0);
     if (chain_main && mid_a_here) CUP2D_HIP_CHECK(c, hipEventRecord(c->ev_lists, c->stream));
     if (!(s = stream_for(ST_FISH_PLACE))) return CUP2D_ERR_HIP;
     RC_OB(enqueue_fish_place(c, s));
@@ -2194,8 +2186,7 @@ int enqueue_step_front(cup2d_ctx* c, int compute_dt, const FrontAcc& acc) {
     TimerScope ts(c, T_PUT_OBJECTS);
     hipLaunchKernelGGL(k_obst_begin, dim3(1), dim3(NT), 0, c->stream, c->g, c->sp, c->ss, c->st,
                        c->ob, c->ob_prev, c->obmap, c->ubidx, c->fishd, c->maxpart, c->nwg,
-                       c->ramp, compute_dt, c->graph_capture ? -1 : c->host_step, 0, end_prev,
-                       nullptr);
+                       c->ramp, compute_dt, c->graph_capture ? -1 : c->host_step, 0, end_prev);
   }
   const int NX = c->g.NX, gx = strips_x(NX), gy = c->g.NY / STENCIL_RY;
   const int nplace = 2 * G, nforces = forces ? G : 0, nfront = (nplace + nforces + 7) / 8 * 8;
@@ -2338,8 +2329,6 @@ int obstacles_alloc(cup2d_ctx* c) {
   // list builder holds while the actual obstacle blocks fit: the list
   // builder reports CUP2D_ERR_CAPACITY when they do not
   cap = cap > OBST_LIST_CAP ? OBST_LIST_CAP : cap;
-  if (c->hfish.size() > 1)
-    CUP2D_HIP_CHECK(c, hipMalloc(&c->fish_touch, c->hfish.size() * (size_t)nblocks));
   int rc = obstacles_alloc_one(c, c->ob, cap);
   if (rc) return rc;
   return obstacles_alloc_one(c, c->ob_prev, cap);
