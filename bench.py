@@ -49,7 +49,7 @@ STEP_BALG_METRIC = {"periodic": 18, "freespace": 23}
 # 76: rows 16 (R p; W double spectrum), apply columns 16, the residual's
 # inverse rows 16 (R spectrum, b; W the residual's FP32 half spectrum: its
 # forward rows are fused in), FP32 columns 8 and inverse rows 20 (R float
-# spectrum, R and W p).  Without the fusion (mirrored cosine rows) the
+# spectrum, R and W p).  Without the fusion (cosine rows) the
 # residual plane is written and read back: 84.
 STEP_BYTES_FP32 = {"base": 76, "sweep": 76, "sweep_unfused": 84}
 FULL_GRID = list(BALG)
