@@ -1963,9 +1963,15 @@ struct ForceLog {
   unsigned long long* cnt;   // records written so far
   int cap;
 };
-__device__ void forces_fin_wg(const Grid& g, cup2d_shape_state* __restrict__ ss,
-                              const Obstacles& ob, StepState* __restrict__ st, int end_step,
-                              const ForceSnap* __restrict__ snap, ForceLog flog, int deferred) {
+// (forced inline: with two callers the compiler made it a function of 248
+// registers with a stack in device memory, 228 B a lane, in both kernels; the
+// totals' launch is on the path of every disk step, 155 -> 150 us for a step
+// with its host reads at 1024 x 512, 88.5 -> 86.5 us for one of eight disks at
+// 512 x 256)
+__device__ __forceinline__ void forces_fin_wg(const Grid& g, cup2d_shape_state* __restrict__ ss,
+                                              const Obstacles& ob, StepState* __restrict__ st,
+                                              int end_step, const ForceSnap* __restrict__ snap,
+                                              ForceLog flog, int deferred) {
   const unsigned long long nrec = flog.rec ? *flog.cnt : 0ull;
   for (int k = threadIdx.x / 64; k < g.nshapes; k += NT / 64) {  // a shape per wave
     double a[18];
