@@ -166,20 +166,29 @@ int sync_all(cup2d_ctx* c) {
   return wait_streams(c);
 }
 
-// The step scalars (and one shape's state) after everything enqueued so far,
-// in c->mail: a kernel of one wave writes them to pinned host memory, so one
-// stream wait replaces a wait and a device-to-host copy, which took about as
-// long as a small step's whole solve (a cosine solve of 1024 x 512 through
-// cup2d_poisson_solve 43 -> 33 us).
-int fetch_state(cup2d_ctx* c, int shape = -1) {
+// The step scalars (st) and one shape's state (ss) after everything enqueued
+// so far: a kernel of one wave writes them to pinned host memory (c->mail), so
+// one stream wait replaces a wait and a device-to-host copy, which took about
+// as long as a small step's whole solve (a cosine solve of 1024 x 512 through
+// cup2d_poisson_solve 43 -> 33 us).  The mailbox is held from the publishing
+// kernel to the copy out of it: threads that read one simulation's state at
+// the same time each get what they asked for.
+int fetch_state(cup2d_ctx* c, StepState* st, int shape = -1, cup2d_shape_state* ss = nullptr) {
+  std::lock_guard<std::mutex> hold(c->mail_lock);
   RC(enqueue_pending(c));
   RC(enqueue_publish(c, shape));
-  return wait_streams(c);
+  RC(wait_streams(c));
+  if (st) *st = c->mail->st;
+  if (ss) *ss = c->mail->ss;
+  return CUP2D_OK;
 }
 
-int sync_and_check(cup2d_ctx* c) {
-  RC(fetch_state(c));
-  const int err = c->mail->st.error;
+// st (if given) is filled unless the call fails with CUP2D_ERR_HIP
+int sync_and_check(cup2d_ctx* c, StepState* st = nullptr) {
+  StepState own;
+  if (!st) st = &own;
+  RC(fetch_state(c, st));
+  const int err = st->error;
   if (err == CUP2D_ERR_BODY_OUT) return fail(c, err, "a body left the domain");
   if (err == CUP2D_ERR_CAPACITY) return fail(c, err, "obstacle-block pool exhausted");
   if (err == CUP2D_ERR_NONFINITE)
@@ -816,8 +825,8 @@ int cup2d_field_device_ptr(cup2d_ctx* c, int f, int comp, void** dptr) {
 int cup2d_get_scalars(cup2d_ctx* c, double* time, double* dt, int* step, double uinf[2],
                       double* h) {
   CHECK_CTX(c);
-  RC(fetch_state(c));
-  const StepState& s = c->mail->st;
+  StepState s;
+  RC(fetch_state(c, &s));
   if (time) *time = s.time;
   if (dt) *dt = s.dt;
   if (step) *step = s.step;
@@ -841,9 +850,7 @@ int cup2d_set_scalars(cup2d_ctx* c, double time, int step, double uinfx, double 
 int cup2d_get_shape(cup2d_ctx* c, int i, cup2d_shape_state* out) {
   CHECK_CTX(c);
   if (i < 0 || i >= c->g.nshapes || !out) return fail(c, CUP2D_ERR_ARG, "bad shape id");
-  RC(fetch_state(c, i));
-  *out = c->mail->ss;
-  return CUP2D_OK;
+  return fetch_state(c, nullptr, i, out);
 }
 
 int cup2d_fish_midline(cup2d_ctx* c, int i, int* Nm, double* out) {
@@ -881,16 +888,18 @@ int cup2d_reset(cup2d_ctx* c) {
 int cup2d_find_max_u(cup2d_ctx* c, double* maxU) {
   CHECK_CTX(c);
   RC(enqueue_find_max_u(c));
-  const int rc = sync_and_check(c);
-  if (maxU && rc != CUP2D_ERR_HIP) *maxU = c->mail->st.maxU;
+  StepState s;
+  const int rc = sync_and_check(c, &s);
+  if (maxU && rc != CUP2D_ERR_HIP) *maxU = s.maxU;
   return rc;
 }
 
 int cup2d_calc_max_timestep(cup2d_ctx* c, double* dt) {
   CHECK_CTX(c);
   RC(enqueue_dt(c));
-  const int rc = sync_and_check(c);
-  if (dt && rc != CUP2D_ERR_HIP) *dt = c->mail->st.dt;
+  StepState s;
+  const int rc = sync_and_check(c, &s);
+  if (dt && rc != CUP2D_ERR_HIP) *dt = s.dt;
   return rc;
 }
 

@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -173,6 +174,7 @@ struct cup2d_ctx {
   bool side_used = false;  // work enqueued on aux or mids since the host last waited for them
   cup2d::HostMail* mail = nullptr;      // pinned host memory
   cup2d::HostMail* mail_dev = nullptr;  // the same in the device's address space
+  std::mutex mail_lock;                 // from the publishing kernel to the copy out of mail
   // third stream: the swimmers' time-only midline part of the next step runs
   // there beside advDiff (a kernel with many workgroups, so one more resident
   // workgroup costs it nothing); the side stream joins it (ev_mid) while idle
