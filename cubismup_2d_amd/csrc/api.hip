@@ -275,6 +275,41 @@ int pressure_iterator(cup2d_ctx* c, int* iters_out, double* reldf_out) {
 #define CUP2D_SYNC_EVENT_FLAGS (hipEventDisableTiming | hipEventDisableSystemFence)
 
 
+// Does this step of a run with disks only take its parts in launches of their
+// own, so that the timers of those parts read them (the merged launches of
+// enqueue_step_front hold several)?  The parts that are timed in none of this
+// step's launches count as passed.
+bool parts_timed(cup2d_ctx* c) {
+  const bool iter = c->cfg.iterative_penal;
+  const struct { int id; bool launched; } parts[] = {
+      {T_ADVDIFF, true}, {T_FORCES, true}, {T_FLUXFIX, iter}, {T_RHS_OBST, !iter},
+      {T_FADE, !iter && c->band_nblocks > 0}};
+  bool due = false;
+  for (const auto& p : parts) {
+    const Timer& t = c->timers[p.id];
+    due |= p.launched && t.on && t.seen % t.every == 0;
+  }
+  if (!due)
+    for (const auto& p : parts)
+      if (p.launched && c->timers[p.id].on) ++c->timers[p.id].seen;
+  return due;
+}
+
+// The head of a whole step with disks only: the merged launches, or each part
+// by itself on the main stream (the same arithmetic; acc as there).
+int enqueue_disk_head(cup2d_ctx* c, int compute_dt, const FrontAcc& acc = FrontAcc{}) {
+  if (!parts_timed(c)) return enqueue_step_front(c, compute_dt, acc);
+  const bool forces = c->forces_pending;
+  RC(flush_forces(c));
+  if (acc.J && forces) RC(enqueue_adjoint_acc_drag(c, 0, acc.w, acc.J));
+  RC(enqueue_put_objects(c, compute_dt, 0));
+  RC(enqueue_advdiff(c, c->cfg.iterative_penal ? 0 : 1));
+  if (acc.J)
+    CUP2D_HIP_CHECK(c, hipMemcpyAsync(acc.dts + acc.k, &c->st->dt, sizeof(double),
+                                      hipMemcpyDeviceToDevice, c->stream));
+  return CUP2D_OK;
+}
+
 // Simulation::advance.  compute_dt: dt from the findMaxU partials of the
 // previous step (device loop) instead of the value already on the device.
 int advance_enqueued(cup2d_ctx* c, int compute_dt) {
@@ -282,25 +317,25 @@ int advance_enqueued(cup2d_ctx* c, int compute_dt) {
   // step, off the critical path).  With swimmers the placement chain is
   // longer than advDiff: it keeps the main stream and advDiff goes beside it.
   // With disks only, placement, advDiff and the previous step's forces share
-  // launches on the main stream.
+  // launches on the main stream (enqueue_disk_head).
   const bool fish = !c->hfish.empty(), chain_main = fish && !c->cfg.iterative_penal;
-  const bool front = !fish && c->g.nshapes > 0;
-  if (front)
-    RC(enqueue_step_front(c, compute_dt));
+  const bool disks = !fish && c->g.nshapes > 0;
+  if (disks)
+    RC(enqueue_disk_head(c, compute_dt));
   else
     RC(enqueue_put_objects(c, compute_dt, chain_main ? 2 : (fish ? 1 : 0)));
   if (c->cfg.iterative_penal) {
-    if (front) {
+    if (c->front_fused) {
       c->front_fused = false;
       RC(flush_commit(c));
       RC(enqueue_flux_fix(c, c->stream));
-    } else {
+    } else if (!disks) {
       RC(enqueue_advdiff(c, 0));
     }
     RC(pressure_iterator(c, nullptr, nullptr));
     RC(enqueue_find_max_u_partials(c));  // for the next step's dt
   } else {
-    if (!front && !chain_main) RC(enqueue_advdiff(c, 1));
+    if (!disks && !chain_main) RC(enqueue_advdiff(c, 1));
     RC(pressure_single(c, 1));
   }
   RC(enqueue_forces(c, 1, 1));
@@ -463,7 +498,7 @@ int adjoint_eligible(cup2d_ctx* c) {
 int adjoint_recompute_step(cup2d_ctx* c, double dt, double* w, double* u1, double* p) {
   const size_t n = (size_t)c->g.NX * c->g.NY;
   RC(enqueue_set_dt(c, dt));
-  RC(enqueue_step_front(c, 0));
+  RC(enqueue_disk_head(c, 0));
   RC(enqueue_adjoint_record_w(c, w, w + n));
   RC(pressure_single(c, 1));
   RC(enqueue_adjoint_record(c, u1, u1 + n, p));
@@ -1076,7 +1111,7 @@ int cup2d_adjoint_forward(cup2d_ctx* c, int nsteps, int every, const double* dts
   if (!dts_in) RC(enqueue_find_max_u_partials(c));
   for (int k = 0; k < nsteps; ++k) {
     if (dts_in) RC(enqueue_set_dt(c, dts_in[k]));
-    RC(enqueue_step_front(c, dts_in ? 0 : 1, FrontAcc{a->scal, wJ, a->dts_dev, k}));
+    RC(enqueue_disk_head(c, dts_in ? 0 : 1, FrontAcc{a->scal, wJ, a->dts_dev, k}));
     RC(pressure_single(c, 1));
     RC(enqueue_forces(c, 1, 1));
     c->host_step += 1;

@@ -1329,7 +1329,6 @@ __global__ __launch_bounds__(NT) void k_step_rhs2(Grid g, StepState* __restrict_
 
 static int enqueue_step_rhs(cup2d_ctx* c) {
   const int G = grid_cap(c), nb = c->band_nblocks;
-  TimerScope ts(c, T_RHS_OBST);
   CUP2D_REAL_DISPATCH(c, hipLaunchKernelGGL(k_step_rhs1<T>, dim3(G + 1 + nb), dim3(NT), 0,
                                             c->stream, c->g, c->st, c->ob, G, c->chi,
                                             tp<T>(c->rhs), tp<T>(c->u), tp<T>(c->v), c->ss,
@@ -2196,20 +2195,15 @@ int enqueue_step_front(cup2d_ctx* c, int compute_dt, const FrontAcc& acc) {
   }
   const int NX = c->g.NX, gx = strips_x(NX), gy = c->g.NY / STENCIL_RY;
   const int nplace = 2 * G, nforces = forces ? G : 0, nfront = (nplace + nforces + 7) / 8 * 8;
-  {
-    KernelTimer kt(c, T_ADVDIFF);
-    // strips narrower than a workgroup (NX < 256) are ragged ones of it
-    strip_dispatch(c, 256, [&](auto rg, auto stream, auto real) {
-      using T = decltype(real);
-      CUP2D_TIMED_LAUNCH(c, (k_step_place<T, rg(), stream()>), dim3(nfront + gx * gy), dim3(256), 0,
-                         c->stream, c->g, (const ShapeParams*)c->sp,
-                         (const cup2d_shape_state*)c->ss, c->ob, c->ob_prev,
-                         (const unsigned char*)c->obmap, (const int*)c->ubidx, c->chi, c->udx,
-                         c->udy, c->invrho, nplace, nforces, nfront, (const ForceSnap*)c->fsnap,
-                         (const double*)c->pres, surf_of(c), tp<T>(c->u), tp<T>(c->v),
-                         tp<T>(c->tu), tp<T>(c->tv), (const StepState*)c->st, c->fluxpart, gx, gy);
-    });
-  }
+  // strips narrower than a workgroup (NX < 256) are ragged ones of it
+  strip_dispatch(c, 256, [&](auto rg, auto stream, auto real) {
+    using T = decltype(real);
+    hipLaunchKernelGGL((k_step_place<T, rg(), stream()>), dim3(nfront + gx * gy), dim3(256), 0,
+                       c->stream, c->g, c->sp, c->ss, c->ob, c->ob_prev, c->obmap, c->ubidx,
+                       c->chi, c->udx, c->udy, c->invrho, nplace, nforces, nfront, c->fsnap,
+                       c->pres, surf_of(c), tp<T>(c->u), tp<T>(c->v), tp<T>(c->tu), tp<T>(c->tv),
+                       c->st, c->fluxpart, gx, gy);
+  });
   std::swap(c->u, c->tu);  // advDiff.cpp:81-87 copy tmpV -> vel
   std::swap(c->v, c->tv);
   c->flux_deferred = true;

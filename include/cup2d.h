@@ -265,7 +265,11 @@ int cup2d_force_log_read(cup2d_ctx* ctx, int shape_id, int max_records, double* 
  * fft_cols fft_rows_inv pressure_correction put_objects body_update penalize
  * forces, or "*".  reserve_launches > 0 enables (pre-creating that many HIP
  * event pairs), 0 disables.  Each launch is bracketed by two events on the
- * context's stream.  timer_read returns and clears the summed duration. */
+ * context's stream.  timer_read returns and clears the summed duration.
+ * A whole step with disks only otherwise takes advdiff, flux_fix,
+ * rhs_obstacles, fade and forces as parts of merged launches; a step in which
+ * one of them is timed runs each as its own launch (the same arithmetic; only
+ * with an obstacle in the fade band the fade sums are added in another order). */
 int cup2d_timer_enable(cup2d_ctx* ctx, const char* kernel, int reserve_launches);
 int cup2d_timer_read(cup2d_ctx* ctx, const char* kernel, double* total_ms, int* launches);
 /* Time only every n-th launch of the kernel ("*": all timers; n >= 1, default
