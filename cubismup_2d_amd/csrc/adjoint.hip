@@ -414,6 +414,7 @@ __device__ void adj_obst2_wg(int wg, const Grid& g, const Obstacles& ob, int sha
       if (cX[it] > cO[it]) continue;
       const bool perim = cg[it] > 0;
       const double X = cO[it], rr = cr[it];
+      if (X == 0 && !perim) continue;  // the correction leaves the cell alone
       const double T = rr + (-X * rr);
       double sigma = 0;
       if (perim && T > 0 && corr > 0) sigma = 1;
@@ -428,8 +429,12 @@ __device__ void adj_obst2_wg(int wg, const Grid& g, const Obstacles& ob, int sha
 }
 
 // The two passes of the fade's and of the obstacle correction's adjoint side
-// by side: nb band blocks, then the obstacle blocks (the disk's blocks lie
-// outside the band, so the two touch different cells).
+// by side: nb band blocks, then the obstacle blocks.  They must write
+// different cells.  cup2d_adjoint_forward refuses a disk whose blocks reach
+// the band, and a fixed disk keeps its place; should rounding of its centre
+// add a block that its box (2 h wider than the disk) only just meets, chi and
+// its gradient are zero there and pass 2 writes nothing.  A body that moves
+// would need the passes one after the other.
 __global__ __launch_bounds__(ANT) void k_adj_rhs1(Grid g, const int* __restrict__ blocks, int nb,
                                                   Obstacles ob, int shape, double facDiv,
                                                   const double* __restrict__ chi,

@@ -474,7 +474,8 @@ void adjoint_free(cup2d_ctx* c) {
 }
 
 // the forced, fixed single disk with an imposed surface velocity, explicit
-// penalization, FP64: the configuration the adjoint is written for
+// penalization, FP64: the configuration the adjoint is written for (k_adj_rhs1
+// and k_adj_rhs2 also depend on the disk keeping its blocks)
 int adjoint_eligible(cup2d_ctx* c) {
   if (!c->shapes_frozen) return fail(c, CUP2D_ERR_STATE, "call reset first");
   if (c->f32) return fail(c, CUP2D_ERR_STATE, "the adjoint runs at FP64 precision");
@@ -1060,7 +1061,8 @@ int cup2d_adjoint_forward(cup2d_ctx* c, int nsteps, int every, const double* dts
   if (nsteps < 1 || every < 1) return fail(c, CUP2D_ERR_ARG, "nsteps and every must be >= 1");
   RC(sync_all(c));
   // the obstacle blocks and the fade band must not overlap (the adjoint of
-  // the fade holds the RHS formed by the divergence alone)
+  // the fade holds the RHS formed by the divergence alone, and its passes run
+  // beside those of the obstacle correction: k_adj_rhs1, k_adj_rhs2)
   {
     std::vector<unsigned char> om((size_t)c->g.bpdx * c->g.bpdy);
     CUP2D_HIP_CHECK(c, hipMemcpy(om.data(), c->obmap, om.size(), hipMemcpyDeviceToHost));
