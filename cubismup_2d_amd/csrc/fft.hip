@@ -1298,9 +1298,9 @@ __global__ void k_ghat_extract(const double2* __restrict__ spec, int Lc, int ncg
 constexpr int MAX_LR = 8192, MAX_LC = 4096;
 
 template <int L, int KIND, typename S>
-static void launch_rows_fwd(cup2d_ctx* c, const S* in, int pitch, int ncols, int nrows,
-                            cplx<S>* spec, int spec_rows, const cplx<S>* tw, int src,
-                            const RowSource& fd, hipStream_t st) {
+static int launch_rows_fwd(cup2d_ctx* c, const S* in, int pitch, int ncols, int nrows,
+                           cplx<S>* spec, int spec_rows, const cplx<S>* tw, int src,
+                           const RowSource& fd, hipStream_t st) {
   constexpr int RE = row_e<L>();
   constexpr int NP = rows_np<L, RE>();
   const size_t shm = (size_t)NP * lds_len<L, RE>() * sizeof(cplx<S>);
@@ -1314,9 +1314,12 @@ static void launch_rows_fwd(cup2d_ctx* c, const S* in, int pitch, int ncols, int
   else if (src == SRC_PLAIN)
     CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_PLAIN, S, KIND>), grid, block, shm, st,
                        in, pitch, ncols, nrows, spec, spec_rows, tw, fd);
-  else if constexpr (KIND != KIND_COS)  // the cosine solver has no early row pass to patch
+  else if constexpr (KIND != KIND_COS)
     CUP2D_TIMED_LAUNCH(c, (k_rows_fwd<L, NP, RE, SRC_PATCH, S, KIND>), grid, block, shm, st, in,
                        pitch, ncols, nrows, spec, spec_rows, tw, fd);
+  else  // the cosine solver has no early row pass to patch (enqueue_rows_early)
+    return CUP2D_ERR_ARG;
+  return CUP2D_OK;
 }
 template <int L, int KIND, typename S, int OUT>
 static void launch_rows_inv(cup2d_ctx* c, const cplx<S>* spec, int spec_rows, void* out,
@@ -1367,8 +1370,8 @@ static int rows_fwd(cup2d_ctx* c, int L, const S* in, int pitch, int ncols, int 
                     const RowSource& fd, hipStream_t st = nullptr) {
   if (!st) st = c->stream;
   return with_length<KIND == KIND_COS ? MAX_LR / 2 : MAX_LR>(L, [&](auto len) {
-    launch_rows_fwd<len(), KIND, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src, fd, st);
-    return CUP2D_OK;
+    return launch_rows_fwd<len(), KIND, S>(c, in, pitch, ncols, nrows, spec, spec_rows, tw, src,
+                                           fd, st);
   });
 }
 template <typename S, int OUT, int KIND = KIND_SEQ>
