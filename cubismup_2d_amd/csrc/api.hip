@@ -473,6 +473,24 @@ void adjoint_free(cup2d_ctx* c) {
   c->adj = nullptr;
 }
 
+int adjoint_alloc(cup2d_ctx* c, size_t n, int every, int nseg) {
+  AdjointState* a = c->adj = new AdjointState();
+  a->n = n;
+  a->every = every;
+  a->nseg = nseg;
+  a->ck.assign(nseg + 1, nullptr);
+  for (double*& p : a->ck) CUP2D_HIP_CHECK(c, hipMalloc(&p, sizeof(double) * 2 * n));
+  CUP2D_HIP_CHECK(c, hipMalloc(&a->seg, sizeof(double) * n * (5 * (size_t)every + 2)));
+  CUP2D_HIP_CHECK(c, hipMalloc(&a->work, sizeof(double) * n * 6));
+  const int G = c->ob.cap > 0 ? c->ob.cap : 1;
+  const int nblk = G + c->band_nblocks;
+  CUP2D_HIP_CHECK(c, hipMalloc(&a->part, sizeof(double) * 5 * (size_t)(nblk + 1)));
+  CUP2D_HIP_CHECK(c, hipMalloc(&a->theta_part, sizeof(double) * 4 * SURF_MAX_MODES * (size_t)G));
+  CUP2D_HIP_CHECK(c, hipMalloc(&a->theta, sizeof(double) * 4 * SURF_MAX_MODES));
+  CUP2D_HIP_CHECK(c, hipMalloc(&a->scal, sizeof(double) * 4));
+  return CUP2D_OK;
+}
+
 // the forced, fixed single disk with an imposed surface velocity, explicit
 // penalization, FP64: the configuration the adjoint is written for (k_adj_rhs1
 // and k_adj_rhs2 also depend on the disk keeping its blocks)
@@ -1076,20 +1094,13 @@ int cup2d_adjoint_forward(cup2d_ctx* c, int nsteps, int every, const double* dts
   AdjointState* a = c->adj;
   if (!a || a->n != n || a->every != every || a->nseg < nseg) {
     adjoint_free(c);
-    a = c->adj = new AdjointState();
-    a->n = n;
-    a->every = every;
-    a->nseg = nseg;
-    a->ck.assign(nseg + 1, nullptr);
-    for (double*& p : a->ck) CUP2D_HIP_CHECK(c, hipMalloc(&p, sizeof(double) * 2 * n));
-    CUP2D_HIP_CHECK(c, hipMalloc(&a->seg, sizeof(double) * n * (2 * (every + 1) + 3 * every)));
-    CUP2D_HIP_CHECK(c, hipMalloc(&a->work, sizeof(double) * n * 6));
-    const int G = c->ob.cap > 0 ? c->ob.cap : 1;
-    const int nblk = G + c->band_nblocks;
-    CUP2D_HIP_CHECK(c, hipMalloc(&a->part, sizeof(double) * 5 * (size_t)(nblk + 1)));
-    CUP2D_HIP_CHECK(c, hipMalloc(&a->theta_part, sizeof(double) * 4 * SURF_MAX_MODES * (size_t)G));
-    CUP2D_HIP_CHECK(c, hipMalloc(&a->theta, sizeof(double) * 4 * SURF_MAX_MODES));
-    CUP2D_HIP_CHECK(c, hipMalloc(&a->scal, sizeof(double) * 4));
+    const int rc = adjoint_alloc(c, n, every, nseg);
+    if (rc) {  // not half of the buffers for a later call
+      adjoint_free(c);
+      (void)hipGetLastError();  // reported; not again by the next launch check
+      return rc;
+    }
+    a = c->adj;
   }
   if (a->dts_cap < nsteps) {
     if (a->dts_dev) (void)hipFree(a->dts_dev);
