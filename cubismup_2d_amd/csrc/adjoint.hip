@@ -10,7 +10,7 @@
 // function of max|u|), and the body is forced and fixed, so its velocity,
 // position and chi are the same every step.
 //
-// The forward step (operator path, FP64, explicit penalization):
+// The forward step (FP64, explicit penalization):
 //   w     = advDiff(u_n)                        advDiff.cpp:14-79
 //   wf    = (I - e e^T / nb) w                   boundary-flux correction,
 //                                               advDiff.cpp:89-116 (e: +1 on
@@ -25,12 +25,13 @@
 // Its adjoint, run backwards one step at a time (kernels below, in the order
 // the host calls them): drag -> penalization (and the parameter gradient) ->
 // projection -> S (the solve is symmetric: even Green's function, real even
-// symbols) -> fade -> obstacle correction -> divergence -> flux correction
-// (a symmetric projector) -> advDiff linearized at u_n.  The fade and the
-// obstacle correction rescale signed parts by ratios of sums; their adjoints
-// hold the sign pattern (active set) of the forward values and carry the
-// derivative of the ratio, so the adjoint is exact wherever no value sits on
-// a sign change, as it is for the drag's max(0, .) per surface point.
+// symbols) -> fade and, beside it on other blocks, obstacle correction ->
+// divergence -> flux correction (a symmetric projector) -> advDiff linearized
+// at u_n.  The fade and the obstacle correction rescale signed parts by ratios
+// of sums; their adjoints hold the sign pattern (active set) of the forward
+// values and carry the derivative of the ratio, so the adjoint is exact
+// wherever no value sits on a sign change, as it is for the drag's max(0, .)
+// per surface point.
 //
 // Vectors in the adjoint are dense planes like the fields.  The drag's
 // surface stencils scatter with atomic adds (a few hundred surface points);
@@ -284,7 +285,10 @@ __global__ __launch_bounds__(ANT) void k_adj_project(Grid g, double pFac,
 // cub2rhs fade, pass 1: per band block, the forward sums of f = r fa^2
 // (total, positive and negative parts) and the adjoint sums
 // sum rb max(f,0) and sum rb (-min(f,0)); r recomputed from wf.
-__device__ void adj_fade1_wg(int wg, const Grid& g, const int* __restrict__ blocks, int nblocks, double facDiv, const double* __restrict__ wu, const double* __restrict__ wv, const double* __restrict__ rb, double* __restrict__ part, double* lds) {
+__device__ void adj_fade1_wg(int wg, const Grid& g, const int* __restrict__ blocks, int nblocks,
+                             double facDiv, const double* __restrict__ wu,
+                             const double* __restrict__ wv, const double* __restrict__ rb,
+                             double* __restrict__ part, double* lds) {
   const int j = wg;
   const int b = blocks[j], bx = b % g.bpdx, by = b / g.bpdx;
   double a[5] = {0, 0, 0, 0, 0};
@@ -305,7 +309,10 @@ __device__ void adj_fade1_wg(int wg, const Grid& g, const int* __restrict__ bloc
 
 // cub2rhs fade, pass 2: every workgroup sums the partials (same order), forms
 // corr = Sr / (Sr > 0 ? P : N) and applies the transposed fade to its block.
-__device__ void adj_fade2_wg(int wg, const Grid& g, const int* __restrict__ blocks, int nblocks, double facDiv, const double* __restrict__ wu, const double* __restrict__ wv, const double* __restrict__ part, double* __restrict__ rb, double* lds) {
+__device__ void adj_fade2_wg(int wg, const Grid& g, const int* __restrict__ blocks, int nblocks,
+                             double facDiv, const double* __restrict__ wu,
+                             const double* __restrict__ wv, const double* __restrict__ part,
+                             double* __restrict__ rb, double* lds) {
   const int j = wg;
   double tot[5];
   block_sum_table<ANT, 5>(part, nblocks, 5, tot, lds);  // the same order in every workgroup
@@ -332,7 +339,10 @@ __device__ void adj_fade2_wg(int wg, const Grid& g, const int* __restrict__ bloc
 // the shape (S = sum -chi r, positive and negative perimeter parts of
 // T = r (1 - chi)) and the adjoint sums for both signs of corr:
 // sum rb (-T) [perimeter, T > 0] and sum rb T [perimeter, T < 0].
-__device__ void adj_obst1_wg(int wg, const Grid& g, const Obstacles& ob, int shape, double facDiv, const double* __restrict__ chi, const double* __restrict__ wu, const double* __restrict__ wv, const double* __restrict__ rb, double* __restrict__ part, double* lds) {
+__device__ void adj_obst1_wg(int wg, const Grid& g, const Obstacles& ob, int shape, double facDiv,
+                             const double* __restrict__ chi, const double* __restrict__ wu,
+                             const double* __restrict__ wv, const double* __restrict__ rb,
+                             double* __restrict__ part, double* lds) {
   double a[5] = {0, 0, 0, 0, 0};
   const int nub = ob.cnt[1];
   if (wg < nub) {
@@ -376,7 +386,10 @@ __device__ void adj_obst1_wg(int wg, const Grid& g, const Obstacles& ob, int sha
 
 // obstacle RHS correction, pass 2: totals (in order), corr = S / D, and the
 // transposed correction and source term on the block's cells.
-__device__ void adj_obst2_wg(int wg, const Grid& g, const Obstacles& ob, int shape, double facDiv, const double* __restrict__ chi, const double* __restrict__ wu, const double* __restrict__ wv, const double* __restrict__ part, double* __restrict__ rb, double* lds) {
+__device__ void adj_obst2_wg(int wg, const Grid& g, const Obstacles& ob, int shape, double facDiv,
+                             const double* __restrict__ chi, const double* __restrict__ wu,
+                             const double* __restrict__ wv, const double* __restrict__ part,
+                             double* __restrict__ rb, double* lds) {
   const int nub = ob.cnt[1];
   if (wg >= nub) return;
   double tot[5];

@@ -129,6 +129,8 @@ __device__ __forceinline__ void bfly1(V& a, V& c) {
   c = csub(t, c);
 }
 // a, c <- a + w c, a - w c in six fused operations: a - w c = 2 a - (a + w c)
+// (butterflies of six operations for fused multiply-add machines: Linzer and
+// Feig, Math. Comp. 60, 1993, there with scaled twiddle factors)
 template <typename V>
 __device__ __forceinline__ void bfly(V& a, V& c, V w) {
   using S = typename ScalarOf<V>::type;
@@ -438,6 +440,11 @@ constexpr bool row_split() { return L >= 8192 && sizeof(S) == 8 && OUT == 0; }
 
 template <int L, int E>
 constexpr int lds_len() { return L + L / E; }
+// Row pairs per workgroup: as many as fill a wave, by the length alone.
+// Filling 256 threads leaves small grids with a few workgroups: solves of 256
+// x 128 periodic 33.3 against 31.8 us, cosine 26.4 against 24.5, free-space
+// 160 x 96 32.1 against 30.7; from rows of 2048 on the two are the same, and
+// steps of 512 x 256 differ by 1%.
 template <int L, int E>
 constexpr int rows_np() { return (L / E) >= 64 ? 1 : 64 / (L / E); }
 

@@ -166,8 +166,9 @@ struct cup2d_ctx {
   cup2d::Grid g;
   hipStream_t stream = nullptr;
   bool own_stream = false;
-  // side stream: the PutObjectsOnGrid chain after the list builder runs there,
-  // overlapping advDiff and the RHS (neither reads obstacle data)
+  // side stream, used with swimmers only: advDiff, the fade sums and the early
+  // row pass beside the PutObjectsOnGrid chain (iterative penalization: the
+  // chain after the list builder beside advDiff)
   hipStream_t aux = nullptr;
   hipEvent_t ev_begin = nullptr, ev_obst = nullptr, ev_pen = nullptr, ev_frc = nullptr;
   hipEvent_t ev_lists = nullptr;  // this step's midline and lists done (main stream)
@@ -185,9 +186,10 @@ struct cup2d_ctx {
   bool front_fused = false;     // enqueue_step_front ran: the obstacle RHS launches take the fade sums
   // ComputeForces and the step end (time += dt) of the last whole step, not
   // enqueued yet.  The next whole step applies the step end in its list
-  // builder and runs ComputeForces on the side stream after its obstacle
-  // chain (joined before the pressure is overwritten); any other call first
-  // enqueues both on the main stream (flush_forces).
+  // builder and runs ComputeForces within its own launches (disks only), on
+  // the midline stream beside its obstacle chain (swimmers) or on the side
+  // stream after it (swimmers, iterative), before the pressure is overwritten;
+  // any other call first enqueues both on the main stream (flush_forces).
   bool forces_pending = false;
   bool end_pending = false;
   bool frc_join = false;  // the main stream must wait for ev_frc
@@ -220,7 +222,10 @@ struct cup2d_ctx {
   // operators at 4096 x 2048 326 -> 320 us, swimmer step there 338 -> 332 us,
   // 8192 x 4096 1.29 -> 1.265 ms, free-space solve of 4000 x 2016 245 -> 232
   // us; at 2048 x 1024, where the planes fit, 1.7% slower, and with FP32
-  // planes 1% slower at 4096 x 2048.
+  // planes 1% slower at 4096 x 2048.  From the line upwards on free-space grids,
+  // whose padded spectrum adds to the six planes: steps of 2976 x 1920 (5.7 M
+  // cells) 1.3% faster, 3200 x 1920 0.8%, 4096 x 2048 3.1%; periodic steps of
+  // 8192 x 2048 and 4096 x 4096 the same either way.
   bool stream_stores = false;
   // Captured whole steps (cup2d_simulate_graph): two steps per graph, from
   // and back to the quiescent state (nothing pending on the side streams);

@@ -56,9 +56,10 @@ __device__ inline SlotView slot(const Obstacles& ob, int s) {
 
 // A workgroup's slot s, or its distinct block u with the block's first slot
 // (the only one unless shapes overlap): the list entries are loaded together
-// with the count they are tested against (the lists hold at least gridDim
-// entries, so the loads are in bounds), one memory round trip instead of two
-// or three in kernels of a few microseconds.
+// with the count they are tested against, one memory round trip instead of two
+// or three in kernels of a few microseconds.  A workgroup past the lists'
+// capacity (the placement launches twice as many) loads the last entry, which
+// it then does not use.
 struct SlotHead {
   int n, k, b;
   __device__ SlotHead(const Obstacles& ob, int s) {
@@ -961,8 +962,11 @@ __global__ __launch_bounds__(NT) void k_obst_commit(Grid g, cup2d_shape_state* _
 static int grid_cap(cup2d_ctx* c) { return c->ob.cap > 0 ? c->ob.cap : 1; }
 
 // PutObjectsOnGrid::operator() (PutObjectsOnGrid.cpp:186-241).
-// overlap: run everything after the list builder on the side stream; the
-// caller joins with join_obstacles() before the next reader of obstacle data.
+// overlap 0: every stage on the main stream (operator calls; disk steps whose
+// parts are timed).  1 (swimmers with the iterative penalization): everything
+// after the list builder on the side stream; the caller joins with
+// join_obstacles() before the next reader of obstacle data.  2 (swimmers): the
+// chain on the main stream, advDiff on the side stream.
 static int launch_forces(cup2d_ctx* c, hipStream_t s, const Obstacles& lists, int end_step,
                          const double* u, const double* v, int deferred);
 
@@ -2124,10 +2128,16 @@ static int launch_forces(cup2d_ctx* c, hipStream_t s, const Obstacles& lists, in
 // the moments, the flux reduction and the force totals.  (As kernels on two
 // streams the same work needed three cross-stream events per step, 6-9 us
 // each, and the totals waited for launches of one workgroup: whole step at
-// 512 x 256 107 -> 72 us, one disk on 4096 x 2048 317 -> 285 us.)  The parts of a launch touch disjoint data: the
-// placement writes this step's slots and the dense obstacle planes, the forces
-// read the previous step's lists, velocity and pressure.  The latency-bound
-// workgroups come first, so they start at once and the strips fill the rest.
+// 512 x 256 107 -> 68 us, one disk on 4096 x 2048 317 -> 277 us.)  It is taken
+// for any number of disks: with 8, 20, 40 and 64 of them the step went 143 ->
+// 88, 199 -> 128, 614 -> 421 and 1506 -> 964 us at 512 x 256 (where most of
+// the grid is then obstacle blocks) and 350 -> 314, 416 -> 386, 567 -> 493 and
+// 832 -> 665 us at 4096 x 2048.  The parts of a launch touch disjoint data:
+// the placement writes this step's slots and the dense obstacle planes, the
+// forces read the previous step's lists, velocity and pressure.  The
+// latency-bound workgroups come first, so they start at once and the strips
+// fill the rest.  A step whose parts are timed runs them as kernels of their
+// own (enqueue_disk_head).
 template <typename T, bool RAGGED, bool STREAM>
 __global__ __launch_bounds__(256, 4) void k_step_place(
     Grid g, const ShapeParams* __restrict__ sp, const cup2d_shape_state* __restrict__ ss,
