@@ -1967,10 +1967,8 @@ struct ForceLog {
   int cap;
 };
 // (forced inline: with two callers the compiler made it a function of 248
-// registers with a stack in device memory, 228 B a lane, in both kernels; the
-// totals' launch is on the path of every disk step, 155 -> 150 us for a step
-// with its host reads at 1024 x 512, 88.5 -> 86.5 us for one of eight disks at
-// 512 x 256)
+// registers with a stack in device memory, 228 B a lane, in both kernels;
+// k_step_moments, on the path of every disk step, 5.8 -> 4.8 us at 512 x 256)
 __device__ __forceinline__ void forces_fin_wg(const Grid& g, cup2d_shape_state* __restrict__ ss,
                                               const Obstacles& ob, StepState* __restrict__ st,
                                               int end_step, const ForceSnap* __restrict__ snap,
