@@ -411,7 +411,10 @@ int step_graph(cup2d_ctx* c, hipGraphExec_t* out) {
     *out = gr.exec;
     return CUP2D_OK;
   }
-  if (gr.exec) (void)hipGraphExecDestroy(gr.exec);
+  if (gr.exec) {  // its last launch may still run
+    CUP2D_HIP_CHECK(c, hipStreamSynchronize(c->stream));
+    (void)hipGraphExecDestroy(gr.exec);
+  }
   gr = cup2d_ctx::StepGraph{};
   CUP2D_HIP_CHECK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   const int rc = capture_two_steps(c);
@@ -1425,7 +1428,11 @@ bool ens_graph_valid(const cup2d_ensemble* e, int lanes) {
   return true;
 }
 
+// The graphs are destroyed once their last launches are over: a change of
+// parity or of lanes can come while an earlier call's steps still run.
 void ens_drop(cup2d_ensemble* e) {
+  if (!e->exec.empty())
+    for (hipStream_t ls : e->lane_stream) (void)hipStreamSynchronize(ls);
   for (hipGraphExec_t x : e->exec)
     if (x) (void)hipGraphExecDestroy(x);
   e->exec.clear();
