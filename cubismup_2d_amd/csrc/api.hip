@@ -240,6 +240,10 @@ int pressure_single(cup2d_ctx* c, int fused) {
 int pressure_iterator(cup2d_ctx* c, int* iters_out, double* reldf_out) {
   RC(need_fft(c));
   RC(join_obstacles(c));
+  // with swimmers the previous step's ComputeForces may still run on the side
+  // stream: it reads the previous velocity, which the copy overwrites, and the
+  // body snapshot, which every iteration writes
+  RC(join_forces(c));
   RC(enqueue_copy_vel_to_tmpv(c));
   int iter;
   double relDF = 1e3;
