@@ -1973,6 +1973,7 @@ __device__ __forceinline__ void forces_fin_wg(const Grid& g, cup2d_shape_state* 
                                               const Obstacles& ob, StepState* __restrict__ st,
                                               int end_step, const ForceSnap* __restrict__ snap,
                                               ForceLog flog, int deferred) {
+  const bool live = !deferred;  // the bodies as they are now (as in forces_wg)
   const unsigned long long nrec = flog.rec ? *flog.cnt : 0ull;
   for (int k = threadIdx.x / 64; k < g.nshapes; k += NT / 64) {  // a shape per wave
     double a[18];
@@ -1987,7 +1988,7 @@ __device__ __forceinline__ void forces_fin_wg(const Grid& g, cup2d_shape_state* 
     T.Pout = a[13]; T.defPower = a[14]; T.PoutBnd = a[15]; T.defPowerBnd = a[16];
     T.n_surface_points = a[17];
     T.n_obstacle_blocks = ob.slot_of_shape_start[k + 1] - ob.slot_of_shape_start[k];
-    const double su = snap[k].u, sv = snap[k].v;
+    const double su = live ? T.u : snap[k].u, sv = live ? T.v : snap[k].v;
     T.Pthrust = T.thrust * sqrt(su * su + sv * sv);
     T.Pdrag = T.drag * sqrt(su * su + sv * sv);
     const double denUnb = T.Pthrust - dmin(T.defPower, 0.0);
@@ -2015,8 +2016,12 @@ __device__ __forceinline__ void forces_fin_wg(const Grid& g, cup2d_shape_state* 
 }
 
 // ComputeForces.cpp:16-107, per slot; surface points are the cells with D>0.
+// live: the shapes' present state (ComputeForces called by itself: no body
+// update need have come before it, or none since the bodies were placed);
+// nullptr: the state that the step's body update left in snap.
 template <typename RT>
-__device__ void forces_wg(int s, const Grid& g, const ForceSnap* __restrict__ snap,
+__device__ void forces_wg(int s, const Grid& g, const cup2d_shape_state* __restrict__ live,
+                          const ForceSnap* __restrict__ snap,
                           const Obstacles& ob, const RT* __restrict__ u,
                           const RT* __restrict__ v, const double* __restrict__ p, double* lds,
                           const SurfVel& surf) {
@@ -2026,8 +2031,9 @@ __device__ void forces_wg(int s, const Grid& g, const ForceSnap* __restrict__ sn
   const int bx = b % g.bpdx, by = b / g.bpdx;
   SlotView o = slot(ob, s);
   const double NUoH = g.nu / g.h;
-  const double Cx = snap[k].C[0], Cy = snap[k].C[1];
-  const double su = snap[k].u, sv = snap[k].v;
+  const double Cx = live ? live[k].centerOfMass[0] : snap[k].C[0];
+  const double Cy = live ? live[k].centerOfMass[1] : snap[k].C[1];
+  const double su = live ? live[k].u : snap[k].u, sv = live ? live[k].v : snap[k].v;
   const double vel_norm = sqrt(su * su + sv * sv);
   const double vu0 = vel_norm > 0 ? su / vel_norm : 0, vu1 = vel_norm > 0 ? sv / vel_norm : 0;
   double a[18];
@@ -2090,12 +2096,13 @@ __global__ void k_step_end_done(StepState* st) {
 
 // ComputeForces per slot (ComputeForces.cpp:16-107)
 template <typename RT>
-__global__ __launch_bounds__(NT) void k_forces(Grid g, const ForceSnap* __restrict__ snap,
+__global__ __launch_bounds__(NT) void k_forces(Grid g, const cup2d_shape_state* __restrict__ live,
+                                               const ForceSnap* __restrict__ snap,
                                                Obstacles ob, const RT* __restrict__ u,
                                                const RT* __restrict__ v,
                                                const double* __restrict__ p, SurfVel sv) {
   __shared__ double lds[LDS_RED];
-  forces_wg(blockIdx.x, g, snap, ob, u, v, p, lds, sv);
+  forces_wg(blockIdx.x, g, live, snap, ob, u, v, p, lds, sv);
 }
 
 // shape totals (Shape::computeForces, Shape.cpp:252-300) and, with end_step,
@@ -2111,7 +2118,7 @@ static int launch_forces(cup2d_ctx* c, hipStream_t s, const Obstacles& lists, in
                          const double* u, const double* v, int deferred) {
   TimerScope ts(c, T_FORCES, s);
   CUP2D_REAL_DISPATCH(c, hipLaunchKernelGGL(k_forces<T>, dim3(grid_cap(c)), dim3(NT), 0, s, c->g,
-                                            c->fsnap, lists, tp<T>(u), tp<T>(v), c->pres,
+                                            deferred ? nullptr : c->ss, c->fsnap, lists, tp<T>(u), tp<T>(v), c->pres,
                                             surf_of(c)));
   const ForceLog flog{c->flog, c->flog_cnt, c->flog_cap};
   hipLaunchKernelGGL(k_forces_fin, dim3(1), dim3(NT), 0, s, c->g, c->ss, lists, c->st, end_step,
@@ -2153,7 +2160,7 @@ __global__ __launch_bounds__(256, 4) void k_step_place(
   }
   if (w < nfront) {  // nfront: nplace + nforces rounded up to a multiple of 8
     w -= nplace;
-    if (w < nforces) forces_wg(w, g, snap, pv, u, v, p, lds, sv);
+    if (w < nforces) forces_wg(w, g, nullptr, snap, pv, u, v, p, lds, sv);
     return;
   }
   // the strips, each XCD's a contiguous band (workgroup b runs on XCD b % 8)
